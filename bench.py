@@ -271,7 +271,7 @@ def charged_spheres_rate(replicas, legs, far="cell_bounding"):
     k1, ms1 = run_together(chains[:1], legs)
     est = np.array([c.estimators() for c in chains])
     lds_b, lds_p, lds_r = chains[0].launch_lds()
-    kname = "ecmc::chain_many_kernel<3,%d>" % chains[0].kernel_variant()[1]
+    kname = "ecmc::chain_kernel<3,%d>" % chains[0].kernel_variant()[1]
     for c in chains:
         c.close()
     # candidates per leg from a logged run of one more replica of the same system
@@ -320,7 +320,7 @@ def flexible_dipoles_rate(replicas, legs):
     wall = time.perf_counter() - t0
     k1, ms1 = run_together(chains[:1], legs)
     lds_b, lds_p, lds_r = chains[0].launch_lds()
-    kname = "ecmc::chain_many_kernel<3,%d>" % chains[0].kernel_variant()[1]
+    kname = "ecmc::chain_kernel<3,%d>" % chains[0].kernel_variant()[1]
     probe = chains[1].run(300)
     ncand = float(probe["ncand"][1:].mean()) if len(probe) > 1 else 0.0
     desc = chains[0].desc

@@ -189,7 +189,7 @@ int ecmc_system_launch_lds(const ecmc_system *sys, int64_t *bytes, int32_t *posi
  * (bit p for the two-leaf pair potential ECMC_POT_p inverted exactly, bit 9 the merged-image
  * Coulomb factors through the inverse-power Coulomb bound, bit 10 factor-type maps, bit 11 cell
  * bounding, bit 12 the cell veto), *variant the features of the specialized kernel launched for them (its
- * template argument in the kernel's name, ecmc::chain_kernel<dim, variant>).  A launch of
+ * second template argument in the kernel's name, ecmc::chain_kernel<dim, variant, threads, resident>).  A launch of
  * several systems runs the first variant covering all of them.  No reference counterpart: which
  * compiled code runs, for diagnostics and profiles. */
 int ecmc_system_kernel_variant(const ecmc_system *sys, int32_t *features, int32_t *variant);

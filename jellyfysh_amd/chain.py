@@ -203,8 +203,8 @@ class DeviceChain:
 
     def kernel_variant(self):
         """(features the system's taggers use, features of the specialized leg-loop kernel that
-        runs it): the kernel is ecmc::chain_kernel<dim, variant> alone and
-        ecmc::chain_many_kernel<dim, variant> in a launch of several systems of the same variant."""
+        runs it): the kernel is ecmc::chain_kernel<dim, variant, threads, resident>, alone and in a
+        launch of several systems of the same variant."""
         f, v = ctypes.c_int32(), ctypes.c_int32()
         L.check(L.lib().ecmc_system_kernel_variant(self._h, ctypes.byref(f), ctypes.byref(v)))
         return f.value, v.value

@@ -1,5 +1,6 @@
-// ecmc_chain.hip -- one ECMC chain advanced on the GPU, leg after leg, in one persistent
-// workgroup (the plain form).
+// ecmc_chain.hip -- event chains advanced on the GPU, leg after leg, one persistent workgroup per
+// chain (the plain form): host side, kernel variants and table kernels; the leg loop itself is in
+// ecmc_chain_leg.h.
 //
 // A leg follows the reference mediator (mediator/single_process_mediator.py:84-156):
 //   update the cell occupancy for the active unit, run the event handlers of the taggers in
@@ -8,26 +9,21 @@
 //   (tag_activator.py:291-316).
 //
 // Mapping to the hardware:
-//   * the candidate set of a pair tagger (active unit x occupants of the nearby cells,
-//     excluded_cells_tagger.py:129-132) is spread over the 256 threads of the workgroup in
-//     canonical order (nearby cells in itertools.product order, occupants in list order),
-//     one candidate per lane; positions (SoA x[], y[], z[]), the random ring, charges and cell
-//     lists are read from LDS where the launch placed them, else from HBM;
-//   * each candidate's exponential draw is the 2 MT19937 words at its rank in the stream;
-//     words come from a ring that the workgroup refills 624 words at a time with the
-//     three-phase parallel twist, so the draws are those of CPython's random in the
-//     reference's call order;
-//   * the inverse-power candidates are first bracketed in FP32 and only those that can be the
-//     earliest are inverted exactly in FP64;
-//   * the earliest candidate is found by a wavefront shuffle min-reduce over (time, push
-//     rank) followed by a 4-wave LDS reduction; the scheduler keeps, per tagger, the
-//     earliest of its pushed events (all events of one tagger are trashed together), and
-//     ties go to the first pushed event as in list_scheduler.py:129-156; the earliest stored
-//     event is chosen by a butterfly over the first wavefront's lanes, one slot per lane;
-//   * bookkeeping that is sequential in the reference (occupancy lists, end of chain,
-//     sampling, out-states) runs on thread 0 between barriers;
-//   * the leg loop is compiled once per feature set (FEAT_*) and each launch runs the smallest
-//     variant that covers its systems.
+//   * the candidates of a create list's pair taggers are spread over the workgroup in canonical
+//     order (nearby cells in itertools.product order, occupants in list order; excluded_cells_
+//     tagger.py:129-132); positions, the random ring, charges and cell lists are read from LDS
+//     where the launch placed them, else from HBM;
+//   * each candidate's exponential draw is the 2 MT19937 words at its rank in the stream; the
+//     ring holds the MT19937 sequence itself, extended by one wavefront 192 words at a time, so the
+//     draws are those of CPython's random in the reference's call order;
+//   * an FP32 test leaves the few candidates that can decide the leg, which are inverted exactly
+//     in FP64, one per lane;
+//   * the scheduler keeps, per tagger, the earliest of its pushed events (all events of one
+//     tagger are trashed together), and ties go to the first pushed event as in
+//     list_scheduler.py:129-156;
+//   * the sequential bookkeeping runs redundantly in every wavefront;
+//   * the leg loop is compiled once per feature set (FEAT_*) and workgroup size, and each launch
+//     runs the smallest variant that covers its systems.
 #include <hip/hip_runtime.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -43,1047 +39,13 @@
 #include "ecmc_math.h"
 #include "ecmc_potentials.h"
 #include "ecmc_fp32_bounds.h"
+#include "ecmc_chain_leg.h"
 #include "ecmc_common.h"
 
 namespace ecmc {
 
-constexpr int NT = 256;
-
-// The dynamic LDS of a leg-loop launch (positions, then the ring of tempered words), when the
-// launch's arguments place them there (ChainArgs::lds_pos, lds_ring).
-extern __shared__ __align__(16) unsigned char chain_dyn_lds[];
-
-struct ChainArgs;
-__device__ __forceinline__ int32_t *occ_base(const ChainArgs &a);
-__device__ __forceinline__ int32_t *occn_base(const ChainArgs &a);
-constexpr uint32_t MT_UPPER = 0x80000000u, MT_LOWER = 0x7fffffffu, MT_MATRIX = 0x9908b0dfu;
-
-struct Slot {
-    Time t;
-    int64_t seq;
-    int32_t valid, target;
-    double apos[3];
-    Time astamp;
-    double tpos[3];
-    double cb_boundary;
-    int32_t cb_dir, adir;
-    double aspeed;
-    int32_t cb_cell, pad_cb;   // active cell of a cell-bounding candidate; target cell of a cell veto
-    double cv_rate;            // cell veto: bounding event rate of the sampled cell
-    int32_t cv_index, cv_phase;  // cell veto: drawn table entry; 1 = entry pending, 2 = entry drawn
-};
-
-// One entry of Walker's table (walker.py:73-101): item0 with rate0, else the alias item1
-struct CvEntry {
-    double rate0;
-    int32_t item0, item1;
-};
-
-struct ChainState {
-    int32_t active, adir;
-    double aspeed;
-    Time at;
-    int32_t occ_id, occ_cell;
-    int32_t started, done, err, pending_creates, last_tagger, stop_reason;
-    Time last;
-    int64_t seq;
-    Time eoc_last, samp_time;
-    uint64_t cursor, produced;
-    double est[8];
-    int32_t ncand;
-    uint32_t chash;
-    int32_t nsur, pad_s;       // surplus units of a bounded occupancy
-    Slot slot[ECMC_MAX_TAGGERS];
-};
-
-struct ChainArgs {
-    int32_t n, ncells, nb_stride, occ_cap, ring_words, n_taggers, stop_mask, ewald_fc;
-    int32_t leaves;            // leaf units per composite object (1: point masses)
-    int32_t occupancy;         // some tagger reads the cell occupancy (else it is not kept up)
-    double L, half, beta;
-    int32_t cps[3], cum[3];
-    double side[3];
-    Ewald ewald;
-    double *pos;
-    const double *charge;
-    const double *cmin;
-    const int32_t *nearby;
-    const int32_t *nearby_n;
-    int32_t *occ;
-    int32_t *occ_n;
-    uint32_t *mt;
-    uint32_t *ring;
-    ChainState *st;
-    const ecmc_tagger_desc *tg;
-    ecmc_event *log;
-    int64_t max_events;
-    int64_t *n_out;
-    // bounded occupancy (single_active_cell_occupancy.py:62) and cell bounding
-    int32_t max_occ, sur_cap, layers, pad2;
-    int32_t *sur_cell, *sur_id;   // surplus units in the order the reference's dict yields them
-    int32_t *cand;                // the cell-bounding tagger's candidates: their far cells (one occupant each)
-    const double *cbt;            // cell-bound table: (cell offset, direction) -> upper, lower
-    // cell veto: Walker tables [direction * 2 + (0 upper, 1 lower)] of cv_m entries each
-    const CvEntry *cvw;
-    double cv_total[6], cv_mean[6];
-    int32_t cv_m, pad3;
-    // residency in the launch's dynamic LDS: positions (dim x n doubles at offset 0) and the MT
-    // ring (ring_words words at lds_ring_off), copied in at the start of a launch and back at
-    // its end; 0 keeps them in global memory
-    int32_t lds_pos, lds_ring, lds_ring_off, lds_cand_off;   // lds_cand_off < 0: the candidate list in global memory
-    int32_t lds_occ_off, lds_occn_off;                         // < 0: the occupant lists / counts in global memory
-    // the terms of the merged-image Coulomb derivative in the sequential loop's order (real-space
-    // images by k, j, i, then Fourier terms by i, j, k): kind << 24 | (i + 128) << 16 |
-    // (j + 128) << 8 | (k + 128), built on the host
-    const int32_t *ewald_codes;
-    int32_t ewald_ncodes, lds_charge_off;   // lds_charge_off < 0: the charges in global memory
-};
-
-// The cell occupant lists (ncells x occ_cap) and their counts, in LDS for a launch when placed there.
-__device__ __forceinline__ int32_t *occ_base(const ChainArgs &a) {
-    return a.lds_occ_off >= 0 ? reinterpret_cast<int32_t *>(chain_dyn_lds + a.lds_occ_off) : a.occ;
-}
-// The charge of unit id (constant over a run): from LDS when the launch placed the charges there.
-__device__ __forceinline__ double charge_of(const ChainArgs &a, int id) {
-    if (a.lds_charge_off >= 0) return reinterpret_cast<const double *>(chain_dyn_lds + a.lds_charge_off)[id];
-    return a.charge[id];
-}
-__device__ __forceinline__ int32_t *occn_base(const ChainArgs &a) {
-    return a.lds_occn_off >= 0 ? reinterpret_cast<int32_t *>(chain_dyn_lds + a.lds_occn_off) : a.occ_n;
-}
-
-__device__ __forceinline__ uint32_t mt_temper(uint32_t y) {
-    y ^= (y >> 11);
-    y ^= (y << 7) & 0x9d2c5680u;
-    y ^= (y << 15) & 0xefc60000u;
-    y ^= (y >> 18);
-    return y;
-}
-
-// One twist of the 624-word state in LDS, then the tempered words go to the ring.
-// The three phases follow the data dependences of the sequential loop: words 0..226 read
-// only old words; 227..453 read new words 0..226; 454..623 read new words 227..396.
-// Word j of the block goes to ring[(produced + j) & mask] (mask: ring size - 1, all ones for no wrap).
-__device__ __forceinline__ void mt_generate_block(uint32_t *mt, uint32_t *ring, uint64_t mask, uint64_t produced) {
-    const int t = threadIdx.x;
-    uint32_t v = 0;
-    if (t < 227) {
-        uint32_t y = (mt[t] & MT_UPPER) | (mt[t + 1] & MT_LOWER);
-        v = mt[t + 397] ^ (y >> 1) ^ ((y & 1u) ? MT_MATRIX : 0u);
-    }
-    __syncthreads();
-    if (t < 227) mt[t] = v;
-    __syncthreads();
-    if (t < 227) {
-        int i = t + 227;
-        uint32_t y = (mt[i] & MT_UPPER) | (mt[i + 1] & MT_LOWER);
-        v = mt[i - 227] ^ (y >> 1) ^ ((y & 1u) ? MT_MATRIX : 0u);
-    }
-    __syncthreads();
-    if (t < 227) mt[t + 227] = v;
-    __syncthreads();
-    if (t < 170) {
-        int i = t + 454;
-        uint32_t nx = i == 623 ? mt[0] : mt[i + 1];
-        uint32_t y = (mt[i] & MT_UPPER) | (nx & MT_LOWER);
-        v = mt[i - 227] ^ (y >> 1) ^ ((y & 1u) ? MT_MATRIX : 0u);
-    }
-    __syncthreads();
-    if (t < 170) mt[t + 454] = v;
-    __syncthreads();
-    for (int j = t; j < 624; j += NT) ring[(produced + (uint64_t)j) & mask] = mt_temper(mt[j]);
-    __syncthreads();
-}
-
-// Collective: make `need` unread words available in the ring.
-__device__ __forceinline__ void ring_ensure(ChainState &st, uint32_t *mt, const ChainArgs &a, uint64_t need) {
-    if (need + 2 * 624 > (uint64_t)a.ring_words) {   // the ring would overwrite unread words
-        st.err = ECMC_ERR_STATE;
-        return;
-    }
-    while (st.produced < st.cursor + need) {
-        mt_generate_block(mt, a.lds_ring ? reinterpret_cast<uint32_t *>(chain_dyn_lds + a.lds_ring_off) : a.ring,
-                          (uint64_t)(a.ring_words - 1), st.produced);
-        if (threadIdx.x == 0) st.produced += 624;
-        __syncthreads();
-    }
-}
-
-__device__ __forceinline__ uint32_t ring_word(const ChainArgs &a, uint64_t idx) {
-    const uint64_t i = idx & (uint64_t)(a.ring_words - 1);   // ring_words is a power of two
-    if (a.lds_ring) return reinterpret_cast<const uint32_t *>(chain_dyn_lds + a.lds_ring_off)[i];
-    return a.ring[i];
-}
-
-// random() from two words (genrand_res53)
-__device__ __forceinline__ double words_to_random(uint32_t w0, uint32_t w1) {
-    uint32_t x = w0 >> 5, y = w1 >> 6;
-    return (x * 67108864.0 + y) * (1.0 / 9007199254740992.0);
-}
-
-// candidate-set hash term: order dependent, summed over the candidates of a leg
-__device__ __forceinline__ uint32_t cand_mix(uint32_t j, uint32_t target) {
-    uint32_t h = (j * 0x9E3779B9u) ^ target;
-    h ^= h >> 16; h *= 0x85ebca6bu; h ^= h >> 13; h *= 0xc2b2ae35u; h ^= h >> 16;
-    return h;
-}
-
-template <int D>
-__device__ __forceinline__ int pos_to_cell(const ChainArgs &a, const double *p) {
-    long idx = 0;
-#pragma unroll
-    for (int d = 0; d < D; d++) idx += (long)((int)(p[d] / a.side[d])) * a.cum[d];
-    if (idx < 0 || idx >= a.ncells) return -1;
-    return (int)idx;
-}
-
-template <int D>
-__device__ __forceinline__ void load_pos(const ChainArgs &a, int id, double *p) {
-    if (a.lds_pos) {
-        const double *lp = reinterpret_cast<const double *>(chain_dyn_lds);
-#pragma unroll
-        for (int d = 0; d < D; d++) p[d] = lp[d * a.n + id];
-    } else {
-#pragma unroll
-        for (int d = 0; d < D; d++) p[d] = a.pos[(size_t)d * a.n + id];
-    }
-}
-template <int D>
-__device__ __forceinline__ void store_pos(const ChainArgs &a, int id, const double *p) {
-    if (a.lds_pos) {
-        double *lp = reinterpret_cast<double *>(chain_dyn_lds);
-#pragma unroll
-        for (int d = 0; d < D; d++) lp[d * a.n + id] = p[d];
-    } else {
-#pragma unroll
-        for (int d = 0; d < D; d++) a.pos[(size_t)d * a.n + id] = p[d];
-    }
-}
-
-template <int D>
-__device__ __forceinline__ void separation_vector(const ChainArgs &a, const double *ap, const double *tp, double *s) {
-#pragma unroll
-    for (int d = 0; d < D; d++) s[d] = py_mod((tp[d] - ap[d]) + a.half, a.L) - a.half;
-}
-
-// event_handler/abstracts/abstracts.py:82-95 for a velocity with one nonzero component
-template <int D>
-__device__ __forceinline__ void slice_pos(const ChainArgs &a, double *p, int dir, double speed, Time from, Time to) {
-    double dt = time_sub(to, from);
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-        double v = d == dir ? speed : 0.0;
-        p[d] = py_mod(p[d] + v * dt, a.L);
-    }
-}
-
-__device__ __forceinline__ bool pot_draws(const ecmc_tagger_desc &tg) {
-    if (tg.event_handler == ECMC_EH_TWO_LEAF_BOUNDING) return true;
-    return tg.potential != ECMC_POT_HARD_SPHERE && tg.potential != ECMC_POT_HARD_DIPOLE;
-}
-
-// Bounding event rate of a cell-bounding candidate: the InnerPointEstimator bound of the
-// target cell's offset from the active cell along dir, upper or lower by the sign of the
-// charge correction factor (cell_bounding_potential.py:161-201).
-template <int D>
-__device__ __forceinline__ double cell_rate_of_cells(const ChainArgs &a, const ecmc_tagger_desc &tg, int acell, int tcell,
-                                                     int dir, double ca, double ct) {
-    int rel = 0;
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-        const int ti = (tcell / a.cum[d]) % a.cps[d], ai = (acell / a.cum[d]) % a.cps[d];
-        rel += ((ti - ai) % a.cps[d] + a.cps[d]) % a.cps[d] * a.cum[d];
-    }
-    const double *row = a.cbt + (size_t)(rel * 3 + dir) * 2;
-    if (tg.use_charge) {
-        const double cf = ca * ct / tg.bpar[2];
-        return cf > 0.0 ? row[0] * cf : row[1] * cf;
-    }
-    return row[0];
-}
-// The same for a target unit, its cell from its position.
-template <int D>
-__device__ __forceinline__ double cell_rate(const ChainArgs &a, const ecmc_tagger_desc &tg, int acell, int target, int dir,
-                                            double ca, double ct) {
-    double tp[D];
-    load_pos<D>(a, target, tp);
-    return cell_rate_of_cells<D>(a, tg, acell, pos_to_cell<D>(a, tp), dir, ca, ct);
-}
-
-// Is cell c among the nearby cells of cell ac (within `layers` per axis, periodic)?
-__device__ __forceinline__ bool is_nearby(const ChainArgs &a, int dim, int c, int ac) {
-    for (int d = 0; d < dim; d++) {
-        const int ci = (c / a.cum[d]) % a.cps[d], ai = (ac / a.cum[d]) % a.cps[d];
-        const int off = ((ci - ai) % a.cps[d] + a.cps[d]) % a.cps[d];
-        if (off > a.layers && off < a.cps[d] - a.layers) return false;
-    }
-    return true;
-}
-
-// Kernel variants by the features of the systems they run (FM): bit p for the two-leaf pair
-// potential ECMC_POT_p inverted exactly, FEAT_COULOMB for the merged-image Coulomb factors through
-// the inverse-power Coulomb bound (thinning by the Ewald derivative), FEAT_FMAP for factor-type
-// maps, FEAT_CELL_BOUNDING and FEAT_CELL_VETO for the two far-cell schemes.  A variant leaves the
-// code of the other features out of the kernel (a smaller leg loop, fewer instruction-cache
-// misses); the host launches the first variant that covers every feature of its systems.
-constexpr int FEAT_COULOMB = 1 << 9, FEAT_FMAP = 1 << 10, FEAT_CELL_BOUNDING = 1 << 11, FEAT_CELL_VETO = 1 << 12;
-constexpr int FEAT_ALL = (1 << 13) - 1;
-constexpr int FEAT_EWALD = FEAT_COULOMB | FEAT_CELL_BOUNDING | FEAT_CELL_VETO;   // thinning by the Ewald derivative
-constexpr int FEAT_IP_FILTER = (1 << ECMC_POT_INVERSE_POWER) | (1 << ECMC_POT_INVERSE_POWER_TRUNC);
-constexpr int VARIANT_LJ = FEAT_IP_FILTER;
-constexpr int VARIANT_CHARGED_CB = (1 << ECMC_POT_INVERSE_POWER) | FEAT_COULOMB | FEAT_CELL_BOUNDING;
-constexpr int VARIANT_CHARGED_CV = (1 << ECMC_POT_INVERSE_POWER) | FEAT_COULOMB | FEAT_CELL_VETO;
-constexpr int VARIANT_DIPOLES = (1 << ECMC_POT_INVERSE_POWER) | (1 << ECMC_POT_DISPLACED_EVEN_POWER) | FEAT_COULOMB | FEAT_FMAP;
-#define POT_BUILT(p) ((FM >> (p)) & 1)
-
-// Candidate time displacement of one pair (send_event_time of the pair event handlers).
-template <int D, int FM>
-__device__ __forceinline__ double pair_dt(const ChainArgs &a, const ecmc_tagger_desc &tg, int dir, double speed, const double *s,
-                          double c1, double c2, double dU) {
-    if (tg.event_handler == ECMC_EH_TWO_LEAF) {
-        switch (tg.potential) {
-        case ECMC_POT_HARD_SPHERE:
-            if (!POT_BUILT(ECMC_POT_HARD_SPHERE)) return NAN;
-            return hs_displacement<D>(dir, speed, s, tg.par[0]);
-        case ECMC_POT_HARD_DIPOLE:
-            if (!POT_BUILT(ECMC_POT_HARD_DIPOLE)) return NAN;
-            return hd_displacement<D>(dir, speed, s, tg.par[0], tg.par[1]);
-        case ECMC_POT_INVERSE_POWER:
-            if (!POT_BUILT(ECMC_POT_INVERSE_POWER)) return NAN;
-            return ip_displacement<D>(dir, speed, s, c1, c2, tg.par[0], tg.par[1], dU);
-        case ECMC_POT_INVERSE_POWER_TRUNC:
-            if (!POT_BUILT(ECMC_POT_INVERSE_POWER_TRUNC)) return NAN;
-            return ipt_displacement<D>(dir, speed, s, c1, c2, tg.par[0], tg.par[1], tg.par[2], dU);
-        case ECMC_POT_LENNARD_JONES: {
-            if (!POT_BUILT(ECMC_POT_LENNARD_JONES)) return NAN;
-            MexicanHat h = mh_lennard_jones(tg.par[0], tg.par[1]);
-            return mh_displacement<D>(h, dir, speed, s, dU);
-        }
-        case ECMC_POT_DISPLACED_EVEN_POWER: {
-            if (!POT_BUILT(ECMC_POT_DISPLACED_EVEN_POWER)) return NAN;
-            MexicanHat h = mh_displaced_even_power(tg.par[0], tg.par[1], tg.par[2]);
-            return mh_displacement<D>(h, dir, speed, s, dU);
-        }
-        default: return NAN;
-        }
-    }
-    // two_leaf_unit_bounding_potential_event_handler.py:138-143 with the Coulomb bound
-    if (!(FM & FEAT_COULOMB)) return NAN;
-    double p[3] = {0, 0, 0};
-#pragma unroll
-    for (int d = 0; d < 3; d++) p[d] = d < D ? s[(dir + d) % D] : 0.0;
-    return ipcb_displacement(tg.bpar[0] * c1 * c2, p[0], p[1], p[2], dU, a.L) / speed;
-}
-
-// Candidate j of a factor-map tagger (factor_type_maps.py:325-356): a local factor's entries for
-// the active leaf number k; a non-local factor's entries for every other composite object in
-// identifier order, the entry's other leaf in that object (or, for numbers below P, in the
-// active unit's own object).
-__device__ __forceinline__ int fmap_target(const ecmc_tagger_desc &tg, int P, int act, int j) {
-    const int m = act / P, k = act % P, fn = tg.fmap_n[k];
-    if (tg.fmap_local) return m * P + tg.fmap_target[k][j];
-    const int o = j / fn, e = j - o * fn;
-    const int other = o < m ? o : o + 1;
-    const int tl = tg.fmap_target[k][e];
-    return tl < P ? m * P + tl : other * P + (tl - P);
-}
-__device__ __forceinline__ int fmap_count(const ecmc_tagger_desc &tg, int P, int n, int act) {
-    const int fn = tg.fmap_n[act % P];
-    return tg.fmap_local ? fn : (n / P - 1) * fn;
-}
-
-struct Best {
-    double q, r;
-    int32_t j;
-};
-__device__ __forceinline__ bool best_lt(const Best &x, const Best &y) {
-    if (x.q < y.q) return true;
-    if (x.q == y.q) {
-        if (x.r < y.r) return true;
-        if (x.r == y.r) return x.j < y.j;
-    }
-    return false;
-}
-
-// One butterfly step within the 16-lane rows by a DPP lane permutation (CTRL: 0xB1 swaps
-// neighbours, 0x4E pairs of neighbours, 0x141 mirrors each half row, 0x140 the row): after the
-// four steps every lane of a row holds the row's least (time, index) and its hash sum.
-template <int CTRL>
-__device__ __forceinline__ int dpp_move(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false); }
-template <int CTRL>
-__device__ __forceinline__ double dpp_move_d(double v) {
-    return __hiloint2double(dpp_move<CTRL>(__double2hiint(v)), dpp_move<CTRL>(__double2loint(v)));
-}
-template <int CTRL>
-__device__ __forceinline__ void best_dpp_step(Best &b, uint32_t &h) {
-    Best o;
-    o.q = dpp_move_d<CTRL>(b.q);
-    o.r = dpp_move_d<CTRL>(b.r);
-    o.j = dpp_move<CTRL>(b.j);
-    const uint32_t oh = (uint32_t)dpp_move<CTRL>((int)h);
-    if (best_lt(o, b)) b = o;
-    h += oh;
-}
-
-// Collective workgroup min-reduce of (time, index) and sum of the hash terms: DPP steps within
-// each row, shuffles across the rows, LDS across the wavefronts.  The order is total (indices
-// are distinct) and the sum wraps, so the result does not depend on the reduction order.
-__device__ __forceinline__ void block_reduce(Best &b, uint32_t &h, Best *sb, uint32_t *sh) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    best_dpp_step<0xB1>(b, h);
-    best_dpp_step<0x4E>(b, h);
-    best_dpp_step<0x141>(b, h);
-    best_dpp_step<0x140>(b, h);
-#pragma unroll
-    for (int off = 32; off >= 16; off >>= 1) {
-        Best o;
-        o.q = __shfl_xor(b.q, off, 64);
-        o.r = __shfl_xor(b.r, off, 64);
-        o.j = __shfl_xor(b.j, off, 64);
-        uint32_t oh = __shfl_xor(h, off, 64);
-        if (best_lt(o, b)) b = o;
-        h += oh;
-    }
-    if (lane == 0) { sb[wave] = b; sh[wave] = h; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < NT / 64; w++) {
-            if (best_lt(sb[w], sb[0])) sb[0] = sb[w];
-            sh[0] += sh[w];
-        }
-    }
-    __syncthreads();
-    b = sb[0];
-    h = sh[0];
-}
-
-// Collective workgroup minimum of a non-negative float (+inf allowed); sh holds NT / 64 words.
-__device__ __forceinline__ float block_min_float(float v, uint32_t *sh) {
-    v = fminf(v, __int_as_float(dpp_move<0xB1>(__float_as_int(v))));
-    v = fminf(v, __int_as_float(dpp_move<0x4E>(__float_as_int(v))));
-    v = fminf(v, __int_as_float(dpp_move<0x141>(__float_as_int(v))));
-    v = fminf(v, __int_as_float(dpp_move<0x140>(__float_as_int(v))));
-#pragma unroll
-    for (int off = 32; off >= 16; off >>= 1) v = fminf(v, __shfl_xor(v, off, 64));
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = __float_as_uint(v);
-    __syncthreads();
-    float r = __uint_as_float(sh[0]);
-    for (int w = 1; w < NT / 64; w++) r = fminf(r, __uint_as_float(sh[w]));
-    __syncthreads();
-    return r;
-}
-
-// The candidate sets whose exact inversions are filtered by FP32 brackets first: two-leaf
-// inverse-power factors (plain and truncated-and-shifted) of an integer power up to 32.  The
-// Coulomb bound's sets are inverted exactly: its brackets (ipcb_time_bounds) cost nearly as much
-// as its exact inversion, and filtering them measured slower.
-__device__ __forceinline__ bool fp32_filter_applies(const ecmc_tagger_desc &tg) {
-    if (tg.event_handler != ECMC_EH_TWO_LEAF) return false;
-    if (tg.potential != ECMC_POT_INVERSE_POWER && tg.potential != ECMC_POT_INVERSE_POWER_TRUNC) return false;
-    const double p = tg.par[0];
-    return p >= 1.0 && p <= 32.0 && p == floor(p);
-}
-
-template <int D, int FM>
-__device__ __forceinline__ void create_pair(const ChainArgs &a, ChainState &st, uint32_t *mt, const ecmc_tagger_desc &tg, int tix,
-                            int *nb_cell, int *nb_pref, Best *sb, uint32_t *sh, int *scan) {
-    const int tid = threadIdx.x;
-    if (tg.kind == ECMC_TAG_PAIR_CELLS) {
-        // the nearby cells (at most 27) and the prefix sums of their occupant counts: one lane
-        // per cell of the first wavefront, an inclusive scan by shuffles
-        if (tid < 64) {
-            const int cell = st.occ_cell;
-            const int cnt = a.nearby_n[cell];
-            int cc = 0, num = 0;
-            if (tid < cnt) {
-                cc = a.nearby[(size_t)cell * a.nb_stride + tid];
-                num = occn_base(a)[cc];
-            }
-            int incl = num;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int v = __shfl_up(incl, o, 64);
-                if (tid >= o) incl += v;
-            }
-            if (tid < cnt) {
-                nb_cell[tid] = cc;
-                nb_pref[tid + 1] = incl;
-            }
-            if (tid == 0) {
-                nb_pref[0] = 0;
-                nb_cell[31] = cnt;
-            }
-        }
-    } else if (tid == 0) {
-        nb_pref[0] = 0;
-        nb_pref[1] = a.n;  // identifiers 0..n-1 minus the active one
-        nb_cell[31] = 1;
-    }
-    __syncthreads();
-    const int nc = nb_cell[31];
-    const bool all = tg.kind == ECMC_TAG_PAIR_ALL;
-    const bool sur = tg.kind == ECMC_TAG_SURPLUS;
-    const bool far = (FM & FEAT_CELL_BOUNDING) && tg.kind == ECMC_TAG_CELL_BOUNDING;
-    const bool fmap = (FM & FEAT_FMAP) && tg.kind == ECMC_TAG_FACTOR_MAP;
-    // the far cells of this create (built and read within it): in LDS when the launch has room
-    int32_t *const cand = a.lds_cand_off >= 0 ? reinterpret_cast<int32_t *>(chain_dyn_lds + a.lds_cand_off) : a.cand;
-    if (far) {
-        // cell_bounding_potential_tagger.py:150-155: the occupied cells that are not nearby the
-        // active cell, in cell order; each threads scans a contiguous run of cells, an
-        // exclusive scan of the counts places its candidates
-        const int ac = st.occ_cell;
-        const int chunk = (a.ncells + NT - 1) / NT;
-        const int lo = min(tid * chunk, a.ncells), hi = min(lo + chunk, a.ncells);
-        // the occupied far cells of this thread's run, as bits when the run has at most 32 cells
-        const bool use_bits = chunk <= 32;
-        uint32_t bits = 0;
-        int cnt = 0;
-        for (int c = lo; c < hi; c++)
-            if (occn_base(a)[c] > 0 && !is_nearby(a, D, c, ac)) {
-                cnt++;
-                if (use_bits) bits |= 1u << (c - lo);
-            }
-        // exclusive scan of the counts over the workgroup: shuffles within each wavefront, the
-        // wavefront totals in scan[NT + 1 ..]
-        const int lane = tid & 63, wave = tid >> 6;
-        int incl = cnt;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += v;
-        }
-        if (lane == 63) scan[NT + 1 + wave] = incl;
-        __syncthreads();
-        int before = 0;
-        for (int w = 0; w < wave; w++) before += scan[NT + 1 + w];
-        int k = before + incl - cnt;
-        if (tid == NT - 1) scan[NT] = before + incl;
-        bool multi = false;
-        for (int c = lo; c < hi; c++)
-            if (use_bits ? ((bits >> (c - lo)) & 1u) != 0 : (occn_base(a)[c] > 0 && !is_nearby(a, D, c, ac))) {
-                if (occn_base(a)[c] != 1) multi = true;
-                cand[k++] = c;   // the cell; its one occupant is the candidate
-            }
-        if (multi) st.err = ECMC_ERR_STATE;   // the handler takes exactly one target unit
-        __syncthreads();
-    }
-    const int M = fmap ? (st.active < 0 ? 0 : fmap_count(tg, a.leaves, a.n, st.active))
-                       : (all ? a.n - 1 : (sur ? st.nsur : (far ? scan[NT] : nb_pref[nc])));
-    const bool draws = pot_draws(tg);
-    ring_ensure(st, mt, a, draws ? 2ull * (uint64_t)M : 0ull);
-    const uint64_t base = st.cursor;
-    const int act = st.active, dir = st.adir;
-    const double speed = st.aspeed;
-    const Time at = st.at;
-    double ap[D];
-    load_pos<D>(a, act, ap);
-    const double ca = tg.use_charge ? charge_of(a, act) : 1.0;
-    const int jbase = st.ncand;
-    Best best = {INFINITY, INFINITY, 0x7fffffff};
-    uint32_t hsum = 0;
-    auto cand_target = [&](int j) {
-        if (fmap) return fmap_target(tg, a.leaves, act, j);
-        if (all) return j < act ? j : j + 1;
-        if (sur) return (int)a.sur_id[j];
-        if (far) return (int)occ_base(a)[(size_t)cand[j] * a.occ_cap];
-        // the nearby cell holding candidate j: the largest c with nb_pref[c] <= j (binary search
-        // over the nc + 1 prefix sums; empty cells repeat a prefix)
-        int lo = 0, hi = nc;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (nb_pref[mid] <= j) lo = mid;
-            else hi = mid;
-        }
-        return (int)occ_base(a)[(size_t)nb_cell[lo] * a.occ_cap + (j - nb_pref[lo])];
-    };
-    // FP32 filter: every candidate's time displacement is bracketed [lb, ub] from its separation
-    // and the leading word of its draw; a candidate whose lb exceeds the smallest ub of the set
-    // by more than the rounding of the active time can make up ends strictly later, so it can
-    // be neither the earliest nor tie with it and is not inverted exactly; lb = +inf marks a
-    // candidate without an event.  The earliest candidate and every candidate of equal time are
-    // inverted exactly as before, so the result is the unfiltered one, unless a candidate left
-    // out would have raised the reference's ValueError (a negative square root from rounding),
-    // which the exact inversion flags.
-    const bool filt = (FM & FEAT_IP_FILTER) && fp32_filter_applies(tg) && M > 1;
-    float lbk0 = 0.f, lbk1 = 0.f;
-    double cull_above = INFINITY;
-    const int fp = (int)tg.par[0];
-    const float two_over_p = 2.f / (float)fp;
-    const bool ftrunc = tg.potential == ECMC_POT_INVERSE_POWER_TRUNC;
-    const float rc2f = ftrunc ? (float)(tg.par[2] * tg.par[2]) : 0.f;
-    const float ibf = (float)(1.0 / a.beta), isf = (float)(1.0 / speed);
-    // the separation of the brackets: the difference wrapped by one box length, within two ulps
-    // of L of separation_vector's Python-modulo form except near +-L/2, where the candidate keeps
-    // the trivial brackets
-    const double edge = a.half * (1.0 - 0x1p-40);
-    const float sep_slack = (float)(a.L * 0x1p-49);
-    auto cand_bounds = [&](int j, int target, float &lb, float &ub) {
-        double tp[D], s[D];
-        load_pos<D>(a, target, tp);
-        bool near_edge = false;
-#pragma unroll
-        for (int d = 0; d < D; d++) {
-            double v = tp[d] - ap[d];
-            v = v >= a.half ? v - a.L : (v < -a.half ? v + a.L : v);
-            near_edge = near_edge || !(fabs(v) < edge);
-            s[d] = v;
-        }
-        const double ct = tg.use_charge ? charge_of(a, target) : 1.0;
-        lb = 0.f;
-        ub = INFINITY;
-        const double pp = tg.par[1] * (ca * ct);
-        const float K = (float)fabs(pp);
-        if (!near_edge && K >= 0x1p-100f && K <= 0x1p100f) {
-            const uint32_t w0 = ring_word(a, base + 2ull * j);
-            ip_time_bounds<D>(s, dir, K, pp > 0.0, fp, two_over_p, ftrunc, dn(rc2f), up(rc2f),
-                              dU_lower(w0, ibf * (1.f - 0x1p-22f)), dU_upper(w0, ibf * (1.f + 0x1p-22f)),
-                              isf * (1.f - 0x1p-22f), isf * (1.f + 0x1p-22f), lb, ub, sep_slack);
-        }
-    };
-    if (filt) {
-        float ubmin = INFINITY;
-        // two candidates per iteration, evaluated side by side (the second one a repeat of the
-        // first past the end of the set, its result dropped)
-        for (int j0 = tid; j0 < M; j0 += 2 * NT) {
-            const int j1 = j0 + NT;
-            const bool has1 = j1 < M;
-            const int t0 = cand_target(j0), t1 = cand_target(has1 ? j1 : j0);
-            float lb0, ub0, lb1, ub1;
-            cand_bounds(j0, t0, lb0, ub0);
-            cand_bounds(has1 ? j1 : j0, t1, lb1, ub1);
-            if (j0 == tid) {
-                lbk0 = lb0;
-                lbk1 = lb1;
-            }
-            ubmin = fminf(ubmin, ub0);
-            hsum += cand_mix((uint32_t)(jbase + j0), (uint32_t)t0);
-            if (has1) {
-                ubmin = fminf(ubmin, ub1);
-                hsum += cand_mix((uint32_t)(jbase + j1), (uint32_t)t1);
-            }
-        }
-        ubmin = block_min_float(ubmin, sh);
-        // a displacement beyond ubmin + 2^-48 (1 + ubmin) ends later than ubmin does: the active
-        // time's remainder lies in [0, 1), so the two sums with it round to doubles at least one
-        // ulp apart, and Time's divmod by one keeps their order strict
-        if (ubmin < INFINITY) cull_above = (double)ubmin + 0x1p-48 * (1.0 + (double)ubmin);
-    }
-    int kk = 0;
-    for (int j = tid; j < M; j += NT, kk++) {
-        if (filt) {
-            float lb, ub;
-            if (kk == 0) lb = lbk0;
-            else if (kk == 1) lb = lbk1;
-            else cand_bounds(j, cand_target(j), lb, ub);
-            if (lb == INFINITY) {
-                const Best c = {INFINITY, INFINITY, j};
-                if (best_lt(c, best)) best = c;
-                continue;
-            }
-            // lb = 0 never culls: the exact FP64 displacement can round below zero there
-            if (lb > 0.f && (double)lb > cull_above) continue;
-        }
-        const int target = cand_target(j);
-        double tp[D], s[D];
-        load_pos<D>(a, target, tp);
-        separation_vector<D>(a, ap, tp, s);
-        double dU = 0.0;
-        if (draws) {
-            double u = words_to_random(ring_word(a, base + 2ull * j), ring_word(a, base + 2ull * j + 1));
-            dU = -cr_log(1.0 - u) / a.beta;
-        }
-        const double ct = tg.use_charge ? charge_of(a, target) : 1.0;
-        double dt;
-        if ((FM & FEAT_CELL_BOUNDING) && tg.event_handler == ECMC_EH_CELL_BOUNDING) {
-            // two_leaf_unit_cell_bounding_potential_event_handler.py:171-177
-            const double rate = far ? cell_rate_of_cells<D>(a, tg, st.occ_cell, (int)cand[j], dir, ca, ct)
-                                    : cell_rate<D>(a, tg, st.occ_cell, target, dir, ca, ct);
-            dt = (rate > 0 ? dU / rate : INFINITY) / speed;
-        } else {
-            dt = pair_dt<D, FM>(a, tg, dir, speed, s, ca, ct, dU);
-        }
-        Time t = time_add(at, dt);
-        Best c = {t.q, t.r, j};
-        if (isnan(dt)) c.q = -INFINITY;  // flags a ValueError of the reference code
-        if (best_lt(c, best)) best = c;
-        if (!filt) hsum += cand_mix((uint32_t)(jbase + j), (uint32_t)target);
-    }
-    block_reduce(best, hsum, sb, sh);
-    if (tid == 0) {
-        if (draws) st.cursor += 2ull * (uint64_t)M;
-        st.ncand += M;
-        st.chash += hsum;
-        Slot &sl = st.slot[tix];
-        if (M == 0) {
-            sl.valid = 0;
-        } else if (best.q == -INFINITY) {
-            st.err = ECMC_ERR_NUMERIC;
-        } else {
-            const int j = best.j, target = cand_target(j);
-            sl.valid = 1;
-            sl.cb_cell = st.occ_cell;
-            sl.t.q = best.q;
-            sl.t.r = best.r;
-            sl.seq = st.seq + j;
-            sl.target = target;
-            sl.adir = dir;
-            sl.aspeed = speed;
-            double tp[D];
-            load_pos<D>(a, target, tp);
-            double p[D];
-#pragma unroll
-            for (int d = 0; d < D; d++) { p[d] = ap[d]; sl.tpos[d] = tp[d]; }
-            if (!isinf(sl.t.q)) slice_pos<D>(a, p, dir, speed, at, sl.t);
-#pragma unroll
-            for (int d = 0; d < D; d++) sl.apos[d] = p[d];
-            sl.astamp = sl.t;
-        }
-        st.seq += M;
-    }
-    __syncthreads();
-}
-
-// Collective: moves the entries [from, to) of the parallel arrays x and y (y may be NULL) by
-// one slot up (by > 0) or down, in chunks of one entry per thread, every chunk read before it
-// is written and the chunks ordered so that no entry is overwritten before it was read.
-__device__ __forceinline__ void shift_entries(int32_t *x, int32_t *y, int from, int to, int by) {
-    const int tid = threadIdx.x;
-    if (by > 0) {
-        for (int top = to; top > from; top -= NT) {
-            const int lo = top - NT > from ? top - NT : from, i = lo + tid;
-            const bool act = i < top;
-            int32_t vx = 0, vy = 0;
-            if (act) { vx = x[i]; if (y) vy = y[i]; }
-            __syncthreads();
-            if (act) { x[i + 1] = vx; if (y) y[i + 1] = vy; }
-            __syncthreads();
-        }
-    } else {
-        for (int lo = from; lo < to; lo += NT) {
-            const int i = lo + tid;
-            const bool act = i < to;
-            int32_t vx = 0, vy = 0;
-            if (act) { vx = x[i]; if (y) vy = y[i]; }
-            __syncthreads();
-            if (act) { x[i - 1] = vx; if (y) y[i - 1] = vy; }
-            __syncthreads();
-        }
-    }
-}
-
-// Collective: the largest (want_max) or smallest index i < count with x[i] == vx and, when y is
-// given, y[i] == vy; -1 when there is none.  red holds NT / 64 ints of workgroup scratch.
-__device__ __forceinline__ int find_entry(const int32_t *x, const int32_t *y, int count, int32_t vx, int32_t vy, bool want_max,
-                          int *red) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int best = want_max ? -1 : 0x7fffffff;
-    for (int i = tid; i < count; i += NT)
-        if (x[i] == vx && (!y || y[i] == vy)) best = want_max ? (i > best ? i : best) : (i < best ? i : best);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const int v = __shfl_xor(best, o, 64);
-        best = want_max ? (v > best ? v : best) : (v < best ? v : best);
-    }
-    if (lane == 0) red[wave] = best;
-    __syncthreads();
-    int r = red[0];
-    for (int w = 1; w < NT / 64; w++) r = want_max ? (red[w] > r ? red[w] : r) : (red[w] < r ? red[w] : r);
-    __syncthreads();
-    return r == 0x7fffffff ? -1 : r;
-}
-
-// Collective, single_active_cell_occupancy.py:149-203: the unit that stops being active joins
-// its cell's occupants, or the surplus when the cell is full (self._surplus.setdefault(cell,
-// []).append(id) on the flat list in dict order: after the cell's last surplus entry, or at the
-// end); the new active unit leaves the occupants or the surplus (the surplus never moves into
-// the occupants: that branch of the reference needs an empty surplus list, which it deletes
-// right away).  The list searches and shifts run over the workgroup.
-template <int D>
-__device__ __forceinline__ void occupancy_update(const ChainArgs &a, ChainState &st, int *red) {
-    const int tid = threadIdx.x;
-    const int id = st.active, old_id = st.occ_id, old_cell = st.occ_cell;
-    const int n_old = (id != old_id && old_id >= 0) ? occn_base(a)[old_cell] : 0;
-    double p[D];
-    load_pos<D>(a, id, p);
-    const int c = pos_to_cell<D>(a, p);
-    __syncthreads();   // every thread has read the state and the counts before thread 0 changes them
-    if (id == old_id) {
-        if (tid == 0) {
-            if (c < 0) st.err = ECMC_ERR_STATE;
-            else st.occ_cell = c;
-        }
-        __syncthreads();
-        return;
-    }
-    if (old_id >= 0) {
-        const int n = n_old;
-        if (a.max_occ <= 0 || n < a.max_occ) {
-            if (tid == 0) {
-                if (n >= a.occ_cap) st.err = ECMC_ERR_STATE;
-                else {
-                    occ_base(a)[(size_t)old_cell * a.occ_cap + n] = old_id;
-                    occn_base(a)[old_cell] = n + 1;
-                }
-            }
-        } else {
-            const int nsur = st.nsur;
-            if (nsur >= a.sur_cap) {
-                if (tid == 0) st.err = ECMC_ERR_STATE;
-            } else {
-                const int last = find_entry(a.sur_cell, nullptr, nsur, old_cell, 0, true, red);
-                const int at = last >= 0 ? last + 1 : nsur;
-                shift_entries(a.sur_cell, a.sur_id, at, nsur, +1);
-                if (tid == 0) {
-                    a.sur_cell[at] = old_cell;
-                    a.sur_id[at] = old_id;
-                    st.nsur = nsur + 1;
-                }
-            }
-        }
-        __syncthreads();
-        if (st.err) return;
-    }
-    if (c < 0) {
-        if (tid == 0) st.err = ECMC_ERR_STATE;
-        __syncthreads();
-        return;
-    }
-    int32_t *Lc = occ_base(a) + (size_t)c * a.occ_cap;
-    const int n = occn_base(a)[c];
-    const int i = find_entry(Lc, nullptr, n, id, 0, false, red);
-    if (i >= 0) {
-        shift_entries(Lc, nullptr, i + 1, n, -1);
-        if (tid == 0) occn_base(a)[c] = n - 1;
-    } else {
-        const int nsur = st.nsur;
-        const int k = find_entry(a.sur_cell, a.sur_id, nsur, c, id, false, red);
-        if (k < 0) {
-            if (tid == 0) st.err = ECMC_ERR_STATE;
-        } else {
-            shift_entries(a.sur_cell, a.sur_id, k + 1, nsur, -1);
-            if (tid == 0) st.nsur = nsur - 1;
-        }
-    }
-    if (tid == 0) {
-        st.occ_cell = c;
-        st.occ_id = id;
-    }
-    __syncthreads();
-}
-
-// Creates of one non-pair tagger (thread 0 only, ring words made available by the caller).
-template <int D>
-__device__ __forceinline__ void create_single(const ChainArgs &a, ChainState &st, const ecmc_tagger_desc &tg, int tix) {
-    Slot &sl = st.slot[tix];
-    switch (tg.kind) {
-    case ECMC_TAG_CELL_BOUNDARY: {
-        // cell_boundary_event_handler.py:98-156
-        double p[D];
-        load_pos<D>(a, st.active, p);
-        int cell = pos_to_cell<D>(a, p);
-        if (cell < 0) { st.err = ECMC_ERR_STATE; return; }
-        int dir = st.adir;
-        int id = (cell / a.cum[dir]) % a.cps[dir];
-        int nid = (id + 1) % a.cps[dir];
-        int nb = cell + (nid - id) * a.cum[dir];
-        double boundary = a.cmin[(size_t)nb * D + dir];
-        double sep = boundary - p[dir];
-        if (sep < 0.0) sep = sep + a.L;
-        double dt = sep / st.aspeed;
-        sl.t = time_add(st.at, dt);
-#pragma unroll
-        for (int d = 0; d < D; d++) sl.apos[d] = p[d];
-        sl.astamp = st.at;
-        sl.cb_boundary = boundary;
-        sl.cb_dir = dir;
-        sl.adir = dir;
-        sl.aspeed = st.aspeed;
-        sl.valid = 1;
-        sl.seq = st.seq++;
-        break;
-    }
-    case ECMC_TAG_SAMPLING:
-        st.samp_time = time_add(st.samp_time, tg.value);
-        sl.t = st.samp_time;
-        sl.valid = 1;
-        sl.seq = st.seq++;
-        break;
-    case ECMC_TAG_END_OF_RUN:
-        sl.t = time_from_float(tg.value);
-        sl.valid = 1;
-        sl.seq = st.seq++;
-        break;
-    case ECMC_TAG_START_OF_RUN:
-        sl.t.q = 0.0;
-        sl.t.r = 0.0;
-        sl.valid = 1;
-        sl.seq = st.seq++;
-        break;
-    default: break;
-    }
-}
-
-// end of chain: chain time and the randint of the next active unit
-// (single_independent_active_periodic_direction_end_of_chain_event_handler.py:176-237): with
-// composite objects the root's randint, then the leaf's.  Returns false when the ring ran out of
-// words before the draws completed; the root already drawn is kept in the slot (cv_index).
-__device__ __forceinline__ bool create_end_of_chain(const ChainArgs &a, ChainState &st, const ecmc_tagger_desc &tg, int tix) {
-    Slot &sl = st.slot[tix];
-    if (!sl.valid || sl.target >= 0x40000000) {
-        if (!sl.valid || sl.target != 0x40000000) {
-            double since = time_sub(st.at, st.eoc_last);
-            if (!(0.0 <= since && since <= tg.value)) { st.err = ECMC_ERR_CONFIGURATION; return true; }
-            double chain = time_sub(st.eoc_last, st.at) + tg.value;
-            sl.t = time_add(st.at, chain);
-            sl.valid = 1;
-            sl.target = 0x40000000;  // draws pending
-            sl.cv_index = -1;        // no root drawn yet
-        }
-    }
-    const int P = a.leaves;
-    while (true) {
-        const bool root_phase = sl.cv_index < 0;
-        const uint32_t nrange = root_phase ? (uint32_t)(a.n / P) : (uint32_t)P;
-        int k = 0;
-        while ((nrange >> k) != 0u) k++;
-        bool got = false;
-        uint32_t v = 0;
-        while (st.cursor < st.produced) {
-            uint32_t w = ring_word(a, st.cursor);
-            st.cursor++;
-            v = k >= 32 ? w : (w >> (32 - k));
-            if (v < nrange) { got = true; break; }
-        }
-        if (!got) return false;
-        if (root_phase && P > 1) {
-            sl.cv_index = (int32_t)v;
-            continue;
-        }
-        sl.target = root_phase ? (int32_t)v : sl.cv_index * P + (int32_t)v;
-        sl.seq = st.seq++;
-        return true;
-    }
-}
-
-// cell veto send_event_time (cell_veto_event_handler.py:190-238): the Walker table by the sign
-// of the charge correction factor; random.choice over its entries (rejection on bit_length
-// words), uniform(0, mean) for item or alias, then expovariate / (total rate * speed).
-// Thread 0 only.  Returns false when the ring ran out of words; the drawn entry is kept in the
-// slot, so the call resumes after a refill.
-template <int D>
-__device__ __forceinline__ bool create_cell_veto(const ChainArgs &a, ChainState &st, const ecmc_tagger_desc &tg, int tix) {
-    Slot &sl = st.slot[tix];
-    const int act = st.active, dir = st.adir;
-    double cf = (tg.use_charge ? charge_of(a, act) : 1.0) * 1.0 / tg.bpar[2];
-    int b = 0;
-    if (!(cf > 0.0)) { cf *= -1.0; b = 1; }
-    const int wt = dir * 2 + b;
-    const uint32_t m = (uint32_t)a.cv_m;
-    if (sl.cv_phase != 2) {
-        sl.cv_phase = 1;
-        int k = 0;
-        while ((m >> k) != 0u) k++;
-        while (st.cursor < st.produced) {
-            const uint32_t w = ring_word(a, st.cursor);
-            st.cursor++;
-            const uint32_t v = k >= 32 ? w : (w >> (32 - k));
-            if (v < m) { sl.cv_index = (int32_t)v; sl.cv_phase = 2; break; }
-        }
-        if (sl.cv_phase != 2) return false;
-    }
-    if (st.produced - st.cursor < 4) return false;
-    const CvEntry e = a.cvw[(size_t)wt * m + sl.cv_index];
-    const double u = 0.0 + (a.cv_mean[wt] - 0.0) * words_to_random(ring_word(a, st.cursor), ring_word(a, st.cursor + 1));
-    const int rel = u <= e.rate0 ? e.item0 : e.item1;
-    const double u2 = words_to_random(ring_word(a, st.cursor + 2), ring_word(a, st.cursor + 3));
-    const double dU = -cr_log(1.0 - u2) / a.beta;
-    st.cursor += 4;
-    sl.cv_phase = 0;
-    const double total = a.cv_total[wt] * cf;
-    const double row = a.cbt[(size_t)(rel * 3 + dir) * 2 + b];
-    sl.cv_rate = (b ? -row : row) * cf;
-    if (!(sl.cv_rate > 0.0) || rel < 0) { st.err = ECMC_ERR_NUMERIC; return true; }
-    double ap[D];
-    load_pos<D>(a, act, ap);
-    const int acell = pos_to_cell<D>(a, ap);
-    // cuboid_periodic_cells.py:182-207: the cell centre shifted by the relative cell's lower
-    // corner lies half a cell from every wall, so the per-axis identifier sum is that cell
-    int tcell = 0;
-#pragma unroll
-    for (int d = 0; d < D; d++) {
-        const int ai = (acell / a.cum[d]) % a.cps[d], ri = (rel / a.cum[d]) % a.cps[d];
-        tcell += ((ai + ri) % a.cps[d]) * a.cum[d];
-    }
-    const double dt = dU / (total * st.aspeed);
-    sl.t = time_add(st.at, dt);
-    sl.valid = 1;
-    sl.seq = st.seq++;
-    sl.target = -1;
-    sl.cb_cell = tcell;
-    sl.adir = dir;
-    sl.aspeed = st.aspeed;
-    if (!isinf(sl.t.q)) slice_pos<D>(a, ap, dir, st.aspeed, st.at, sl.t);
-#pragma unroll
-    for (int d = 0; d < D; d++) sl.apos[d] = ap[d];
-    sl.astamp = sl.t;
-    return true;
-}
-
-// ewald_derivative over one wavefront, all 64 lanes calling with the same separation.  The
-// host lists the terms of the sequential loop (the real-space images by k, j, i, then the
-// Fourier terms by i, j, k); term g belongs to lane g % 64, slot g / 64.  Each lane evaluates
-// its terms with the sequential loop's operations (a Fourier factor by stepping the same
-// cos/sin recurrence from its start as far as that term), adds its slots in order, and a
-// butterfly over the lanes adds the 64 partial sums (commutative pairings, so every lane ends
-// with the same sum).  The order of the additions differs from the sequential loop's, so the
-// result agrees with it to rounding.  More than 256 terms fall back to the sequential function.
-// The sequential form where the wave form does not apply: called, not inlined (a rare path).
-__device__ __noinline__ static double ewald_derivative_call(const Ewald &e, double sx, double sy, double sz) {
-    return ewald_derivative(e, sx, sy, sz);
-}
-__device__ __forceinline__ double ewald_derivative_wave(const Ewald &e, const int32_t *codes, int ncodes, double sx, double sy,
-                                        double sz) {
-    if (ncodes > 256 || !codes) return ewald_derivative_call(e, sx, sy, sz);
-    const int lane = threadIdx.x & 63;
-    const int n = e.fc + 1;
-    const double L = e.L;
-    int code[4];
-#pragma unroll
-    for (int s = 0; s < 4; s++) code[s] = lane + 64 * s < ncodes ? codes[lane + 64 * s] : -1;
-    // cos and sin of tpol s_d on lane d (the same functions per component), broadcast
-    double cd, sd;
-    sincos(e.tpol * (lane == 0 ? sx : (lane == 1 ? sy : sz)), &sd, &cd);
-    const double dcx = __shfl(cd, 0, 64), dsx = __shfl(sd, 0, 64);
-    const double dcy = __shfl(cd, 1, 64), dsy = __shfl(sd, 1, 64);
-    const double dcz = __shfl(cd, 2, 64), dsz = __shfl(sd, 2, 64);
-    double sum = 0.0;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        double v = 0.0;
-        const int c = code[s];
-        if (c >= 0) {
-            const int i = ((c >> 16) & 255) - 128, j = ((c >> 8) & 255) - 128, k = (c & 255) - 128;
-            if (c >> 24) {
-                double tmp, cxv = dcx, sxv = dsx, cyv = 1.0, syv = 0.0, czv = 1.0, szv = 0.0;
-                for (int r = 1; r < i; r++) { tmp = cxv; cxv = tmp * dcx - sxv * dsx; sxv = sxv * dcx + tmp * dsx; }
-                for (int r = 0; r < j; r++) { tmp = cyv; cyv = tmp * dcy - syv * dsy; syv = syv * dcy + tmp * dsy; }
-                for (int r = 0; r < k; r++) { tmp = czv; czv = tmp * dcz - szv * dsz; szv = szv * dcz + tmp * dsz; }
-                v = e.f[(i * n + j) * n + k] * sxv * cyv * czv;
-            } else {
-                const double vz2 = (sz + k * L) * (sz + k * L);
-                const double vy2 = (sy + j * L) * (sy + j * L);
-                const double vx = sx + i * L;
-                const double v2 = vx * vx + vy2 + vz2;
-                const double vn = sqrt(v2);
-                v = vx * (e.two_aol_rpi * exp(-e.aol2 * v2) + erfc(e.aol * vn) / vn) / v2;
-            }
-        }
-        sum += v;
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-    return sum;
-}
+constexpr int NT = 256;   // workgroup size of the table kernels
+constexpr double ONE_WAVE_CANDIDATES = 96.0;   // pair candidates of a leg up to which one wavefront runs a system
 
 // The terms of ewald_derivative in its loop order, as the codes of ewald_derivative_wave.
 static std::vector<int32_t> ewald_term_codes(int fc, int pc) {
@@ -1103,473 +65,6 @@ static std::vector<int32_t> ewald_term_codes(int fc, int pc) {
         }
     }
     return out;
-}
-
-// The separation (permuted: x along the motion) at which the commit of tagger w's stored
-// event evaluates the merged-image Coulomb derivative, or false when it evaluates none.
-template <int D>
-__device__ __forceinline__ bool thinning_separation(const ChainArgs &a, const ChainState &st, const ecmc_tagger_desc &T, int w,
-                                    double *q3) {
-    const Slot &sl = st.slot[w];
-    double s[D];
-    if ((T.kind == ECMC_TAG_PAIR_CELLS || T.kind == ECMC_TAG_PAIR_ALL || T.kind == ECMC_TAG_SURPLUS ||
-         T.kind == ECMC_TAG_CELL_BOUNDING || T.kind == ECMC_TAG_FACTOR_MAP) &&
-        (T.event_handler == ECMC_EH_CELL_BOUNDING || T.event_handler == ECMC_EH_TWO_LEAF_BOUNDING)) {
-        separation_vector<D>(a, sl.apos, sl.tpos, s);
-    } else if (T.kind == ECMC_TAG_CELL_VETO) {
-        if (occn_base(a)[sl.cb_cell] != 1) return false;
-        double tp[D];
-        load_pos<D>(a, occ_base(a)[(size_t)sl.cb_cell * a.occ_cap], tp);
-        separation_vector<D>(a, sl.apos, tp, s);
-    } else {
-        return false;
-    }
-    q3[0] = q3[1] = q3[2] = 0.0;
-    for (int d = 0; d < D; d++) q3[d] = s[(sl.adir + d) % D];
-    return true;
-}
-
-// Shared memory of the leg loop's collective steps.
-struct LegShared {
-    int nb_cell[32];
-    int nb_pref[33];
-    Best sb[NT / 64];
-    uint32_t sh[NT / 64];
-    int scan[NT + 1 + NT / 64];
-    int flag;
-};
-
-// The event handlers of tagger t send their candidate event times: the pair taggers' candidate
-// sets over the workgroup, the cell veto and the end of chain with their bounded ring refills,
-// the others on thread 0 (collective; tag_activator.py:228-289 for one tag of a create list).
-template <int D, int FM>
-__device__ __forceinline__ void create_tagger(const ChainArgs &a, ChainState &st, uint32_t *mt, const ecmc_tagger_desc &c, int t,
-                              LegShared &ls) {
-    const int tid = threadIdx.x;
-    if (c.kind == ECMC_TAG_PAIR_CELLS || c.kind == ECMC_TAG_PAIR_ALL || c.kind == ECMC_TAG_SURPLUS ||
-        c.kind == ECMC_TAG_CELL_BOUNDING || c.kind == ECMC_TAG_FACTOR_MAP) {
-        create_pair<D, FM>(a, st, mt, c, t, ls.nb_cell, ls.nb_pref, ls.sb, ls.sh, ls.scan);
-    } else if ((FM & FEAT_CELL_VETO) && c.kind == ECMC_TAG_CELL_VETO) {
-        if (tid == 0) { st.slot[t].valid = 0; st.slot[t].cv_phase = 0; }
-        __syncthreads();
-        // the same bounded refill loop as the end-of-chain randint below
-        for (int attempt = 0;; attempt++) {
-            ring_ensure(st, mt, a, 64);
-            if (tid == 0) {
-                ls.flag = (st.active < 0 || create_cell_veto<D>(a, st, c, t)) ? 1 : 0;
-                if (!ls.flag && attempt >= 64) { st.err = ECMC_ERR_STATE; ls.flag = 1; }
-            }
-            __syncthreads();
-            if (ls.flag) break;
-            ring_ensure(st, mt, a, 624);
-        }
-    } else if (c.kind == ECMC_TAG_END_OF_CHAIN) {
-        if (tid == 0) st.slot[t].valid = 0;
-        __syncthreads();
-        // randint's rejection loop: each word is accepted with probability >= 1/2,
-        // so 64 refills (40k words) without success only happen after a defect
-        for (int attempt = 0;; attempt++) {
-            ring_ensure(st, mt, a, 64);
-            if (tid == 0) {
-                ls.flag = create_end_of_chain(a, st, c, t) ? 1 : 0;
-                if (!ls.flag && attempt >= 64) { st.err = ECMC_ERR_STATE; ls.flag = 1; }
-            }
-            __syncthreads();
-            if (ls.flag) break;
-            ring_ensure(st, mt, a, 624);
-        }
-    } else {
-        if (tid == 0) create_single<D>(a, st, c, t);
-        __syncthreads();
-    }
-}
-
-__device__ __forceinline__ bool commit_thins(const ecmc_tagger_desc &T) {
-    return ((T.kind == ECMC_TAG_PAIR_CELLS || T.kind == ECMC_TAG_PAIR_ALL || T.kind == ECMC_TAG_SURPLUS ||
-             T.kind == ECMC_TAG_CELL_BOUNDING || T.kind == ECMC_TAG_FACTOR_MAP) &&
-            (T.event_handler == ECMC_EH_TWO_LEAF_BOUNDING || T.event_handler == ECMC_EH_CELL_BOUNDING)) ||
-           T.kind == ECMC_TAG_CELL_VETO;
-}
-
-// The out-state of tagger w's stored event, committed to the state (thread 0; the caller made
-// two ring words available when the event thins): send_out_state of its event handler and
-// insert_into_global_state (mediator/single_process_mediator.py:130-150).
-template <int D, int FM>
-__device__ __forceinline__ void commit_event(const ChainArgs &a, ChainState &st, const ecmc_tagger_desc &T, int w, ecmc_event &ev,
-                             double ewald_pre) {
-    Slot &sl = st.slot[w];
-    ev.tagger = w;
-    ev.flags = 0;
-    ev.active = st.active;
-    ev.target = -1;
-    ev.tq = sl.t.q;
-    ev.tr = sl.t.r;
-    ev.ncand = st.ncand;
-    ev.chash = st.chash;
-    const int act = st.active;
-    double p[D];
-    switch (T.kind) {
-    case ECMC_TAG_PAIR_CELLS:
-    case ECMC_TAG_PAIR_ALL:
-    case ECMC_TAG_SURPLUS:
-    case ECMC_TAG_CELL_BOUNDING:
-    case ECMC_TAG_FACTOR_MAP: {
-        ev.target = sl.target;
-        bool lift = true;
-        double s[D];
-        separation_vector<D>(a, sl.apos, sl.tpos, s);
-        if ((FM & FEAT_CELL_BOUNDING) && T.event_handler == ECMC_EH_CELL_BOUNDING) {
-            // two_leaf_unit_cell_bounding_potential_event_handler.py:181-211: the active
-            // unit is still in its cell; bound = the candidate's rate; thinning as below
-            if (pos_to_cell<D>(a, sl.apos) != sl.cb_cell) { st.err = ECMC_ERR_STATE; break; }
-            double q3[3] = {0, 0, 0};
-            for (int d = 0; d < D; d++) q3[d] = s[(sl.adir + d) % D];
-            const double c1 = T.use_charge ? charge_of(a, act) : 1.0;
-            const double c2 = T.use_charge ? charge_of(a, sl.target) : 1.0;
-            double bound = cell_rate<D>(a, T, sl.cb_cell, sl.target, sl.adir, c1, c2) * sl.aspeed;
-            const double der = isnan(ewald_pre) ? ewald_derivative_call(a.ewald, q3[0], q3[1], q3[2]) : ewald_pre;
-            double real = T.par[3] * c1 * c2 * der * sl.aspeed;
-            lift = false;
-            if (real > 0) {
-                double u = words_to_random(ring_word(a, st.cursor), ring_word(a, st.cursor + 1));
-                st.cursor += 2;
-                u = 0 + (bound - 0) * u;
-                if (u < real) lift = true;
-            }
-            if (!lift) st.est[6] += 1.0;
-        } else if ((FM & FEAT_COULOMB) && T.event_handler == ECMC_EH_TWO_LEAF_BOUNDING) {
-            // event_handler_with_bounding_potential.py:75-101
-            double q3[3] = {0, 0, 0};
-            for (int d = 0; d < D; d++) q3[d] = s[(sl.adir + d) % D];
-            const double c1 = T.use_charge ? charge_of(a, act) : 1.0;
-            const double c2 = T.use_charge ? charge_of(a, sl.target) : 1.0;
-            double bound = ipcb_derivative(T.bpar[0] * c1 * c2, q3[0], q3[1], q3[2]) * sl.aspeed;
-            const double der = isnan(ewald_pre) ? ewald_derivative_call(a.ewald, q3[0], q3[1], q3[2]) : ewald_pre;
-            double real = T.par[3] * c1 * c2 * der * sl.aspeed;
-            lift = false;
-            if (real > 0) {
-                double u = words_to_random(ring_word(a, st.cursor), ring_word(a, st.cursor + 1));
-                st.cursor += 2;
-                u = 0 + (bound - 0) * u;
-                if (u < real) lift = true;
-            }
-            if (!lift) st.est[6] += 1.0;
-        }
-        store_pos<D>(a, act, sl.apos);
-        st.at = sl.astamp;
-        if (lift) {
-            st.est[0] += s[sl.adir];
-            st.est[4] += 1.0;
-            st.active = sl.target;
-            ev.flags |= 1;
-        }
-        st.est[2] += 1.0;
-        break;
-    }
-    case ECMC_TAG_CELL_VETO: {
-        if (!(FM & FEAT_CELL_VETO)) { st.err = ECMC_ERR_CONFIGURATION; break; }
-        // mediator.py:265-292: the occupant of the sampled cell, or none;
-        // leaf_unit_cell_veto_event_handler.py:127-149 with
-        // event_handler_with_bounding_potential.py:75-101: thinning of the stored rate
-        const int tc = sl.cb_cell;
-        const int no = occn_base(a)[tc];
-        if (no > 1) { st.err = ECMC_ERR_STATE; break; }
-        bool lift = false;
-        double s[D];
-#pragma unroll
-        for (int d = 0; d < D; d++) s[d] = 0.0;
-        if (no == 1) {
-            const int tid2 = occ_base(a)[(size_t)tc * a.occ_cap];
-            ev.target = tid2;
-            double tp[D];
-            load_pos<D>(a, tid2, tp);
-            separation_vector<D>(a, sl.apos, tp, s);
-            double q3[3] = {0, 0, 0};
-            for (int d = 0; d < D; d++) q3[d] = s[(sl.adir + d) % D];
-            const double c1 = T.use_charge ? charge_of(a, act) : 1.0;
-            const double c2 = T.use_charge ? charge_of(a, tid2) : 1.0;
-            const double der = isnan(ewald_pre) ? ewald_derivative_call(a.ewald, q3[0], q3[1], q3[2]) : ewald_pre;
-            const double real = T.par[3] * c1 * c2 * der * sl.aspeed;
-            if (real > 0) {
-                double u = words_to_random(ring_word(a, st.cursor), ring_word(a, st.cursor + 1));
-                st.cursor += 2;
-                u = 0 + (sl.cv_rate - 0) * u;
-                if (u < real) lift = true;
-            }
-        }
-        store_pos<D>(a, act, sl.apos);
-        st.at = sl.astamp;
-        if (lift) {
-            st.est[0] += s[sl.adir];
-            st.est[4] += 1.0;
-            st.active = ev.target;
-            ev.flags |= 1;
-        } else {
-            st.est[6] += 1.0;
-        }
-        st.est[2] += 1.0;
-        break;
-    }
-    case ECMC_TAG_CELL_BOUNDARY: {
-#pragma unroll
-        for (int d = 0; d < D; d++) p[d] = sl.apos[d];
-        slice_pos<D>(a, p, sl.adir, sl.aspeed, sl.astamp, sl.t);
-        p[sl.cb_dir] = sl.cb_boundary;
-        store_pos<D>(a, act, p);
-        st.at = sl.t;
-        st.est[3] += 1.0;
-        break;
-    }
-    case ECMC_TAG_SAMPLING:
-    case ECMC_TAG_END_OF_RUN: {
-        load_pos<D>(a, act, p);
-        slice_pos<D>(a, p, st.adir, st.aspeed, st.at, sl.t);
-        store_pos<D>(a, act, p);
-        st.at = sl.t;
-        if (T.kind == ECMC_TAG_END_OF_RUN) st.done = 1;
-        break;
-    }
-    case ECMC_TAG_END_OF_CHAIN: {
-        load_pos<D>(a, act, p);
-        slice_pos<D>(a, p, st.adir, st.aspeed, st.at, sl.t);
-        store_pos<D>(a, act, p);
-        st.at = sl.t;
-        st.eoc_last = sl.t;
-        ev.target = sl.target;
-        st.est[1] += T.value * st.aspeed;
-        st.est[5] += 1.0;
-        st.adir = (st.adir + 1) % D;
-        if (sl.target != act) ev.flags |= 1;
-        st.active = sl.target;
-        break;
-    }
-    case ECMC_TAG_START_OF_RUN:
-        st.active = T.ivalue2;
-        st.adir = T.ivalue;
-        st.aspeed = T.value;
-        st.at.q = 0.0;
-        st.at.r = 0.0;
-        break;
-    default:
-        st.err = ECMC_ERR_CONFIGURATION;
-    }
-    ev.pos[0] = ev.pos[1] = ev.pos[2] = 0.0;
-    if (act >= 0) {
-        double q[D];
-        load_pos<D>(a, act, q);
-        for (int d = 0; d < D; d++) ev.pos[d] = q[d];
-    }
-}
-
-// One workgroup runs one system's legs (the whole leg loop of the reference's mediator).
-template <int D, int FM>
-__device__ __forceinline__ void chain_body(const ChainArgs &a) {
-    __shared__ ChainState st;
-    __shared__ ecmc_tagger_desc tg[ECMC_MAX_TAGGERS];
-    __shared__ uint32_t mt[624];
-    __shared__ LegShared ls;
-    int &flag = ls.flag;
-    const int tid = threadIdx.x;
-    // the positions and the MT ring move into LDS for the launch when the host sized it so (the
-    // accessors load_pos, store_pos, ring_word and ring_ensure follow the flags)
-    if (a.lds_pos) {
-        double *lp = reinterpret_cast<double *>(chain_dyn_lds);
-        for (int i = tid; i < D * a.n; i += NT) lp[i] = a.pos[i];
-    }
-    if (a.lds_ring) {
-        uint32_t *lr = reinterpret_cast<uint32_t *>(chain_dyn_lds + a.lds_ring_off);
-        for (int i = tid; i < a.ring_words; i += NT) lr[i] = a.ring[i];
-    }
-    if (a.lds_occn_off >= 0) {
-        int32_t *lc = occn_base(a);
-        for (int i = tid; i < a.ncells; i += NT) lc[i] = a.occ_n[i];
-    }
-    if (a.lds_charge_off >= 0) {
-        double *lq = reinterpret_cast<double *>(chain_dyn_lds + a.lds_charge_off);
-        for (int i = tid; i < a.n; i += NT) lq[i] = a.charge[i];
-    }
-    if (a.lds_occ_off >= 0) {
-        int32_t *lo = occ_base(a);
-        for (int i = tid; i < a.ncells * a.occ_cap; i += NT) lo[i] = a.occ[i];
-    }
-    if (tid == 0) st = *a.st;
-    for (int i = tid; i < a.n_taggers; i += NT) tg[i] = a.tg[i];
-    for (int i = tid; i < 624; i += NT) mt[i] = a.mt[i];
-    __syncthreads();
-    int64_t k = 0;
-    while (k < a.max_events) {
-        if (st.done || st.err) break;
-        // every wave takes its branch decision before thread 0 changes the flags inside it
-        const int started = st.started, pending = st.pending_creates;
-        __syncthreads();
-        if (!started) {
-            if (tid == 0) {
-                int sor = -1;
-                for (int t = 0; t < a.n_taggers; t++)
-                    if (tg[t].kind == ECMC_TAG_START_OF_RUN) sor = t;
-                if (sor < 0) st.err = ECMC_ERR_CONFIGURATION;
-                else create_single<D>(a, st, tg[sor], sor);
-                st.started = 1;
-                st.ncand = 0;
-                st.chash = 0;
-            }
-            __syncthreads();
-        } else if (pending) {
-            if (a.occupancy) occupancy_update<D>(a, st, ls.scan);
-            if (tid == 0) {
-                st.ncand = 0;
-                st.chash = 0;
-            }
-            __syncthreads();
-            const ecmc_tagger_desc &w = tg[st.last_tagger];
-            for (int ci = 0; ci < w.n_create && !st.err; ci++) {
-                const int t = w.create[ci];
-                create_tagger<D, FM>(a, st, mt, tg[t], t, ls);
-            }
-            if (tid == 0) st.pending_creates = 0;
-            __syncthreads();
-            if (st.err) break;
-        }
-        // earliest stored event (ties: first pushed): lane t of the first wavefront holds slot t,
-        // a butterfly over the ECMC_MAX_TAGGERS lanes keeps the least (time, push counter) of the
-        // valid slots (push counters are distinct, so the result is the sequential scan's)
-        static_assert(ECMC_MAX_TAGGERS == 16, "the select butterfly spans 16 lanes");
-        if (tid < 64) {
-            const Slot &sl = st.slot[tid < ECMC_MAX_TAGGERS ? tid : 0];
-            const bool v = tid < a.n_taggers && sl.valid;
-            double q = v ? sl.t.q : 0.0, r = v ? sl.t.r : 0.0;
-            int64_t sq = v ? sl.seq : 0;
-            int w = v ? tid : -1;
-#pragma unroll
-            for (int off = 1; off < ECMC_MAX_TAGGERS; off <<= 1) {
-                const double oq = __shfl_xor(q, off, 64), orr = __shfl_xor(r, off, 64);
-                const int64_t os = __shfl_xor((long long)sq, off, 64);
-                const int ow = __shfl_xor(w, off, 64);
-                if (ow >= 0 && (w < 0 || oq < q || (oq == q && (orr < r || (orr == r && os < sq))))) {
-                    q = oq;
-                    r = orr;
-                    sq = os;
-                    w = ow;
-                }
-            }
-            if (tid == 0) {
-                if (w < 0) st.err = ECMC_ERR_SCHEDULER;
-                else if (time_lt(st.slot[w].t, st.last)) st.err = ECMC_ERR_SCHEDULER;
-                else st.last = st.slot[w].t;
-                flag = w;
-            }
-        }
-        __syncthreads();
-        if (st.err) break;
-        const int w = flag;
-        if (commit_thins(tg[w])) ring_ensure(st, mt, a, 2);
-        double ewald_pre = NAN;
-        if ((FM & FEAT_EWALD) && tid < 64) {
-            double q3[3];
-            if (thinning_separation<D>(a, st, tg[w], w, q3)) ewald_pre = ewald_derivative_wave(a.ewald, a.ewald_codes, a.ewald_ncodes, q3[0], q3[1], q3[2]);
-        }
-        if (tid == 0) {
-            ecmc_event ev;
-            commit_event<D, FM>(a, st, tg[w], w, ev, ewald_pre);
-            const ecmc_tagger_desc &T = tg[w];
-            // trash by tag
-            for (int i = 0; i < T.n_trash; i++) st.slot[T.trash[i]].valid = 0;
-            if (a.log) a.log[k] = ev;
-            st.pending_creates = 1;
-            st.last_tagger = w;
-            if (a.stop_mask & (1 << w)) st.stop_reason = 1;
-        }
-        k++;
-        __syncthreads();
-        if (st.stop_reason) break;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        st.stop_reason = 0;
-        *a.st = st;
-        *a.n_out = k;
-    }
-    for (int i = tid; i < 624; i += NT) a.mt[i] = mt[i];
-    if (a.lds_pos) {
-        const double *lp = reinterpret_cast<const double *>(chain_dyn_lds);
-        for (int i = tid; i < D * a.n; i += NT) a.pos[i] = lp[i];
-    }
-    if (a.lds_ring) {
-        const uint32_t *lr = reinterpret_cast<const uint32_t *>(chain_dyn_lds + a.lds_ring_off);
-        for (int i = tid; i < a.ring_words; i += NT) a.ring[i] = lr[i];
-    }
-    if (a.lds_occn_off >= 0) {
-        const int32_t *lc = occn_base(a);
-        for (int i = tid; i < a.ncells; i += NT) a.occ_n[i] = lc[i];
-    }
-    if (a.lds_occ_off >= 0) {
-        const int32_t *lo = occ_base(a);
-        for (int i = tid; i < a.ncells * a.occ_cap; i += NT) a.occ[i] = lo[i];
-    }
-}
-
-// One system; its arguments in device memory (s->d_args), read at a uniform address.
-template <int D, int FM>
-__global__ __launch_bounds__(NT) void chain_kernel(const ChainArgs *__restrict__ args) {
-    chain_body<D, FM>(*args);
-}
-
-// One step of a leg driven from the host, for the set-level event handler (the mediator and
-// its scheduler stay on the host, the state and the candidate sets on the device):
-//   op 0  the start of a leg: the cell occupancy follows the active unit and the candidate
-//         statistics restart (the activator's internal-state update, tag_activator.py:205-226);
-//   op 1  send_event_time of tagger t's handlers: its candidates' times, the earliest kept in
-//         slot t (time, target, in-state copies);
-//   op 2  send_out_state of tagger t's stored event, committed to the state; *out receives it.
-template <int D, int FM>
-__global__ __launch_bounds__(NT) void chain_step_kernel(const ChainArgs *__restrict__ args, int op, int t,
-                                                        ecmc_event *out) {
-    const ChainArgs &a = *args;
-    __shared__ ChainState st;
-    __shared__ ecmc_tagger_desc tg[ECMC_MAX_TAGGERS];
-    __shared__ uint32_t mt[624];
-    __shared__ LegShared ls;
-    const int tid = threadIdx.x;
-    if (tid == 0) st = *a.st;
-    for (int i = tid; i < a.n_taggers; i += NT) tg[i] = a.tg[i];
-    for (int i = tid; i < 624; i += NT) mt[i] = a.mt[i];
-    __syncthreads();
-    if (op == 0) {
-        if (a.occupancy && st.active >= 0) occupancy_update<D>(a, st, ls.scan);
-        if (tid == 0) {
-            st.ncand = 0;
-            st.chash = 0;
-        }
-        __syncthreads();
-    } else if (op == 1) {
-        // the occupancy follows the active unit here too (a no-op after op 0 in the same leg), so
-        // that a cell tagger never reads the cell of a unit that stopped being active
-        if (a.occupancy && st.active >= 0) occupancy_update<D>(a, st, ls.scan);
-        create_tagger<D, FM>(a, st, mt, tg[t], t, ls);
-    } else {
-        if (commit_thins(tg[t])) ring_ensure(st, mt, a, 2);
-        double ewald_pre = NAN;
-        if ((FM & FEAT_EWALD) && tid < 64) {
-            double q3[3];
-            if (thinning_separation<D>(a, st, tg[t], t, q3)) ewald_pre = ewald_derivative_wave(a.ewald, a.ewald_codes, a.ewald_ncodes, q3[0], q3[1], q3[2]);
-        }
-        if (tid == 0) {
-            ecmc_event ev;
-            commit_event<D, FM>(a, st, tg[t], t, ev, ewald_pre);
-            st.last = st.slot[t].t;
-            *out = ev;
-        }
-    }
-    __syncthreads();
-    if (tid == 0) *a.st = st;
-    for (int i = tid; i < 624; i += NT) a.mt[i] = mt[i];
-}
-
-// Independent systems in one launch: workgroup b runs system b (its own positions, cell
-// occupancy, random stream and state), exactly as chain_kernel runs it alone.
-template <int D, int FM>
-__global__ __launch_bounds__(NT) void chain_many_kernel(const ChainArgs *__restrict__ args) {
-    chain_body<D, FM>(args[blockIdx.x]);   // the arguments stay in global memory, read at a uniform address
 }
 
 // InnerPointEstimator.derivative_bound (inner_point_estimator.py:108-171) for the cell
@@ -1694,10 +189,10 @@ struct ecmc_system {
     double *d_pos = nullptr, *d_charge = nullptr, *d_cmin = nullptr, *d_ewald = nullptr;
     int32_t *d_ewald_codes = nullptr;
     int32_t *d_nearby = nullptr, *d_nearby_n = nullptr, *d_occ = nullptr, *d_occ_n = nullptr;
-    int32_t *d_sur_cell = nullptr, *d_sur_id = nullptr, *d_cand = nullptr;
+    int32_t *d_sur_cell = nullptr, *d_sur_id = nullptr;
     double *d_cbt = nullptr, *d_corners = nullptr;
     CvEntry *d_cvw = nullptr;
-    uint32_t *d_mt = nullptr, *d_ring = nullptr;
+    uint32_t *d_ring = nullptr;
     ChainState *d_st = nullptr;
     ecmc_tagger_desc *d_tg = nullptr;
     ecmc_event *d_log = nullptr;
@@ -1710,6 +205,7 @@ struct ecmc_system {
     int32_t stop_mask = 0;
     int device = 0;          // the device current at creation, which holds its memory
     size_t lds_bytes = 0;    // dynamic LDS of a launch (positions and ring resident there)
+    bool one_wave = false;   // few candidates a leg: workgroups of one wavefront
     int features = FEAT_ALL; // the kernel features the system uses (FEAT_*, potential bits)
     ChainArgs args;
     ChainArgs *d_args = nullptr;   // the arguments of the system's own launches, in device memory
@@ -1739,24 +235,16 @@ static int system_features(const ecmc_system_desc &d) {
 // dimensions run the full kernel): the first whose features cover a launch's runs it.
 struct ChainVariant {
     int features;
-    const void *one, *many;   // chain_kernel, chain_many_kernel
+    const void *one_wave, *four_waves, *global;   // resident systems with 64 and 256 threads, others
 };
-static const ChainVariant CHAIN_VARIANTS_3D[] = {
-    {VARIANT_LJ, reinterpret_cast<const void *>(&chain_kernel<3, VARIANT_LJ>),
-     reinterpret_cast<const void *>(&chain_many_kernel<3, VARIANT_LJ>)},
-    {VARIANT_CHARGED_CB, reinterpret_cast<const void *>(&chain_kernel<3, VARIANT_CHARGED_CB>),
-     reinterpret_cast<const void *>(&chain_many_kernel<3, VARIANT_CHARGED_CB>)},
-    {VARIANT_CHARGED_CV, reinterpret_cast<const void *>(&chain_kernel<3, VARIANT_CHARGED_CV>),
-     reinterpret_cast<const void *>(&chain_many_kernel<3, VARIANT_CHARGED_CV>)},
-    {VARIANT_DIPOLES, reinterpret_cast<const void *>(&chain_kernel<3, VARIANT_DIPOLES>),
-     reinterpret_cast<const void *>(&chain_many_kernel<3, VARIANT_DIPOLES>)},
-    {FEAT_ALL, reinterpret_cast<const void *>(&chain_kernel<3, FEAT_ALL>),
-     reinterpret_cast<const void *>(&chain_many_kernel<3, FEAT_ALL>)},
-};
-static const ChainVariant CHAIN_VARIANTS_2D[] = {
-    {FEAT_ALL, reinterpret_cast<const void *>(&chain_kernel<2, FEAT_ALL>),
-     reinterpret_cast<const void *>(&chain_many_kernel<2, FEAT_ALL>)},
-};
+#define ECMC_VARIANT(D, FM) \
+    {FM, reinterpret_cast<const void *>(&chain_kernel<D, FM, 64, true>), \
+     reinterpret_cast<const void *>(&chain_kernel<D, FM, 256, true>), reinterpret_cast<const void *>(&chain_kernel<D, FM, 256, false>)}
+static const ChainVariant CHAIN_VARIANTS_3D[] = {ECMC_VARIANT(3, VARIANT_LJ), ECMC_VARIANT(3, VARIANT_CHARGED_CB),
+                                                 ECMC_VARIANT(3, VARIANT_CHARGED_CV), ECMC_VARIANT(3, VARIANT_DIPOLES),
+                                                 ECMC_VARIANT(3, FEAT_ALL)};
+static const ChainVariant CHAIN_VARIANTS_2D[] = {ECMC_VARIANT(2, FEAT_ALL)};
+#undef ECMC_VARIANT
 static const ChainVariant &chain_variant(int dim, int features) {
     if (dim == 2) return CHAIN_VARIANTS_2D[0];
     for (const ChainVariant &v : CHAIN_VARIANTS_3D)
@@ -1764,79 +252,63 @@ static const ChainVariant &chain_variant(int dim, int features) {
     return CHAIN_VARIANTS_3D[sizeof(CHAIN_VARIANTS_3D) / sizeof(CHAIN_VARIANTS_3D[0]) - 1];
 }
 
-// Dynamic LDS of the leg loop for a system of n units in dim dimensions with a ring of
-// ring_words words: the positions first, then the ring, each only while the whole fits next to
-// the kernel's static LDS within the device's per-workgroup limit.
+// Residency of a system: its positions, random ring, charges, occupant counts and surplus lists in
+// the launch's dynamic LDS when they fit next to the kernel's static LDS within the device's
+// per-workgroup limit, with as many occupants of every cell (16-bit) as fit after them; else
+// everything stays in global memory.
 static void plan_lds(ecmc_system *s) {
     int dev_max = 0;
     hipDeviceGetAttribute(&dev_max, hipDeviceAttributeMaxSharedMemoryPerBlock, s->device);
-    hipFuncAttributes fa;
-    size_t stat = 16384;
-    const hipError_t e = hipFuncGetAttributes(&fa, chain_variant(s->dim, FEAT_ALL).one);
-    if (e == hipSuccess) stat = fa.sharedSizeBytes;
+    const size_t stat = sizeof(ChainShared<256>) + 256;
     const size_t budget = dev_max > (int)stat ? (size_t)dev_max - stat : 0;
-    const size_t pos_b = ((size_t)s->dim * s->n * sizeof(double) + 15) & ~(size_t)15;
-    const size_t ring_b = (size_t)s->ring_words * sizeof(uint32_t);
-    ChainArgs &a = s->args;
-    a.lds_pos = a.lds_ring = 0;
-    a.lds_ring_off = 0;
-    size_t used = 0;
-    if (pos_b <= budget) {
-        a.lds_pos = 1;
-        used = pos_b;
-    }
-    if (used + ring_b <= budget) {
-        a.lds_ring = 1;
-        a.lds_ring_off = (int32_t)used;
-        used += ring_b;
-    }
-    // the charges (read per candidate by the Coulomb taggers), the far-cell list of a
-    // cell-bounding tagger (n entries at most), the occupant counts and the occupant lists, each
-    // when it fits after the others
-    a.lds_cand_off = a.lds_occn_off = a.lds_occ_off = a.lds_charge_off = -1;
     bool charged = false;
     for (int t = 0; t < s->desc.n_taggers; t++) charged = charged || s->desc.taggers[t].use_charge;
-    const size_t charge_b = charged ? ((size_t)s->n * sizeof(double) + 15) & ~(size_t)15 : 0;
-    if (charge_b && used + charge_b <= budget) {
-        a.lds_charge_off = (int32_t)used;
-        used += charge_b;
+    ChainArgs &a = s->args;
+    a.resident = 0;
+    a.lds_ring_off = a.lds_charge_off = a.lds_occ_off = a.lds_occn_off = a.lds_sur_off = -1;
+    a.occ_cols = 0;
+    s->lds_bytes = 0;
+    if (s->n > 65536) return;   // the occupants are kept as 16-bit numbers
+    size_t used = 0;
+    auto place = [&](size_t bytes) -> int32_t {
+        const size_t at = used;
+        used += (bytes + 15) & ~(size_t)15;
+        return (int32_t)at;
+    };
+    place((size_t)s->dim * s->n * sizeof(double));
+    a.lds_ring_off = place((size_t)s->ring_words * sizeof(uint32_t));
+    if (charged) a.lds_charge_off = place((size_t)s->n * sizeof(double));
+    if (a.occupancy) {
+        a.lds_occn_off = place((size_t)s->ncells * sizeof(int32_t));
+        if (a.max_occ > 0) a.lds_sur_off = place((size_t)s->n * 2 * sizeof(int32_t));
     }
-    const size_t cand_b = s->d_cand ? ((size_t)s->n * sizeof(int32_t) + 15) & ~(size_t)15 : 0;
-    if (cand_b && used + cand_b <= budget) {
-        a.lds_cand_off = (int32_t)used;
-        used += cand_b;
+    if (used > budget) return;
+    if (a.occupancy) {
+        a.occ_cols = (int32_t)std::min<size_t>((size_t)s->occ_cap, (budget - used) / (2 * (size_t)s->ncells));
+        if (a.occ_cols * 2 * (size_t)s->ncells + used + 16 > budget && a.occ_cols > 0) a.occ_cols--;
+        a.lds_occ_off = place((size_t)s->ncells * a.occ_cols * sizeof(uint16_t));
     }
-    const size_t occn_b = ((size_t)s->ncells * sizeof(int32_t) + 15) & ~(size_t)15;
-    if (used + occn_b <= budget) {
-        a.lds_occn_off = (int32_t)used;
-        used += occn_b;
-    }
-    const size_t occ_b = ((size_t)s->ncells * s->occ_cap * sizeof(int32_t) + 15) & ~(size_t)15;
-    if (used + occ_b <= budget) {
-        a.lds_occ_off = (int32_t)used;
-        used += occ_b;
-    }
-    s->lds_bytes = used;
     if (used > 65536) {
         // every variant may run the system (a launch of several systems takes the variant that
         // covers all of them)
-        bool ok = true;
         const ChainVariant *vs = s->dim == 2 ? CHAIN_VARIANTS_2D : CHAIN_VARIANTS_3D;
         const size_t nv = s->dim == 2 ? sizeof(CHAIN_VARIANTS_2D) / sizeof(ChainVariant) : sizeof(CHAIN_VARIANTS_3D) / sizeof(ChainVariant);
-        for (size_t i = 0; i < nv; i++) {
-            ok = ok && hipFuncSetAttribute(vs[i].one, hipFuncAttributeMaxDynamicSharedMemorySize, (int)used) == hipSuccess;
-            ok = ok && hipFuncSetAttribute(vs[i].many, hipFuncAttributeMaxDynamicSharedMemorySize, (int)used) == hipSuccess;
-        }
-        if (!ok) {
-            // keep within the default limit: the ring alone, or nothing
-            (void)hipGetLastError();
-            a.lds_pos = 0;
-            a.lds_ring = ring_b <= 65536 && ring_b <= budget ? 1 : 0;
-            a.lds_ring_off = 0;
-            a.lds_cand_off = a.lds_occn_off = a.lds_occ_off = a.lds_charge_off = -1;
-            s->lds_bytes = a.lds_ring ? ring_b : 0;
-        }
+        for (size_t i = 0; i < nv; i++)
+            for (const void *f : {vs[i].one_wave, vs[i].four_waves})
+                if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)used) != hipSuccess) {
+                    (void)hipGetLastError();
+                    return;
+                }
     }
+    a.resident = 1;
+    s->lds_bytes = used;
+}
+
+// The kernel and workgroup size of a launch.
+static const void *chain_launch(int dim, int features, bool resident, bool one_wave, dim3 &block) {
+    const ChainVariant &v = chain_variant(dim, features);
+    block = dim3(resident && one_wave ? 64 : 256);
+    return !resident ? v.global : (one_wave ? v.one_wave : v.four_waves);
 }
 
 extern "C" int ecmc_system_set_stop_mask(ecmc_system *sys, int32_t mask) {
@@ -1891,7 +363,6 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     if (P > ECMC_MAX_LEAVES) return ecmc_fail(ECMC_ERR_CONFIGURATION, "more leaf units per composite object than ECMC_MAX_LEAVES");
     if (n % P != 0) return ecmc_fail(ECMC_ERR_CONFIGURATION, "the number of units is not a multiple of leaves_per_root");
     int ewald_tagger = -1, cb_tagger = -1;
-    int64_t max_cand = 0;   // the most pair candidates one tagger creates in a leg
     for (int t = 0; t < desc->n_taggers; t++) {
         const ecmc_tagger_desc &tg = desc->taggers[t];
         if (tg.kind < 0 || tg.kind > ECMC_TAG_FACTOR_MAP) return ecmc_fail(ECMC_ERR_CONFIGURATION, "unknown tagger kind");
@@ -1913,7 +384,6 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
                 }
             }
             const int64_t m = tg.fmap_local ? fmax : (int64_t)(n / P - 1) * fmax;
-            max_cand = m > max_cand ? m : max_cand;
             if (!tg.fmap_local && n / P < 2) return ecmc_fail(ECMC_ERR_CONFIGURATION, "a non-local factor needs two composite objects");
             if (tg.n_handlers > 0 && tg.n_handlers < m)
                 return ecmc_fail(ECMC_ERR_TAG_ACTIVATOR, "not-running event handler list would run empty");
@@ -2024,26 +494,32 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
         for (int d = 0; d < dim; d++) pos_soa[(size_t)d * n + i] = positions[(size_t)i * dim + d];
     std::vector<double> ch(n, 1.0);
     if (charges) for (int i = 0; i < n; i++) ch[i] = charges[i];
-    // the candidates of one create: all other units, the surplus (at most n), the occupants of
-    // the nearby cells (a cell holds at most occ_cap: an overflow stops the run) or the occupied
-    // far cells
+    // the pair candidates of a leg, about: all other units, the surplus, the occupants of the nearby
+    // cells, the occupied far cells, the entries of a factor type map
+    double words = 0.0, typical = 0.0;
     for (int t = 0; t < desc->n_taggers; t++) {
-        const int kind = desc->taggers[t].kind;
-        int64_t m = 0;
-        if (kind == ECMC_TAG_PAIR_ALL || kind == ECMC_TAG_SURPLUS) m = n;
-        else if (kind == ECMC_TAG_PAIR_CELLS) m = (int64_t)grid.nb_stride * cap;
-        else if (kind == ECMC_TAG_CELL_BOUNDING) m = std::max<int64_t>((int64_t)grid.nb_stride * cap, grid.count);
-        max_cand = m > max_cand ? m : max_cand;
+        const ecmc_tagger_desc &tg = desc->taggers[t];
+        double m = 0.0;
+        if (tg.kind == ECMC_TAG_PAIR_ALL) m = n;
+        else if (tg.kind == ECMC_TAG_SURPLUS) m = (double)sur_id.size();
+        else if (tg.kind == ECMC_TAG_PAIR_CELLS) m = std::min((double)n, (double)grid.nb_stride * (n - (double)sur_id.size()) / grid.count);
+        else if (tg.kind == ECMC_TAG_CELL_BOUNDING) m = (double)n - (double)sur_id.size();
+        else if (tg.kind == ECMC_TAG_FACTOR_MAP) {
+            int fmax = 0;
+            for (int k = 0; k < P; k++) fmax = std::max(fmax, tg.fmap_n[k]);
+            m = tg.fmap_local ? fmax : (double)(n / P - 1) * fmax;
+        }
+        typical += m;
+        if (tg.event_handler == ECMC_EH_TWO_LEAF_BOUNDING ||
+            (tg.potential != ECMC_POT_HARD_SPHERE && tg.potential != ECMC_POT_HARD_DIPOLE)) words += 2.0 * m;
     }
-    // the ring holds every word a create may read plus a block in production: a power of two, so
-    // that word indices wrap with a mask
-    {
-        const int64_t need = 624 * ((2 * (int64_t)max_cand + 256) / 624 + 3);
-        int64_t words = 1024;
-        while (words < need) words <<= 1;
-        if (words > (1ll << 30)) { delete s; return ecmc_fail(ECMC_ERR_CONFIGURATION, "candidate sets too large"); }
-        s->ring_words = (int)words;
-    }
+    s->one_wave = typical <= ONE_WAVE_CANDIDATES;
+    // the ring: the words of two legs and the generator's 624 (a leg that needs more evaluates its
+    // candidates in segments), a power of two so that indices wrap with a mask, at most 16384 words
+    // (8192 beside large position arrays, so that both fit into LDS)
+    s->ring_words = 2048;
+    const int ring_max = (size_t)dim * n * sizeof(double) > 65536 ? 8192 : 16384;
+    while (s->ring_words < ring_max && (double)s->ring_words < 2.0 * words + 1600.0) s->ring_words <<= 1;
     uint32_t mt[624];
     mt_seed_host(desc->seed, mt);
     ChainState st;
@@ -2094,7 +570,6 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     ECMC_ALLOC(s->d_nearby_n, sizeof(int32_t) * grid.nearby_n.size());
     ECMC_ALLOC(s->d_occ, sizeof(int32_t) * occ.size());
     ECMC_ALLOC(s->d_occ_n, sizeof(int32_t) * occ_n.size());
-    ECMC_ALLOC(s->d_mt, sizeof(uint32_t) * 624);
     ECMC_ALLOC(s->d_ring, sizeof(uint32_t) * s->ring_words);
     ECMC_ALLOC(s->d_st, sizeof(ChainState));
     ECMC_ALLOC(s->d_tg, sizeof(ecmc_tagger_desc) * ECMC_MAX_TAGGERS);
@@ -2104,7 +579,6 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     if (!ewald_codes.empty()) { ECMC_ALLOC(s->d_ewald_codes, sizeof(int32_t) * ewald_codes.size()); }
     ECMC_ALLOC(s->d_sur_cell, sizeof(int32_t) * n);
     ECMC_ALLOC(s->d_sur_id, sizeof(int32_t) * n);
-    ECMC_ALLOC(s->d_cand, sizeof(int32_t) * n);
     if (!sur_cell.empty()) {
         ECMC_UP(s->d_sur_cell, sur_cell.data(), sizeof(int32_t) * sur_cell.size());
         ECMC_UP(s->d_sur_id, sur_id.data(), sizeof(int32_t) * sur_id.size());
@@ -2116,7 +590,10 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     ECMC_UP(s->d_nearby_n, grid.nearby_n.data(), sizeof(int32_t) * grid.nearby_n.size());
     ECMC_UP(s->d_occ, occ.data(), sizeof(int32_t) * occ.size());
     ECMC_UP(s->d_occ_n, occ_n.data(), sizeof(int32_t) * occ_n.size());
-    ECMC_UP(s->d_mt, mt, sizeof(uint32_t) * 624);
+    // the seeded state is words -624 .. -1 of the sequence
+    std::vector<uint32_t> ring((size_t)s->ring_words, 0u);
+    for (int i = 0; i < 624; i++) ring[s->ring_words - 624 + i] = mt[i];
+    ECMC_UP(s->d_ring, ring.data(), sizeof(uint32_t) * ring.size());
     ECMC_UP(s->d_st, &st, sizeof(ChainState));
     ECMC_UP(s->d_tg, desc->taggers, sizeof(ecmc_tagger_desc) * ECMC_MAX_TAGGERS);
     if (!ewald.empty()) { ECMC_UP(s->d_ewald, ewald.data(), sizeof(double) * ewald.size()); }
@@ -2137,6 +614,8 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     }
     a.ncells = grid.count;
     a.nb_stride = grid.nb_stride;
+    for (int d = 0; d < dim; d++)
+        if (grid.cps[d] < 2 * desc->neighbor_layers + 1) a.nb_table = 1;
     a.occ_cap = cap;
     a.ring_words = s->ring_words;
     a.n_taggers = desc->n_taggers;
@@ -2155,7 +634,6 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     a.nearby_n = s->d_nearby_n;
     a.occ = s->d_occ;
     a.occ_n = s->d_occ_n;
-    a.mt = s->d_mt;
     a.ring = s->d_ring;
     a.st = s->d_st;
     a.tg = s->d_tg;
@@ -2164,11 +642,9 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     a.ewald_ncodes = (int32_t)ewald_codes.size();
     a.n_out = s->d_nout;
     a.max_occ = desc->max_occupants;
-    a.sur_cap = n;
     a.layers = desc->neighbor_layers;
     a.sur_cell = s->d_sur_cell;
     a.sur_id = s->d_sur_id;
-    a.cand = s->d_cand;
     if (cb_tagger >= 0) {
         // cell-bound tables on the device (cell_bounding_potential.py:100-126)
         const ecmc_tagger_desc &tg = desc->taggers[cb_tagger];
@@ -2216,6 +692,15 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
             cell_bound_cache_store(key, table);
         }
         a.cbt = s->d_cbt;
+        for (int d = 0; d < 3; d++) {
+            double m = 0.0;
+            for (int c = 0; c < grid.count; c++)
+                for (int b = 0; b < 2; b++) {
+                    const double v = fabs(table[(size_t)(c * 3 + d) * 2 + b]);
+                    if (v > m) m = v;   // NaN marks a nearby separation
+                }
+            a.cb_max[d] = nextafterf((float)m, INFINITY);
+        }
         bool veto = false;
         for (int t = 0; t < desc->n_taggers; t++) veto = veto || desc->taggers[t].kind == ECMC_TAG_CELL_VETO;
         if (veto) {
@@ -2260,8 +745,8 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
 extern "C" void ecmc_system_destroy(ecmc_system *s) {
     if (!s) return;
     hipFree(s->d_pos); hipFree(s->d_charge); hipFree(s->d_cmin); hipFree(s->d_nearby); hipFree(s->d_nearby_n);
-    hipFree(s->d_occ); hipFree(s->d_occ_n); hipFree(s->d_mt); hipFree(s->d_ring); hipFree(s->d_st);
-    hipFree(s->d_sur_cell); hipFree(s->d_sur_id); hipFree(s->d_cand); hipFree(s->d_cbt); hipFree(s->d_corners);
+    hipFree(s->d_occ); hipFree(s->d_occ_n); hipFree(s->d_ring); hipFree(s->d_st);
+    hipFree(s->d_sur_cell); hipFree(s->d_sur_id); hipFree(s->d_cbt); hipFree(s->d_corners);
     hipFree(s->d_cvw);
     hipFree(s->d_tg); hipFree(s->d_nout); hipFree(s->d_log); hipFree(s->d_ewald); hipFree(s->d_ewald_codes); hipFree(s->d_step_ev); hipFree(s->d_args);
     if (s->ev0) hipEventDestroy(s->ev0);
@@ -2301,7 +786,9 @@ extern "C" int ecmc_system_run(ecmc_system *s, int64_t max_events, ecmc_event *h
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy of the launch arguments failed");
     {
         void *kargs[] = {&s->d_args};
-        hipLaunchKernel(chain_variant(s->dim, s->features).one, dim3(1), dim3(NT), kargs, s->lds_bytes, s->stream);
+        dim3 block;
+        const void *kernel = chain_launch(s->dim, s->features, s->args.resident, s->one_wave, block);
+        hipLaunchKernel(kernel, dim3(1), block, kargs, s->lds_bytes, s->stream);
     }
     hipEventRecord(s->ev1, s->stream);
     if (hipGetLastError() != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "kernel launch failed");
@@ -2343,9 +830,16 @@ static int systems_run_staged(ecmc_system *const *systems, int32_t count, int64_
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy of the launch arguments failed");
     hipEventRecord(s0->ev0, s0->stream);
     int features = 0;
-    for (int i = 0; i < count; i++) features |= systems[i]->features;
+    bool one_wave = true, resident = true;
+    for (int i = 0; i < count; i++) {
+        features |= systems[i]->features;
+        one_wave = one_wave && systems[i]->one_wave;
+        resident = resident && systems[i]->args.resident;
+    }
     void *kargs[] = {&d_args};
-    hipLaunchKernel(chain_variant(dim, features).many, dim3(count), dim3(NT), kargs, lds, s0->stream);
+    dim3 block;
+    const void *kernel = chain_launch(dim, features, resident, one_wave, block);
+    hipLaunchKernel(kernel, dim3(count), block, kargs, resident ? lds : 0, s0->stream);
     hipEventRecord(s0->ev1, s0->stream);
     const bool launched = hipGetLastError() == hipSuccess;
     const bool ran = hipStreamSynchronize(s0->stream) == hipSuccess;
@@ -2437,13 +931,11 @@ extern "C" int ecmc_systems_run_noalloc(ecmc_system *const *systems, int32_t cou
 static int system_step(ecmc_system *s, int op, int tagger, ChainState &st) {
     if (!s) return ecmc_fail(ECMC_ERR_ARGUMENT, "null system");
     if (op != 0 && (tagger < 0 || tagger >= s->desc.n_taggers)) return ecmc_fail(ECMC_ERR_ARGUMENT, "no such tagger");
-    ChainArgs sa = s->args;   // one step works on global memory
-    sa.lds_pos = sa.lds_ring = 0;
-    sa.lds_cand_off = sa.lds_occn_off = sa.lds_occ_off = sa.lds_charge_off = -1;
+    const ChainArgs &sa = s->args;   // one step works on global memory
     if (hipMemcpyAsync(s->d_args, &sa, sizeof(ChainArgs), hipMemcpyHostToDevice, s->stream) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy of the launch arguments failed");
-    if (s->dim == 2) hipLaunchKernelGGL((chain_step_kernel<2, FEAT_ALL>), dim3(1), dim3(NT), 0, s->stream, s->d_args, op, tagger, s->d_step_ev);
-    else hipLaunchKernelGGL((chain_step_kernel<3, FEAT_ALL>), dim3(1), dim3(NT), 0, s->stream, s->d_args, op, tagger, s->d_step_ev);
+    if (s->dim == 2) hipLaunchKernelGGL((chain_step_kernel<2, FEAT_ALL, 256>), dim3(1), dim3(256), 0, s->stream, s->d_args, op, tagger, s->d_step_ev);
+    else hipLaunchKernelGGL((chain_step_kernel<3, FEAT_ALL, 256>), dim3(1), dim3(256), 0, s->stream, s->d_args, op, tagger, s->d_step_ev);
     if (hipGetLastError() != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "kernel launch failed");
     if (hipStreamSynchronize(s->stream) != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "kernel execution failed");
     if (hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
@@ -2537,8 +1029,8 @@ extern "C" int ecmc_system_rng_words(const ecmc_system *s, int64_t *words) {
 extern "C" int ecmc_system_launch_lds(const ecmc_system *s, int64_t *bytes, int32_t *positions, int32_t *ring) {
     if (!s) return ecmc_fail(ECMC_ERR_ARGUMENT, "null system");
     if (bytes) *bytes = (int64_t)s->lds_bytes;
-    if (positions) *positions = s->args.lds_pos;
-    if (ring) *ring = s->args.lds_ring;
+    if (positions) *positions = s->args.resident;
+    if (ring) *ring = s->args.resident;
     return ECMC_OK;
 }
 
@@ -2566,13 +1058,15 @@ extern "C" int ecmc_system_last_kernel_ms(const ecmc_system *s, double *ms) {
     return ECMC_OK;
 }
 
-// ---- MT19937 words on the device (testing the parallel twist against CPython) ----------
-__global__ __launch_bounds__(NT) void mt_words_kernel(uint32_t *state, uint32_t *out, int64_t n) {
-    __shared__ uint32_t mt[624];
-    for (int i = threadIdx.x; i < 624; i += NT) mt[i] = state[i];
+// ---- MT19937 words on the device (testing the ring against CPython) ----------------------
+__global__ __launch_bounds__(64) void mt_words_kernel(const uint32_t *state, uint32_t *out, int64_t n) {
+    __shared__ uint32_t ring[2048];
+    for (int i = threadIdx.x; i < 624; i += 64) ring[2048 - 624 + i] = state[i];
     __syncthreads();
-    for (int64_t produced = 0; produced < n; produced += 624) {
-        mt_generate_block(mt, out + produced, ~0ull, 0);
+    for (int64_t from = 0; from < n; from += RING_STEP) {
+        ring_make(ring, 2047u, (uint64_t)from, 1);
+        for (int i = threadIdx.x; i < RING_STEP && from + i < n; i += 64) out[from + i] = mt_temper(ring[(from + i) & 2047]);
+        __syncthreads();
     }
 }
 
@@ -2586,7 +1080,7 @@ extern "C" int ecmc_mt_words(uint64_t seed, int64_t n, uint32_t *d_out, void *st
     if (hipMalloc((void **)&d_state, sizeof(mt)) != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "hipMalloc failed");
     hipStream_t st = (hipStream_t)stream;
     hipMemcpyAsync(d_state, mt, sizeof(mt), hipMemcpyHostToDevice, st);
-    hipLaunchKernelGGL(mt_words_kernel, dim3(1), dim3(NT), 0, st, d_state, d_out, n);
+    hipLaunchKernelGGL(mt_words_kernel, dim3(1), dim3(64), 0, st, d_state, d_out, n);
     hipError_t e = hipStreamSynchronize(st);
     hipFree(d_state);
     if (e != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "mt kernel failed");
