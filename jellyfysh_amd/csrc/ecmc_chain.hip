@@ -699,7 +699,8 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
                     const double v = fabs(table[(size_t)(c * 3 + d) * 2 + b]);
                     if (v > m) m = v;   // NaN marks a nearby separation
                 }
-            a.cb_max[d] = nextafterf((float)m, INFINITY);
+            // per unit of the charge product: bounds use it divided by the target charge
+            a.cb_max[d] = nextafterf((float)(tg.use_charge ? m / fabs(tg.bpar[2]) : m), INFINITY) * (1.f + 0x1p-20f);
         }
         bool veto = false;
         for (int t = 0; t < desc->n_taggers; t++) veto = veto || desc->taggers[t].kind == ECMC_TAG_CELL_VETO;

@@ -3,9 +3,8 @@
 // One workgroup of NT threads (one or four wavefronts) advances one chain.  Every wavefront keeps
 // the chain's state (active unit, its position, time, random cursor, estimators) in registers
 // and runs the sequential part of a leg -- create lists, cell-boundary and end-of-chain events,
-// selection, commit -- redundantly on the same values, so nothing of it is broadcast; the stored
-// events live in one LDS copy per wavefront for the same reason.  Only wavefront 0 writes the
-// shared lists (cell occupants, positions) and memory.  A leg has at most three barriers: after
+// selection, commit -- redundantly on the same values, so nothing of it is broadcast.  Only
+// wavefront 0 writes the shared lists (cell occupants, positions, stored events) and memory.  A leg has at most three barriers: after
 // the occupancy update when the active unit changed, after the candidate tests, and after the
 // exact inversions.
 //
@@ -155,9 +154,11 @@ template <int D>
 struct Geo {
     unsigned char *dyn;        // the launch's dynamic LDS
     int n, ncells, occ_cols, occ_cap, ring_mask, leaves, max_occ, o_ring, o_charge, o_occn, o_occ, o_sur;
-    double L, half;
+    float inv_beta;            // 1 / beta rounded down
+    double L, half, beta;
     double side[D], inv[D];    // cell side and its rounded inverse
     int cps[D], cum[D];
+    float cb_max[3];           // cell bounding: the largest |rate| per direction and unit charge product
     int noff[D];               // lane k: the offset of the k-th nearby cell
     int nb_cells;              // nearby cells (0: read from the table)
     uint64_t kinds;            // 4 bits per tagger: its kind
@@ -601,15 +602,22 @@ struct HotList {
     uint32_t trashers;      // bit t: tagger t trashes all of this list
 };
 
+struct SlotTime {
+    Time t;
+    int64_t seq;
+    int32_t valid, pad;
+};
 template <int NT>
 struct ChainShared {
     static constexpr int NW = NT / 64;
-    Slot slot[NW][ECMC_MAX_TAGGERS];
+    Slot slot[ECMC_MAX_TAGGERS];             // payloads of the stored events, written by thread 0
+    SlotTime time[NW][ECMC_MAX_TAGGERS];     // their times as every wavefront sees them, around a rare step
     ecmc_tagger_desc tg[ECMC_MAX_TAGGERS];
     TaggerPlan plan[ECMC_MAX_TAGGERS];
     Contender queue[NW][QCAP];
     Winner win[NW];
-    int32_t nb_cell[NW][32], nb_pref[NW][33];
+    alignas(16) int32_t nb_cell[NW][32];     // nearby cells and exclusive prefix sums of their occupants
+    alignas(16) int32_t nb_pref[NW][32];
     uint32_t far_word[NW][64], far_pref[NW][64];
     uint32_t occupied[64];       // one bit per occupied cell (cell bounding, grids of at most FAR_BLOCK cells)
     int32_t qn[NW];
@@ -624,9 +632,9 @@ struct ChainShared {
 };
 
 // The leg to and from LDS around a rare step: uniform fields by the first lane, the stored events'
-// times by their lanes into their slots.
+// times by their lanes.
 template <int D>
-__device__ __forceinline__ void leg_to(const Leg<D> &g, Leg<3> &m, Slot *slot) {
+__device__ __forceinline__ void leg_to(const Leg<D> &g, Leg<3> &m, SlotTime *time) {
     const int lane = threadIdx.x & 63;
     if (lane == 0) {
         m.active = g.active; m.adir = g.adir; m.aspeed = g.aspeed; m.at = g.at;
@@ -640,11 +648,11 @@ __device__ __forceinline__ void leg_to(const Leg<D> &g, Leg<3> &m, Slot *slot) {
         m.ncand = g.ncand; m.chash = g.chash; m.nsur = g.nsur; m.mean_step = g.mean_step;
     }
     if (lane < ECMC_MAX_TAGGERS) {
-        slot[lane].t = g.lt; slot[lane].seq = g.lseq; slot[lane].valid = g.lvalid;
+        time[lane].t = g.lt; time[lane].seq = g.lseq; time[lane].valid = g.lvalid;
     }
 }
 template <int D>
-__device__ __forceinline__ void leg_from(const Leg<3> &m, const Slot *slot, Leg<D> &g) {
+__device__ __forceinline__ void leg_from(const Leg<3> &m, const SlotTime *time, Leg<D> &g) {
     const int lane = threadIdx.x & 63;
     g.active = uni(m.active); g.adir = uni(m.adir); g.aspeed = uni(m.aspeed); g.at = uni(m.at);
 #pragma unroll
@@ -655,7 +663,7 @@ __device__ __forceinline__ void leg_from(const Leg<3> &m, const Slot *slot, Leg<
     g.last = uni(m.last); g.seq = (int64_t)uni((uint64_t)m.seq); g.eoc_last = uni(m.eoc_last); g.samp_time = uni(m.samp_time);
     g.cursor = uni(m.cursor); g.produced = uni(m.produced); g.keep = uni(m.keep);
     g.ncand = uni(m.ncand); g.chash = (uint32_t)uni((int)m.chash); g.nsur = uni(m.nsur); g.mean_step = uni(m.mean_step);
-    const Slot &sl = slot[lane & 15];
+    const SlotTime &sl = time[lane & 15];
     g.lt = sl.t; g.lseq = sl.seq; g.lvalid = lane < ECMC_MAX_TAGGERS && sl.valid;
 }
 // The launch's constants: the offsets of lane k's nearby cell (the product of the offsets, the last
@@ -676,7 +684,7 @@ __device__ __forceinline__ void geo_load(const Geo<3> &m, const ChainArgs &a, Ge
     q.n = uni(m.n); q.ncells = uni(m.ncells); q.occ_cols = uni(m.occ_cols); q.occ_cap = uni(m.occ_cap);
     q.ring_mask = uni(m.ring_mask); q.leaves = uni(m.leaves); q.max_occ = uni(m.max_occ);
     q.o_ring = uni(m.o_ring); q.o_charge = uni(m.o_charge); q.o_occn = uni(m.o_occn); q.o_occ = uni(m.o_occ); q.o_sur = uni(m.o_sur);
-    q.L = uni(m.L); q.half = uni(m.half);
+    q.L = uni(m.L); q.half = uni(m.half); q.beta = uni(m.beta); q.inv_beta = m.inv_beta;
 #pragma unroll
     for (int d = 0; d < D; d++) {
         q.side[d] = uni(m.side[d]); q.inv[d] = uni(m.inv[d]);
@@ -694,22 +702,22 @@ struct Items {
     uint64_t tags;
     uint32_t word;
     int32_t rank, before;
+    int32_t p;           // launch constants of item i in lane i: TaggerPlan::p, rc2_hi, set_key and the
+    float rc2_hi, pref;  // prefactor of the quick test
+    int32_t set_key;
 };
+__device__ __forceinline__ float item_f(float v, int i) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), i)); }
 __device__ __forceinline__ int item_tag(const Items &it, int i) { return (int)((it.tags >> (4 * i)) & 15u); }
 __device__ __forceinline__ uint32_t item_word(const Items &it, int i) { return (uint32_t)__builtin_amdgcn_readlane((int)it.word, i); }
 __device__ __forceinline__ int item_rank(const Items &it, int i) { return __builtin_amdgcn_readlane(it.rank, i); }
 
-template <int D, int NT>
-__device__ __forceinline__ Slot &own_slot(ChainShared<NT> &sh, int t) {
-    return sh.slot[wave_index<NT>()][t];
-}
 // An estimator's sum, one addition a leg in leg order: by the first lane of wavefront 0, as an LDS
 // operation that nothing waits for.
 template <int NT>
 __device__ __forceinline__ void add_est(ChainShared<NT> &sh, int k, double v) {
     if (threadIdx.x == 0) unsafeAtomicAdd(&sh.est[k], v);
 }
-// The stored event of tagger t as its lane sees it; its payload goes to the wavefront's LDS copy.
+// The stored event of tagger t as its lane sees it (its payload goes to sh.slot by thread 0).
 template <int D>
 __device__ __forceinline__ void lane_slot(Leg<D> &g, int t, Time time, int64_t seq, int valid) {
     if ((int)(threadIdx.x & 63) == t) {
@@ -939,22 +947,28 @@ __device__ __forceinline__ int nearby_cell(const ChainArgs &a, const Geo<D> &q, 
     }
     return cc;
 }
+// Every fourth prefix sum stays uniform (group[k]: of cell 4 (k + 1)), so that a candidate's cell
+// takes seven comparisons and one LDS access of the four cells left.
+struct Counts {
+    int nb, far;        // candidates in the nearby and the far cells (-1: not counted yet)
+    int group[7];
+};
 template <int D, int NT, bool RES>
-__device__ __forceinline__ int nearby_prefix(const ChainArgs &a, const Geo<D> &q, const Leg<D> &g, ChainShared<NT> &sh, int &ncell) {
+__device__ __forceinline__ void nearby_prefix(const ChainArgs &a, const Geo<D> &q, const Leg<D> &g, ChainShared<NT> &sh, Counts &n) {
     const int lane = threadIdx.x & 63, wave = wave_index<NT>();
     int cnt;
     const int cc = nearby_cell<D, NT, RES>(a, q, g, cnt);
     int num = 0;
     if (lane < cnt) num = occ_count<RES>(a, q, cc);
     const int incl = scan32(num, lane);
-    if (lane < cnt) {
+    if (lane < 32) {
         sh.nb_cell[wave][lane] = cc;
-        sh.nb_pref[wave][lane + 1] = incl;
+        sh.nb_pref[wave][lane] = incl - num;
     }
-    if (lane == 0) sh.nb_pref[wave][0] = 0;
+#pragma unroll
+    for (int k = 0; k < 7; k++) n.group[k] = __builtin_amdgcn_readlane(incl, 4 * k + 3);
+    n.nb = __builtin_amdgcn_readlane(incl, 31);
     wave_sync();
-    ncell = cnt;
-    return cnt ? __builtin_amdgcn_readlane(incl, cnt - 1) : 0;
 }
 
 // The far cells of the active cell, cell bounding: occupied and not nearby
@@ -998,10 +1012,7 @@ __device__ __forceinline__ int far_prefix(const ChainArgs &a, const Geo<D> &q, c
 
 // ---- candidates ---------------------------------------------------------------------------
 // Number of pair candidates of tagger t (kind: its kind) in this leg; the nearby and far prefixes
-// are built once per leg (nb < 0 / far < 0 before).
-struct Counts {
-    int nb, nb_cells, far;
-};
+// are built once per leg.
 template <int D, int FM, int NT, bool RES>
 __device__ __forceinline__ int candidate_count(const ChainArgs &a, const Geo<D> &q, const Leg<D> &g, ChainShared<NT> &sh, int t,
                                                int kind, Counts &n) {
@@ -1016,7 +1027,7 @@ __device__ __forceinline__ int candidate_count(const ChainArgs &a, const Geo<D> 
         }
         return n.far;
     }
-    if (n.nb < 0) n.nb = nearby_prefix<D, NT, RES>(a, q, g, sh, n.nb_cells);
+    if (n.nb < 0) nearby_prefix<D, NT, RES>(a, q, g, sh, n);
     return n.nb;
 }
 
@@ -1028,11 +1039,11 @@ struct Candidates {
     const Geo<D> &q;
     ChainShared<NT> &sh;
     const ecmc_tagger_desc &tg;
-    int kind, act, wave, nb_cells, M, m, k, fn, first;
+    const Counts &n;
+    int kind, act, wave, M, m, k, fn, first;
     __device__ __forceinline__ Candidates(const ChainArgs &a_, const Geo<D> &q_, ChainShared<NT> &s_, int t, int kind_, int act_, int M_,
-                                          int nbc)
-        : a(a_), q(q_), sh(s_), tg(s_.tg[t]), kind(kind_), act(act_), wave(wave_index<NT>()), nb_cells(nbc), M(M_), m(0), k(0), fn(1),
-          first(0) {
+                                          const Counts &n_)
+        : a(a_), q(q_), sh(s_), tg(s_.tg[t]), n(n_), kind(kind_), act(act_), wave(wave_index<NT>()), M(M_), m(0), k(0), fn(1), first(0) {
         if ((FM & FEAT_FMAP) && kind == ECMC_TAG_FACTOR_MAP) {
             m = act / q.leaves;
             k = act % q.leaves;
@@ -1056,15 +1067,16 @@ struct Candidates {
         else if (kind == ECMC_TAG_PAIR_ALL) target = idx < act ? idx : idx + 1;
         else if (kind == ECMC_TAG_SURPLUS) target = sur_id<RES>(a, q, idx);
         else {
-            // the nearby cell holding candidate idx: the largest c with pref[c] <= idx, a fixed
-            // five-step search (pref[nb_cells] = M > idx; empty cells repeat a prefix)
-            int lo = 0;
+            // the nearby cell holding candidate idx: the largest c with pref[c] <= idx (empty cells
+            // repeat a prefix, and so do the places after the last cell)
+            int k4 = 0;
 #pragma unroll
-            for (int st = 16; st > 0; st >>= 1) {
-                const int t = min(lo + st, nb_cells);
-                lo = sh.nb_pref[wave][t] <= idx ? t : lo;
-            }
-            target = occ_get<RES>(a, q, sh.nb_cell[wave][lo], idx - sh.nb_pref[wave][lo]);
+            for (int i = 0; i < 7; i++) k4 += n.group[i] <= idx ? 1 : 0;
+            const int4 p = *reinterpret_cast<const int4 *>(&sh.nb_pref[wave][4 * k4]);
+            const int4 c = *reinterpret_cast<const int4 *>(&sh.nb_cell[wave][4 * k4]);
+            const bool b1 = p.y <= idx, b2 = p.z <= idx, b3 = p.w <= idx;
+            const int at = b3 ? p.w : (b2 ? p.z : (b1 ? p.y : p.x)), in = b3 ? c.w : (b2 ? c.z : (b1 ? c.y : c.x));
+            target = occ_get<RES>(a, q, in, idx - at);
         }
         return true;
     }
@@ -1085,19 +1097,24 @@ struct Candidates {
 __device__ __forceinline__ bool quick_cull(int test, int p, float rc2_hi, float pp, float perp2, float sd, bool behind, bool edge,
                                            float hf, float L, float dU_lo) {
     const float K = fabsf(pp);
-    if (!(K >= 0x1p-100f && K <= 0x1p100f) || edge) return false;
+    const bool sure = (K >= 0x1p-100f) & (K <= 0x1p100f) & !edge;
     bool none;
     if (test == QT_INVERSE_POWER) {
         const float slack = (fabsf(sd) + hf) * 0x1p-17f;
         const float e = fmaxf(fmaxf(sd - hf, -sd) - slack, 0.f);
         const float r2 = (perp2 + e * e) * (1.f - 0x1p-16f);
         none = pp > 0.f ? behind : sd - slack > hf;
-        none = none || r2 >= rc2_hi;
-        float rp = (p & 1) ? __builtin_amdgcn_sqrtf(r2) : 1.f;
-#pragma unroll 1
-        for (int i = 0; i < (p >> 1); i++) rp *= r2;
+        none = none | (r2 >= rc2_hi);
+        // r^p for 1 <= p <= 32 by binary powering of r2 (p uniform: at most nine products)
+        const float r = __builtin_amdgcn_sqrtf(r2), r4 = r2 * r2, r8 = r4 * r4, r16 = r8 * r8;
+        float rp = (p & 1) ? r : 1.f;
+        rp = (p & 2) ? rp * r2 : rp;
+        rp = (p & 4) ? rp * r4 : rp;
+        rp = (p & 8) ? rp * r8 : rp;
+        rp = (p & 16) ? rp * r16 : rp;
+        rp = (p & 32) ? rp * (r16 * r16) : rp;
         const float A = dU_lo * rp * (1.f - 0x1p-15f);
-        none = none || A > K || A * __builtin_amdgcn_sqrtf(r2) * (1.f - 0x1p-20f) > (float)p * K * hf;
+        none = none | (A > K) | (A * r * (1.f - 0x1p-20f) > (float)p * K * hf);
     } else {
         // the Coulomb bound runs over the periodic images along the motion: within a quarter box the
         // nearest image passed lies at |x| >= min(e, L / 4)
@@ -1105,10 +1122,19 @@ __device__ __forceinline__ bool quick_cull(int test, int p, float rc2_hi, float 
         const float slack = (fabsf(sd) + L) * 0x1p-16f;
         const float e = near ? fminf(fmaxf(fmaxf(sd - hf, -sd) - slack, 0.f), 0.25f * L) : 0.f;
         const float r2 = (perp2 + e * e) * (1.f - 0x1p-16f);
-        none = near && (pp > 0.f ? (sd < -slack && sd - hf > -0.5f * L + slack) : sd - hf > slack);
-        none = none || dU_lo * r2 * (1.f - 0x1p-15f) > K * hf;
+        none = near & (pp > 0.f ? (sd < -slack) & (sd - hf > -0.5f * L + slack) : sd - hf > slack);
+        none = none | (dU_lo * r2 * (1.f - 0x1p-15f) > K * hf);
     }
-    return none;
+    return none & sure;
+}
+
+// dU_lower (ecmc_fp32_bounds.h) without its branch: u24 below 2^-10, else the hardware logarithm
+// that log2f is for its normal argument, less its error bound.
+__device__ __forceinline__ float draw_lower(uint32_t a, float inv_beta_lo) {
+    const float u24 = (float)(a >> 8) * 0x1p-24f;
+    const float ml2 = -__builtin_amdgcn_logf(1.f - u24);
+    const float l = (ml2 - LOG2F_ERR * fmaxf(ml2, 1.f)) * 0x1.62e42ep-1f;
+    return fmaxf((u24 < 0x1p-10f ? u24 : l) * inv_beta_lo * (1.f - 0x1p-20f), 0.f);
 }
 
 // Pass 1 of a leg: every candidate of the items tested against the horizon h (time); the
@@ -1120,20 +1146,25 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
     const int lane = threadIdx.x & 63, wave = wave_index<NT>();
     const float Lf = (float)q.L;
     const float hf = (float)(h * g.aspeed) * (1.f + 0x1p-16f) + Lf * 0x1p-18f;
-    const float ibf = __builtin_amdgcn_rcpf((float)a.beta) * (1.f - 0x1p-20f);
+    const float ibf = q.inv_beta;
     const double edge_at = q.half * (1.0 - 0x1p-40), behind_at = -q.L * 0x1p-40;
     const int act = g.active, dir = g.adir;
+    const float caf = (FM & FEAT_EWALD) && q.charged ? (float)charge_of<RES>(a, q, act) : 1.f;
+    float cell_rate_max = 0.f;
+    if (FM & FEAT_CELL_BOUNDING) cell_rate_max = pick_axis<3>(q.cb_max, dir);
     int qn = 0;
+#pragma unroll 1
     for (int g0 = 0, g1; g0 < its.count; g0 = g1) {
-        const int t0 = item_tag(its, g0), key = uni(sh.plan[t0].set_key);
+        const int t0 = item_tag(its, g0), key = __builtin_amdgcn_readlane(its.set_key, g0);
         bool geo = false;
+#pragma unroll 1
         for (g1 = g0; g1 < its.count; g1++) {
             const int t = item_tag(its, g1), test = (q.tests >> (2 * t)) & 3;
-            if (g1 > g0 && uni(sh.plan[t].set_key) != key) break;
+            if (g1 > g0 && __builtin_amdgcn_readlane(its.set_key, g1) != key) break;
             geo = geo || test == QT_INVERSE_POWER || test == QT_COULOMB_BOUND;
         }
         const int kind = kind_of(q.kinds, t0);
-        Candidates<D, FM, NT, RES> cs(a, q, sh, t0, kind, act, candidate_count<D, FM, NT, RES>(a, q, g, sh, t0, kind, cn), cn.nb_cells);
+        Candidates<D, FM, NT, RES> cs(a, q, sh, t0, kind, act, candidate_count<D, FM, NT, RES>(a, q, g, sh, t0, kind, cn), cn);
         if (cs.M == 0) continue;
         int before = 0;
         for (;; cs.first += FAR_BLOCK) {   // one pass but for far cells of a large grid
@@ -1184,25 +1215,27 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
 #pragma unroll
                     for (int u = 0; u < U; u++) keep[u] = live[u];
                     if (test != QT_DIRECT) {
-                        const ecmc_tagger_desc &tg = sh.tg[tag];
-                        const int p = uni(sh.plan[tag].p);
-                        const float rc2_hi = sh.plan[tag].rc2_hi;
-                        const bool charged = (q.charged >> tag) & 1u;
-                        const double pref = test == QT_INVERSE_POWER ? tg.par[1] : tg.bpar[0];
-                        const double ca = charged ? charge_of<RES>(a, q, act) : 1.0;
+                        const int p = __builtin_amdgcn_readlane(its.p, i);
+                        const float rc2_hi = item_f(its.rc2_hi, i);
+                        float pref = item_f(its.pref, i);
+                        if ((FM & FEAT_CELL_BOUNDING) && test == QT_CELL) pref = cell_rate_max;
+                        float dU_lo[U], pp[U];
 #pragma unroll
                         for (int u = 0; u < U; u++) {
-                            const float dU_lo = dU_lower(ring_word<RES>(a, q, (uint32_t)g.keep + word + 2u * (uint32_t)j[u]), ibf);
-                            const double ct = charged ? charge_of<RES>(a, q, target[u]) : 1.0;
-                            bool cull;
-                            if ((FM & FEAT_CELL_BOUNDING) && test == QT_CELL) {
-                                const float cf = charged ? fabsf((float)(ca * ct / tg.bpar[2])) : 1.f;
-                                cull = dU_lo * (1.f - 0x1p-15f) > a.cb_max[dir] * cf * hf;
-                            } else {
-                                cull = quick_cull(test, p, rc2_hi, (float)(pref * (ca * ct)), perp2[u], sd[u], behind[u], edge[u], hf,
-                                                  Lf, dU_lo);
-                            }
-                            keep[u] = keep[u] && !cull;
+                            dU_lo[u] = draw_lower(ring_word<RES>(a, q, (uint32_t)g.keep + word + 2u * (uint32_t)j[u]), ibf);
+                            pp[u] = pref;
+                        }
+                        if ((q.charged >> tag) & 1u) {
+#pragma unroll
+                            for (int u = 0; u < U; u++) pp[u] *= caf * (float)charge_of<RES>(a, q, target[u]);
+                        }
+#pragma unroll
+                        for (int u = 0; u < U; u++) {
+                            // (a cell bound's prefactor is its largest rate per unit charge factor)
+                            const bool cull = (FM & FEAT_CELL_BOUNDING) && test == QT_CELL
+                                                  ? dU_lo[u] * (1.f - 0x1p-15f) > fabsf(pp[u]) * hf
+                                                  : quick_cull(test, p, rc2_hi, pp[u], perp2[u], sd[u], behind[u], edge[u], hf, Lf, dU_lo[u]);
+                            keep[u] = keep[u] & !cull;
                         }
                     }
 #pragma unroll
@@ -1243,7 +1276,7 @@ __device__ __forceinline__ double candidate_dt(const ChainArgs &a, const Geo<D> 
     if ((q.draws >> tag) & 1u) {
         w0 = ring_word<RES>(a, q, (uint32_t)g.keep + word);
         w1 = ring_word<RES>(a, q, (uint32_t)g.keep + word + 1u);
-        beta = a.beta;
+        beta = q.beta;
     }
     double ca = 1.0, ct = 1.0;
     if ((q.charged >> tag) & 1u) {
@@ -1311,7 +1344,7 @@ __device__ __forceinline__ uint32_t candidate_hash(const ChainArgs &a, const Geo
                                                    int kind, int M, const Counts &cn, int joff) {
     const int lane = threadIdx.x & 63, wave = wave_index<NT>();
     uint32_t h = 0;
-    Candidates<D, FM, NT, RES> cs(a, q, sh, t, kind, g.active, M, cn.nb_cells);
+    Candidates<D, FM, NT, RES> cs(a, q, sh, t, kind, g.active, M, cn);
     int before = 0;
 #pragma unroll 1
     for (;; cs.first += FAR_BLOCK) {
@@ -1362,8 +1395,8 @@ __device__ __forceinline__ void create_boundary(const ChainArgs &a, const Geo<D>
 }
 template <int D, int NT>
 __device__ __forceinline__ void store_boundary(Leg<D> &g, ChainShared<NT> &sh, const Boundary &b) {
-    if ((threadIdx.x & 63) == 0) {
-        Slot &sl = own_slot<D, NT>(sh, b.p.w);
+    if (threadIdx.x == 0) {
+        Slot &sl = sh.slot[b.p.w];
 #pragma unroll
         for (int d = 0; d < D; d++) sl.apos[d] = g.ap[d];
         sl.astamp = g.at;
@@ -1405,7 +1438,7 @@ __device__ __forceinline__ void create_end_of_chain(const ChainArgs &a, const Ge
         }
         if (phase == 0) root = v;
     }
-    if ((threadIdx.x & 63) == 0) own_slot<D, NT>(sh, t).target = P > 1 ? root * P + v : v;
+    if (threadIdx.x == 0) sh.slot[t].target = P > 1 ? root * P + v : v;
     lane_slot(g, t, time, g.seq++, 1);
 }
 
@@ -1458,8 +1491,8 @@ __device__ __forceinline__ void create_cell_veto(const ChainArgs &a, const Geo<D
 #pragma unroll
     for (int d = 0; d < D; d++) ap[d] = g.ap[d];
     if (ub(!isinf(time.q))) slice_pos<D>(q, ap, dir, g.aspeed, g.at, time);
-    if ((threadIdx.x & 63) == 0) {
-        Slot &sl = own_slot<D, NT>(sh, t);
+    if (threadIdx.x == 0) {
+        Slot &sl = sh.slot[t];
         sl.target = -1;
         sl.cb_cell = tcell;
         sl.cv_rate = rate;
@@ -1508,8 +1541,8 @@ __device__ __forceinline__ void store_winner(const ChainArgs &a, const Geo<D> &q
 #pragma unroll
     for (int d = 0; d < D; d++) p[d] = g.ap[d];
     if (ub(!isinf(w.t.q))) slice_pos<D>(q, p, g.adir, g.aspeed, g.at, w.t);
-    if ((threadIdx.x & 63) == 0) {
-        Slot &sl = own_slot<D, NT>(sh, t);
+    if (threadIdx.x == 0) {
+        Slot &sl = sh.slot[t];
         sl.cb_cell = g.occ_cell;
         sl.target = w.target;
         sl.adir = g.adir;
@@ -1591,7 +1624,7 @@ struct Event {
 };
 template <int D, int NT>
 __device__ __forceinline__ void event_of_slot(ChainShared<NT> &sh, int t, Event<D> &e) {
-    const Slot &sl = own_slot<D, NT>(sh, t);
+    const Slot &sl = sh.slot[t];
     e.tagger = t;
     e.target = uni(sl.target);
     e.adir = uni(sl.adir);
@@ -1810,8 +1843,11 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
     q.leaves = a.leaves; q.max_occ = a.max_occ;
     q.o_ring = a.lds_ring_off; q.o_charge = a.lds_charge_off; q.o_occn = a.lds_occn_off; q.o_occ = a.lds_occ_off;
     q.o_sur = a.lds_sur_off;
-    q.L = a.L; q.half = a.half;
+    q.L = a.L; q.half = a.half; q.beta = a.beta;
+    q.inv_beta = (float)(1.0 / a.beta) * (1.f - 0x1p-20f);
     q.nb_cells = a.nb_table ? 0 : a.nb_stride;
+#pragma unroll
+    for (int d = 0; d < 3; d++) q.cb_max[d] = a.cb_max[d];
     nearby_offsets<D>(a, q);
 #pragma unroll
     for (int d = 0; d < D; d++) {
@@ -1859,8 +1895,8 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
         for (int i = tid; i < (int)(sizeof(ecmc_tagger_desc) / 4) * a.n_taggers; i += NT) dst[i] = src[i];
         const uint32_t *ss = reinterpret_cast<const uint32_t *>(s.slot);
         const int words = (int)sizeof(Slot) / 4 * ECMC_MAX_TAGGERS;
-        uint32_t *ds = reinterpret_cast<uint32_t *>(sh.slot[wave_index<NT>()]);
-        for (int i = lane; i < words; i += 64) ds[i] = ss[i];
+        uint32_t *ds = reinterpret_cast<uint32_t *>(sh.slot);
+        for (int i = tid; i < words; i += NT) ds[i] = ss[i];
     }
     for (int i = tid; i < 3 * AXIS_CELLS; i += NT) {
         const int d = i / AXIS_CELLS, c = i % AXIS_CELLS;
@@ -1938,7 +1974,7 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
         m.n = q.n; m.ncells = q.ncells; m.occ_cols = q.occ_cols; m.occ_cap = q.occ_cap; m.ring_mask = q.ring_mask;
         m.leaves = q.leaves; m.max_occ = q.max_occ;
         m.o_ring = q.o_ring; m.o_charge = q.o_charge; m.o_occn = q.o_occn; m.o_occ = q.o_occ; m.o_sur = q.o_sur;
-        m.L = q.L; m.half = q.half;
+        m.L = q.L; m.half = q.half; m.beta = q.beta; m.inv_beta = q.inv_beta;
 #pragma unroll
         for (int d = 0; d < D; d++) { m.side[d] = q.side[d]; m.inv[d] = q.inv[d]; m.cps[d] = q.cps[d]; m.cum[d] = q.cum[d]; }
         m.nb_cells = q.nb_cells; m.kinds = q.kinds; m.tests = q.tests; m.draws = q.draws; m.charged = q.charged;
@@ -1955,7 +1991,7 @@ __device__ __forceinline__ void launch_store(const ChainArgs &a, const Geo<D> &q
     __syncthreads();
     ChainState &s = *a.st;
     if (tid < ECMC_MAX_TAGGERS) {
-        Slot sl = sh.slot[0][tid];
+        Slot sl = sh.slot[tid];
         sl.t = g.lt; sl.seq = g.lseq; sl.valid = g.lvalid;
         s.slot[tid] = sl;
     }
@@ -2043,7 +2079,7 @@ __device__ __forceinline__ void create_pair_full(const ChainArgs &a, const Geo<D
         if (draws) ring_ensure<RES, D, NT>(a, q, g, g.keep + 2ull * (uint64_t)(hi - lo));
         if (g.err) return;
         Winner m = no_winner();
-        Candidates<D, FM, NT, RES> cs(a, q, sh, t, kind, g.active, M, cn.nb_cells);
+        Candidates<D, FM, NT, RES> cs(a, q, sh, t, kind, g.active, M, cn);
         int before = 0;
 #pragma unroll 1
         for (;; cs.first += FAR_BLOCK) {
@@ -2084,7 +2120,8 @@ template <int D, int FM, int NT, bool RES>
 __device__ __forceinline__ void general_creates(const ChainArgs &a, const Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh, int creator, int ci,
                                                 int end, bool hashed) {
     const uint64_t create = uni(sh.plan[creator].create);
-    Counts cn = {-1, 0, -1};
+    Counts cn;
+    cn.nb = cn.far = -1;
 #pragma unroll 1
     for (; ci < end && !g.err; ci++) {
         const int t = (int)((create >> (4 * ci)) & 15u), kind = kind_of(q.kinds, t);
@@ -2121,7 +2158,7 @@ __device__ __noinline__ static void rare_step(const ChainArgs *args, ChainShared
     Geo<D> q;
     geo_load<D>(sh.geo, a, q);
     Leg<D> g;
-    leg_from<D>(sh.leg[wave], sh.slot[wave], g);
+    leg_from<D>(sh.leg[wave], sh.time[wave], g);
     const bool hashed = a.log != nullptr;
     if (step == STEP_CREATE) {
         general_creates<D, FM, NT, RES>(a, q, g, sh, arg, 0, from, hashed);
@@ -2146,7 +2183,8 @@ __device__ __noinline__ static void rare_step(const ChainArgs *args, ChainShared
             if (chosen < 0) g.err = ECMC_ERR_SCHEDULER;
         }
         if (!g.err) {
-            wave_sync();
+            if (NT > 64) __syncthreads();   // the payloads are thread 0's
+            else wave_sync();
             Event<D> e;
             event_of_slot<D, NT>(sh, chosen, e);
             e.t.q = lane_d(g.lt.q, chosen);
@@ -2166,7 +2204,7 @@ __device__ __noinline__ static void rare_step(const ChainArgs *args, ChainShared
         }
     }
     if (NT > 64) __syncthreads();   // lists that other wavefronts read are edited by the next leg
-    leg_to<D>(g, sh.leg[wave], sh.slot[wave]);
+    leg_to<D>(g, sh.leg[wave], sh.time[wave]);
     wave_sync();
 }
 
@@ -2176,7 +2214,7 @@ __device__ __noinline__ static void rare_step(const ChainArgs *args, ChainShared
 enum { HOT_EVENT = 0, HOT_STORED = 1, HOT_GENERAL = 2 };
 template <int D, int FM, int NT, bool RES>
 __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh, const HotList &hot,
-                                          const Pick &stored, bool hashed, Event<D> &e) {
+                                          const Items &constants, const Pick &stored, bool hashed, Event<D> &e) {
     constexpr int NW = NT / 64;
     const int lane = threadIdx.x & 63, wave = wave_index<NT>();
     const uint64_t cursor0 = g.cursor;
@@ -2211,10 +2249,9 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
         if (S.w < 0 || ub(time_lt(B.p.t, S.t))) S = B.p;
         else if (ub(time_eq(B.p.t, S.t))) return general();
     }
-    Counts cn = {-1, 0, -1};
-    Items its;
-    its.count = hot.items;
-    its.tags = hot.tags;
+    Counts cn;
+    cn.nb = cn.far = -1;
+    Items its = constants;
     its.word = (uint32_t)(g.cursor - cursor0);
     its.rank = its.before = 0;
     const int pre = (int)(g.seq - seq0) - (hot.boundary >= 0 ? 1 : 0);
@@ -2294,7 +2331,7 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
         const int workers = NW > 1 && !direct ? NW - 1 : NW;
         int b = direct ? wave * 64 : (NW > 1 ? (wave == 0 ? 0 : (wave == maker ? total : (wave - 1) * 64)) : 0);
         const int count = direct ? M0 : total;
-        Candidates<D, FM, NT, RES> cs(a, q, sh, tag0, kind_of(q.kinds, tag0), g.active, M0, cn.nb_cells);
+        Candidates<D, FM, NT, RES> cs(a, q, sh, tag0, kind_of(q.kinds, tag0), g.active, M0, cn);
         const uint32_t word0 = item_word(its, 0);
         const int rank0 = item_rank(its, 0);
 #pragma unroll 1
@@ -2393,13 +2430,27 @@ __device__ __forceinline__ void chain_body(const ChainArgs &a) {
     hot.creators = (uint32_t)uni((int)sh.hot.creators);
     hot.prefixed = (uint32_t)uni((int)sh.hot.prefixed);
     hot.trashers = (uint32_t)uni((int)sh.hot.trashers);
+    Items its;
+    its.count = hot.items;
+    its.tags = hot.tags;
+    its.word = 0;
+    its.rank = its.before = 0;
+    {
+        const int i = min((int)(threadIdx.x & 63), HOT_ITEMS - 1), t = item_tag(its, i);
+        const ecmc_tagger_desc &tg = sh.tg[t];
+        const int test = (q.tests >> (2 * t)) & 3;
+        its.p = sh.plan[t].p;
+        its.rc2_hi = sh.plan[t].rc2_hi;
+        its.set_key = sh.plan[t].set_key;
+        its.pref = test == QT_INVERSE_POWER ? (float)tg.par[1] : (float)tg.bpar[0];
+    }
     const int64_t max_events = a.max_events;
     ecmc_event *const log = a.log;
     const int stop_mask = a.stop_mask, occupancy = a.occupancy;
     auto rare = [&](int step, int arg, int from) {
-        leg_to<D>(g, sh.leg[wave], sh.slot[wave]);
+        leg_to<D>(g, sh.leg[wave], sh.time[wave]);
         rare_step<D, FM, NT, RES>(&a, &sh, step, arg, from);
-        leg_from<D>(sh.leg[wave], sh.slot[wave], g);
+        leg_from<D>(sh.leg[wave], sh.time[wave], g);
     };
     Pick stored = pick_stored(g);
     int64_t k = 0;
@@ -2428,7 +2479,7 @@ __device__ __forceinline__ void chain_body(const ChainArgs &a) {
                     if ((hot.mask >> (threadIdx.x & 15)) & 1u) g.lvalid = 0;   // created anew
                     stored = pick_stored(g);
                 }
-                done = hot_events<D, FM, NT, RES>(a, q, g, sh, hot, stored, log != nullptr, e);
+                done = hot_events<D, FM, NT, RES>(a, q, g, sh, hot, its, stored, log != nullptr, e);
             }
         }
         int w;
@@ -2500,7 +2551,8 @@ __global__ __launch_bounds__(NT) void chain_step_kernel(const ChainArgs *__restr
             g.chash = 0;
         } else if (!g.err) {
             const int kind = kind_of(q.kinds, t);
-            Counts cn = {-1, 0, -1};
+            Counts cn;
+            cn.nb = cn.far = -1;
             if (kind == ECMC_TAG_CELL_BOUNDARY) {
                 Boundary b;
                 b.p.w = -1;
@@ -2515,7 +2567,7 @@ __global__ __launch_bounds__(NT) void chain_step_kernel(const ChainArgs *__restr
     } else {
         Event<D> e;
         event_of_slot<D, NT>(sh, t, e);
-        e.t = uni(own_slot<D, NT>(sh, t).t);
+        e.t = uni(sh.slot[t].t);
         ecmc_event ev;
         commit_event<D, F, NT, false, false>(a, q, g, sh, e, ev);
         g.last = e.t;
