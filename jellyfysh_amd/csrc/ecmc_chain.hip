@@ -198,6 +198,7 @@ struct ecmc_system {
     ecmc_event *d_log = nullptr;
     int64_t log_cap = 0;
     int64_t *d_nout = nullptr;
+    HostView *host = nullptr;          // pinned: what the last launch left for the host to read
     ecmc_event *d_step_ev = nullptr;   // the event of the last host-driven commit
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -739,6 +740,20 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
         }
     }
     plan_lds(s);
+    // the host view; a system without one (pinned memory exhausted) copies what it reads
+    const bool res_positions = s->args.resident != 0;
+    if (hipHostMalloc((void **)&s->host, sizeof(HostView) + (res_positions ? sizeof(double) * dim * n : 0),
+                      hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
+        void *seen = nullptr;
+        if (hipHostGetDevicePointer(&seen, s->host, 0) != hipSuccess) { ecmc_system_destroy(s); return ecmc_fail(ECMC_ERR_HIP, "hipHostGetDevicePointer failed"); }
+        s->host->st = st;
+        s->host->n_out = 0;
+        s->host->has_positions = 0;
+        a.host = (HostView *)seen;
+    } else {
+        s->host = nullptr;
+        (void)hipGetLastError();
+    }
     *out = s;
     return ECMC_OK;
 }
@@ -749,6 +764,7 @@ extern "C" void ecmc_system_destroy(ecmc_system *s) {
     hipFree(s->d_occ); hipFree(s->d_occ_n); hipFree(s->d_ring); hipFree(s->d_st);
     hipFree(s->d_sur_cell); hipFree(s->d_sur_id); hipFree(s->d_cbt); hipFree(s->d_corners);
     hipFree(s->d_cvw);
+    if (s->host) hipHostFree(s->host);
     hipFree(s->d_tg); hipFree(s->d_nout); hipFree(s->d_log); hipFree(s->d_ewald); hipFree(s->d_ewald_codes); hipFree(s->d_step_ev); hipFree(s->d_args);
     if (s->ev0) hipEventDestroy(s->ev0);
     if (s->ev1) hipEventDestroy(s->ev1);
@@ -756,15 +772,35 @@ extern "C" void ecmc_system_destroy(ecmc_system *s) {
     delete s;
 }
 
-static int status_of_state(const ChainState &st) {
-    switch (st.err) {
+static int status_of_state(int err) {
+    switch (err) {
     case 0: return ECMC_OK;
     case ECMC_ERR_SCHEDULER: return ecmc_fail(ECMC_ERR_SCHEDULER, "SchedulerError: no event or decreasing event time");
     case ECMC_ERR_STATE: return ecmc_fail(ECMC_ERR_STATE, "a position left the cell system or an occupancy list overflowed");
     case ECMC_ERR_NUMERIC: return ecmc_fail(ECMC_ERR_NUMERIC, "ValueError: math domain error in a displacement");
     case ECMC_ERR_CONFIGURATION: return ecmc_fail(ECMC_ERR_CONFIGURATION, "end-of-chain time assertion or missing start of run");
-    default: return ecmc_fail(st.err, "device error");
+    default: return ecmc_fail(err, "device error");
     }
+}
+
+// The state that the last launch left (or the initial one): from the host view, else copied.
+static int read_state(const ecmc_system *s, ChainState &st) {
+    if (s->host) st = s->host->st;
+    else if (hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
+        return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
+    return ECMC_OK;
+}
+
+// The committed legs of the launch that just ended and its error code.
+static int read_launch(const ecmc_system *s, int64_t &k, int &err) {
+    if (s->host) {
+        k = s->host->n_out;
+        err = s->host->st.err;
+    } else if (hipMemcpy(&k, s->d_nout, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess ||
+               hipMemcpy(&err, (const char *)s->d_st + offsetof(ChainState, err), sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
+        return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
+    }
+    return ECMC_OK;
 }
 
 extern "C" int ecmc_system_run(ecmc_system *s, int64_t max_events, ecmc_event *host_log, int64_t *n_committed) {
@@ -798,15 +834,13 @@ extern "C" int ecmc_system_run(ecmc_system *s, int64_t max_events, ecmc_event *h
     hipEventElapsedTime(&ms, s->ev0, s->ev1);
     s->last_ms = ms;
     int64_t k = 0;
-    ChainState st;
-    if (hipMemcpy(&k, s->d_nout, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess ||
-        hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
-        return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
+    int err = 0, rc = read_launch(s, k, err);
+    if (rc) return rc;
     if (host_log && k > 0 &&
         hipMemcpy(host_log, s->d_log, sizeof(ecmc_event) * k, hipMemcpyDeviceToHost) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy of the event log failed");
     if (n_committed) *n_committed = k;
-    return status_of_state(st);
+    return status_of_state(err);
 }
 
 // The launch of independent systems with their arguments staged in `host_args` (count
@@ -853,12 +887,10 @@ static int systems_run_staged(ecmc_system *const *systems, int32_t count, int64_
         ecmc_system *s = systems[i];
         s->last_ms = ms;
         int64_t k = 0;
-        ChainState st;
-        if (hipMemcpy(&k, s->d_nout, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess ||
-            hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
-            return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
+        int err = 0, read = read_launch(s, k, err);
+        if (read) return read;
         if (n_committed) n_committed[i] = k;
-        if (rc == ECMC_OK) rc = status_of_state(st);
+        if (rc == ECMC_OK) rc = status_of_state(err);
     }
     return rc;
 }
@@ -939,9 +971,9 @@ static int system_step(ecmc_system *s, int op, int tagger, ChainState &st) {
     else hipLaunchKernelGGL((chain_step_kernel<3, FEAT_ALL, 256>), dim3(1), dim3(256), 0, s->stream, s->d_args, op, tagger, s->d_step_ev);
     if (hipGetLastError() != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "kernel launch failed");
     if (hipStreamSynchronize(s->stream) != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "kernel execution failed");
-    if (hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
-        return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
-    return status_of_state(st);
+    const int rc = read_state(s, st);
+    if (rc) return rc;
+    return status_of_state(st.err);
 }
 
 extern "C" int ecmc_system_begin_leg(ecmc_system *s) {
@@ -966,11 +998,9 @@ extern "C" int ecmc_system_send_out_state(ecmc_system *s, int32_t tagger, ecmc_e
     ChainState st;
     if (s && tagger >= 0 && tagger < s->desc.n_taggers) {
         // the handler must hold an event (the host's scheduler never returns one without)
-        Slot sl;
-        if (hipMemcpy(&sl, (const char *)s->d_st + offsetof(ChainState, slot) + sizeof(Slot) * tagger, sizeof(Slot),
-                      hipMemcpyDeviceToHost) != hipSuccess)
-            return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
-        if (!sl.valid) return ecmc_fail(ECMC_ERR_SCHEDULER, "the event handler holds no event");
+        const int read = read_state(s, st);
+        if (read) return read;
+        if (!st.slot[tagger].valid) return ecmc_fail(ECMC_ERR_SCHEDULER, "the event handler holds no event");
     }
     const int rc = system_step(s, 2, tagger, st);
     if (rc) return rc;
@@ -981,17 +1011,15 @@ extern "C" int ecmc_system_send_out_state(ecmc_system *s, int32_t tagger, ecmc_e
 
 extern "C" int ecmc_system_positions(const ecmc_system *s, double *out) {
     if (!s || !out) return ecmc_fail(ECMC_ERR_ARGUMENT, "null argument");
+    if (s->host && s->host->has_positions) {
+        memcpy(out, s->host + 1, sizeof(double) * s->dim * s->n);
+        return ECMC_OK;
+    }
     std::vector<double> soa((size_t)s->dim * s->n);
     if (hipMemcpy(soa.data(), s->d_pos, sizeof(double) * soa.size(), hipMemcpyDeviceToHost) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
     for (int i = 0; i < s->n; i++)
         for (int d = 0; d < s->dim; d++) out[(size_t)i * s->dim + d] = soa[(size_t)d * s->n + i];
-    return ECMC_OK;
-}
-
-static int read_state(const ecmc_system *s, ChainState &st) {
-    if (hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
-        return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
     return ECMC_OK;
 }
 

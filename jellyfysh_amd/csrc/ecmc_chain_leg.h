@@ -80,6 +80,18 @@ struct ChainState {
     Slot slot[ECMC_MAX_TAGGERS];
 };
 
+// What the host reads after a launch, written by the launch's last instructions into pinned host
+// memory that the system owns: the state, the committed legs and, of a launch that kept the
+// positions in LDS, the positions (n x dim) behind this block.  Reading it costs no copy command:
+// the four of a system (committed legs, state, positions, estimators), at 10 to 17 us each, were
+// 14.1 of 40.6 ms where 256 systems of 512 units run 1000 legs and 14.6 of 26.5 ms where 256
+// two-unit systems run to their next sample.
+struct HostView {
+    ChainState st;
+    int64_t n_out;
+    int32_t has_positions, pad;
+};
+
 struct ChainArgs {
     int32_t n, ncells, nb_stride, occ_cap, ring_words, n_taggers, stop_mask, leaves;   // leaves: leaf units per
                                                                                        // composite object (1: point masses)
@@ -101,6 +113,7 @@ struct ChainArgs {
     const ecmc_tagger_desc *tg;
     ecmc_event *log;
     int64_t max_events;
+    HostView *host;            // device address of the system's host view (null: the host copies what it reads)
     int64_t *n_out;
     // bounded occupancy (single_active_cell_occupancy.py:62) and cell bounding
     int32_t max_occ, layers;
@@ -2020,6 +2033,21 @@ __device__ __forceinline__ void launch_store(const ChainArgs &a, const Geo<D> &q
                     a.sur_cell[i] = sur_cell<true>(a, q, i);
                     a.sur_id[i] = sur_id<true>(a, q, i);
                 }
+        }
+    }
+    if (a.host) {
+        __syncthreads();   // the state is thread 0's and the first lanes'
+        const uint64_t *from = reinterpret_cast<const uint64_t *>(a.st);
+        uint64_t *to = reinterpret_cast<uint64_t *>(&a.host->st);
+        for (int i = tid; i < (int)(sizeof(ChainState) / 8); i += NT) to[i] = from[i];
+        if (tid == 0) {
+            a.host->n_out = *a.n_out;
+            a.host->has_positions = RES ? 1 : 0;
+        }
+        if (RES) {
+            const double *lp = reinterpret_cast<const double *>(q.dyn);
+            double *out = reinterpret_cast<double *>(a.host + 1);
+            for (int i = tid; i < D * q.n; i += NT) out[i] = lp[(i % D) * q.n + i / D];
         }
     }
 }
