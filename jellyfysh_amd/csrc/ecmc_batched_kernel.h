@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "../../include/jellyfysh_amd.h"
 #include "ecmc_math.h"
 #include "ecmc_potentials.h"
@@ -11,10 +13,10 @@ namespace ecmc {
 
 constexpr int B_MAX_WPR = 8;
 constexpr int B_CONTENDERS = 48;     // contenders per leg (about 7 typical; beyond, all candidates go exact)
-constexpr int B_QUEUE = 128;         // per-wavefront queue of candidates past the geometric test
+constexpr int B_QUEUE = 256;         // per-wavefront queue of candidates past the capsule test (63 left + 3 x 64)
 constexpr int B_MAX_CPS = 8;         // cells per side handled in LDS (512 cells)
 // the chunk start counts units per cell in the (then idle) contender and queue area
-static_assert(36 * B_CONTENDERS + 4 * B_QUEUE >= 4 * B_MAX_CPS * B_MAX_CPS * B_MAX_CPS, "cell counts do not fit");
+static_assert(36 * B_CONTENDERS + 2 * B_QUEUE >= 4 * B_MAX_CPS * B_MAX_CPS * B_MAX_CPS, "cell counts do not fit");
 
 struct ReplicaDev {
     int32_t n, cps;
@@ -87,77 +89,54 @@ __device__ __forceinline__ int bcell1(double x, double side, int cps) {
 // ---- FP32 lower bound of the truncated inverse-power event displacement ------------------
 // (the bracketing helpers up, dn, rcp1, sqrt_up, sqrt_dn and dU_lower are in ecmc_fp32_bounds.h)
 
-// V(r2) = K / r2^(p/2) with p in {6, 12} (integer powers by multiplication), bounded up
-// (hi) or down for an r2 that is itself a lower/upper bound.  Three products (2^-24 each) and
-// K * rcp(rp) (3 x 2^-24) stay inside an 8 x 2^-24 allowance, to which ETA is added; the two
+// 1 / r2^(p/2) with p in {6, 12} (integer powers by multiplication), bounded up (hi) or down for
+// an r2 that is itself a lower/upper bound.  At most four products (2^-24 each), K's conversion
+// and K * rcp(rp) (3 x 2^-24) stay inside an 8 x 2^-24 allowance, to which ETA is added; the two
 // factors are one constant, (1 +- 2^-21)(1 +- 2^-17) without its 2^-38 term (the side that
 // widens the bound), applied with one more rounding.
-__device__ __forceinline__ float vpow_bound(float K, float r2, int half_p, bool hi) {
+__device__ __forceinline__ float vpow_bound(float K, float r2, bool twelve, bool hi) {
     float r3 = r2 * r2 * r2;
-    float rp = half_p == 6 ? r3 * r3 : r3;
+    float rp = twelve ? r3 * r3 : r3;
     float v = K * rcp1(rp);
     return v * (hi ? 1.f + 0x1p-17f + 0x1p-21f : 1.f - 0x1p-17f - 0x1p-21f);
 }
 
-// (K / V)^(2/p) bounded up (hi) or down.
-__device__ __forceinline__ float rstar2_bound(float K, float V, float two_over_p, bool hi) {
-    float q = K * rcp1(V);
-    float r = exp2f(two_over_p * log2f(q));
-    return hi ? r * (1.f + ETA_POW) : r * (1.f - ETA_POW);
-}
-
-struct Geo {
-    float sd_lo, sd_hi, perp2_lo, perp2_hi, r2_lo, r2_hi;
+// A candidate's separation as pass 1 bounds it: along the motion (sd_lo <= sd <= sd_hi), squared
+// across it, squared in all.
+struct Reach {
+    float sd_lo, sd_hi, perp2_lo, perp2_hi;
 };
 
-// Lower bound of the exact displacement of one factor, or +INF when the factor surely has
-// no event, given the exponential draw's lower bound dU_lo.
-__device__ float factor_lower_bound(const Geo &g, float k, int p, float rc2_hi, float vrc_lo, float dU_lo) {
-    const float INF = __int_as_float(0x7f800000);
-    const int half_p = p / 2;
-    const float two_over_p = half_p == 6 ? 1.f / 6.f : 1.f / 3.f;
-    if (g.perp2_lo >= rc2_hi) return INF;
-    if (k > 0.f) {
-        if (g.sd_hi <= 0.f) return INF;
-        float ueff_lo = fmaxf(vpow_bound(k, g.r2_hi, half_p, false), vrc_lo);
-        float umax_hi = vpow_bound(k, fmaxf(g.perp2_lo, 1e-30f), half_p, true);
-        float room_hi = up(umax_hi - ueff_lo);
-        if (dU_lo >= room_hi) return INF;
-        float ut_lo = dn(ueff_lo + dU_lo);
-        float rs2_hi = rstar2_bound(k, ut_lo, two_over_p, true);
-        float x_hi = sqrt_up(fmaxf(up(rs2_hi - g.perp2_lo), 0.f));
-        float d = dn(g.sd_lo) - x_hi;
-        d = d - fabsf(d) * 0x1p-22f;
-        return fmaxf(d, 0.f);
-    }
-    const float K = -k;
-    float x0sq_lo = g.sd_hi < 0.f ? sq_lo(-g.sd_hi) : 0.f;
-    float r02_lo = dn(g.perp2_lo + x0sq_lo);
-    if (r02_lo >= rc2_hi) return INF;
-    float vcur_hi = vpow_bound(K, fmaxf(r02_lo, 1e-30f), half_p, true);
-    float room_hi = up(vcur_hi - vrc_lo);
-    if (dU_lo >= room_hi) return INF;
-    float vt_hi = up(vcur_hi - dU_lo);
-    if (!(vt_hi > 0.f)) return 0.f;
-    float rs2_lo = rstar2_bound(K, vt_hi, two_over_p, false);
-    float y_lo = sqrt_dn(fmaxf(dn(rs2_lo - g.perp2_hi), 0.f));
-    float d = g.sd_lo + y_lo;
-    d = d - fabsf(d) * 0x1p-22f - 0x1p-40f;
-    return fmaxf(d, 0.f);
+// True when the factor surely has no event within the displacement hf, given the exponential
+// draw's lower bound dU_lo.  An event within hf means that the truncated energy rises by the draw
+// on the way there, and the energy rises on one stretch only:
+//   repulsive (k > 0)  a unit ahead, from the start (or the cutoff sphere) to the closest approach
+//                      or hf: rise = V(nearest) - max(V(start), V(rc)), V = k / r^p;
+//   attractive         from the closest approach (or the start, for a unit behind) to hf or the
+//                      cutoff: rise = V(nearest) - max(V(at hf), V(rc)), V = |k| / r^p.
+// Bounded up with the nearest distance from below and the farther one from above; no power or
+// logarithm has to be inverted for it (a bound on the displacement itself takes two exp2/log2
+// pairs and a root per factor: 350 instead of 200 instructions per 64 candidates).  Infinite or
+// NaN bounds (a nearest distance of zero) keep the candidate.
+__device__ __forceinline__ bool factor_surely_later(const Reach &g, float k, bool twelve, float rc2_hi, float vrc_lo, float hf,
+                                                    float dU_lo) {
+    const bool rep = k > 0.f;
+    const float K = fabsf(k);
+    const float x_near = fmaxf(rep ? g.sd_lo - hf : -g.sd_hi, 0.f);
+    const float x_far = rep ? fmaxf(fabsf(g.sd_lo), fabsf(g.sd_hi)) : hf - g.sd_lo;
+    const float near2 = dn(fmaf(x_near, x_near, g.perp2_lo)), far2 = up(fmaf(x_far, x_far, g.perp2_hi));
+    const float low = fmaxf(vpow_bound(K, far2, twelve, false), vrc_lo);
+    const float rise = vpow_bound(K, near2, twelve, true) - low;
+    return (near2 >= rc2_hi) | (rep ? g.sd_hi <= 0.f : g.sd_lo > hf) | (up(rise) < dU_lo);
 }
 
-// Smallest displacement any event of the factor can have, from geometry alone: a repulsive
-// factor first has to reach the cutoff sphere, an attractive one first passes the closest
-// approach.
-__device__ __forceinline__ float factor_geometric_floor(const Geo &g, float k, float rc2_hi) {
-    if (k > 0.f) {
-        if (g.r2_lo < rc2_hi) return 0.f;
-        float entry_hi = sqrt_up(fmaxf(up(rc2_hi - g.perp2_lo), 0.f));
-        float d = dn(g.sd_lo) - entry_hi;
-        d = d - fabsf(d) * 0x1p-22f;
-        return fmaxf(d, 0.f);
-    }
-    return fmaxf(dn(g.sd_lo), 0.f);
+// dU_lower (ecmc_fp32_bounds.h) without its branch: u24 below 2^-10, else the hardware logarithm
+// that log2f is for a normal argument (1 - u24 >= 2^-24), less its error bound.
+__device__ __forceinline__ float dU_lower_flat(uint32_t a, float inv_beta_lo) {
+    const float u24 = (float)(a >> 8) * 0x1p-24f;
+    const float ml2 = -__builtin_amdgcn_logf(1.f - u24);
+    const float l = (ml2 - LOG2F_ERR * fmaxf(ml2, 1.f)) * 0x1.62e42ep-1f;
+    return fmaxf((u24 < 0x1p-10f ? u24 : l) * inv_beta_lo * (1.f - 0x1p-20f), 0.f);
 }
 
 struct BKey {
@@ -192,10 +171,10 @@ __device__ __forceinline__ void dpp_min_step(double &d, int &k) {
 // keys (nlive: lanes beyond hold +inf), the result taken from lane 0, and the returned index
 // is the lane holding the winning key (keys are unique; 0 unless a pair wins), from which the
 // caller reads the candidate's position; with several, a shuffle butterfly, the winning lane
-// of each wavefront leaves that candidate's FP64 position in newpos[3 * wave], and the
-// returned index is the winning wavefront.
+// of each wavefront leaves that candidate's FP64 position in newpos[3 * wave] and its slot in
+// newslot[wave], and the returned index is the winning wavefront.
 template <int WPR>
-__device__ int block_min(BKey &b, const BKey &mine, const double *pos, BKey *sk, double *newpos, int nlive) {
+__device__ int block_min(BKey &b, const BKey &mine, const double *pos, int slot, BKey *sk, double *newpos, int *newslot, int nlive) {
     // (rank, j, f) packed into one word orders like the triple (rank < 4, j < 2^27, f < 2)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double d = b.d;
@@ -238,6 +217,7 @@ __device__ int block_min(BKey &b, const BKey &mine, const double *pos, BKey *sk,
         newpos[3 * wave] = pos[0];
         newpos[3 * wave + 1] = pos[1];
         newpos[3 * wave + 2] = pos[2];
+        newslot[wave] = slot;
     }
     int wb = 0;
     if (WPR > 1) {
@@ -308,45 +288,39 @@ __device__ ECMC_BATCHED_EXACT_ATTR double exact_event(uint32_t wa, uint32_t wb, 
 }
 
 // Positions in LDS: 16-bit fixed point per coordinate, q = round(x 2^16 / L) mod 2^16 (x in
-// [0, L)), one uint16 array per axis.  The separation q_j - q_a wrapped into [-2^15, 2^15) is
-// the minimum image exactly in integers; times L 2^-16 it is within L 2^-16 (two roundings of
-// L 2^-17) plus L 2^-25 (the float product) of the true minimum-image separation, unless that
-// is within the same distance of +-L/2.  The slack E = L 2^-15 covers both.
-__device__ __forceinline__ uint16_t quant1(double x, double inv_step) { return (uint16_t)(uint32_t)(x * inv_step + 0.5); }
-__device__ __forceinline__ float qsep(uint32_t qj, uint32_t qa, float step) {
-    return (float)((int)((qj - qa + 0x8000u) & 0xFFFFu) - 0x8000) * step;
+// [0, L)), with the unit's number in one 8-byte record (x | y << 16, z | unit << 16), the records
+// sorted by cell.  The separation q_j - q_a wrapped into [-2^15, 2^15) is the minimum image
+// exactly in integers (the wrap is that of 16-bit subtraction); times L 2^-16 it is within
+// L 2^-16 (two roundings of L 2^-17) plus L 2^-25 (the float product) of the true minimum-image
+// separation, unless that is within the same distance of +-L/2.  The slack E = L 2^-15 (two
+// steps) covers both.  One read of a record follows the candidate's place directly; three arrays
+// by unit behind a list of units by cell cost four reads in two dependent steps.
+__device__ __forceinline__ uint32_t quant1(double x, double inv_step) { return (uint32_t)(x * inv_step + 0.5) & 0xFFFFu; }
+typedef unsigned short bushort2 __attribute__((ext_vector_type(2)));
+typedef short bshort2 __attribute__((ext_vector_type(2)));
+struct Sep {
+    float x, y, z;   // in steps of L 2^-16, exact
+};
+__device__ __forceinline__ Sep qsep(uint2 rec, uint32_t qa01, uint32_t qa2) {
+    const bshort2 xy = __builtin_bit_cast(bshort2, __builtin_bit_cast(bushort2, rec.x) - __builtin_bit_cast(bushort2, qa01));
+    const short z = (short)(rec.y - qa2);
+    return Sep{(float)xy.x, (float)xy.y, (float)z};
+}
+__device__ __forceinline__ bool qsep_ambiguous(const Sep &s) {   // within 2E of +-L/2 on some axis
+    return fmaxf(fmaxf(fabsf(s.x), fabsf(s.y)), fabsf(s.z)) >= 32764.f;
 }
 
-// FP32 geometry of a candidate from its minimum-image separation: bounds with the position
-// slack E, and whether the minimum image is ambiguous (then the candidate is forced into the
-// contender list).
-__device__ __forceinline__ bool cand_geometry(float dx, float dy, float dz, int d, float Lf, float E, bool check_amb,
-                                              Geo &g) {
-    float sv[3] = {dx, dy, dz};
-    bool ambiguous = false;
-    if (check_amb) {
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-            if (fabsf(fabsf(sv[q]) - 0.5f * Lf) <= 2.f * E) ambiguous = true;
-    }
-    const float sd = d == 0 ? sv[0] : (d == 1 ? sv[1] : sv[2]);
+// The separation's bounds with the position slack E.
+__device__ __forceinline__ Reach cand_reach(const Sep &s, int d, float step, float E) {
+    Reach g;
+    const float sd = (d == 0 ? s.x : (d == 1 ? s.y : s.z)) * step;
     g.sd_lo = sd - E;
     g.sd_hi = sd + E;
-    float p2lo = 0.f, p2hi = 0.f;
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-        if (q == d) continue;
-        const float m = fabsf(sv[q]);
-        const float lo = fmaxf(m - E, 0.f), hi = m + E;
-        p2lo += lo * lo;
-        p2hi += hi * hi;
-    }
-    g.perp2_lo = dn(p2lo);
-    g.perp2_hi = up(p2hi);
-    const float mdl = fmaxf(fabsf(sd) - E, 0.f), mdh = fabsf(sd) + E;
-    g.r2_lo = dn(p2lo + mdl * mdl);
-    g.r2_hi = up(p2hi + mdh * mdh);
-    return ambiguous;
+    const float u = fabsf(d == 0 ? s.y : s.x) * step, v = fabsf(d == 2 ? s.y : s.z) * step;
+    const float ul = fmaxf(u - E, 0.f), vl = fmaxf(v - E, 0.f), uh = u + E, vh = v + E;
+    g.perp2_lo = dn(fmaf(ul, ul, vl * vl));
+    g.perp2_hi = up(fmaf(uh, uh, vh * vh));
+    return g;
 }
 
 // Pre-filter of pass 1 on the fixed-point separation (dx, dy, dz): false only for a candidate
@@ -355,34 +329,33 @@ __device__ __forceinline__ bool cand_geometry(float dx, float dy, float dz, int 
 // no event before its unit enters the cutoff sphere (ahead), an attractive one none for a
 // unit behind beyond the cutoff (its distance only grows) and none ahead before the closest
 // approach (at s_d <= h).  The fixed-point separation is within E of the true one on each
-// axis, so within sqrt(3) E < 2E of it; hf >= h; RB2 = ((rc + 2E)(1 + 2^-20))^2 (1 + 2^-20)
-// covers these and the FP32 roundings.  A separation within 2E of +-L/2 on any axis (minimum
-// image not certain) always passes; check_amb false (uniform) skips that test where no such
-// separation can lie in the capsule.
-__device__ __forceinline__ bool cand_near(float dx, float dy, float dz, int d, float halfL, float E2, float RB2,
-                                          float hf, bool check_amb) {
-    bool amb = false;
-    if (check_amb)
-        amb = fabsf(fabsf(dx) - halfL) <= E2 || fabsf(fabsf(dy) - halfL) <= E2 || fabsf(fabsf(dz) - halfL) <= E2;
-    const float sd = d == 0 ? dx : (d == 1 ? dy : dz);
-    const float u = d == 0 ? dy : dx, v = d == 2 ? dy : dz;
-    const float e = sd - fminf(fmaxf(sd, 0.f), hf);
-    return amb || u * u + v * v + e * e < RB2;
+// axis, so within sqrt(3) E < 2E of it; hq >= h and RQ2 >= (rc + 2E)^2, both in steps.  The
+// squared distance is taken as |s|^2 - s_d^2 + e^2, exact but for float roundings of terms below
+// 3 x 2^30: RQ2 holds 2^11 for them.  A separation within 2E of +-L/2 on any axis (minimum image
+// not certain) always passes; check_amb false (uniform) skips that test where no such separation
+// can lie in the capsule.
+__device__ __forceinline__ bool cand_near(const Sep &s, int d, float RQ2, float hq, bool check_amb) {
+    const float sd = d == 0 ? s.x : (d == 1 ? s.y : s.z);
+    const float e = sd - fminf(fmaxf(sd, 0.f), hq);
+    const float r2 = fmaf(s.x, s.x, fmaf(s.y, s.y, s.z * s.z));
+    const bool near = fmaf(e, e, r2 - sd * sd) < RQ2;
+    return check_amb ? near | qsep_ambiguous(s) : near;
 }
 
-// Occupant lists sorted by cell: move unit x, at slot p of cell X's segment, to cell Y != X
+// Records sorted by cell: move record x, at slot p of cell X's segment, to cell Y != X
 // (one wavefront, uniform arguments).  Going up (Y > X), x leaves through X's last slot (X's
 // last unit fills p), every non-empty cell between passes its last unit to the slot before its
 // first, and x becomes Y's first; going down is the mirror image.  Starts of the cells
 // between, and of the far end, shift by one.  Each pass reads all its slots before it writes.
-__device__ void csr_move(int16_t *cu, int16_t *cs, int p, int X, int Y, int x, int lane) {
+__device__ void csr_move(uint2 *cu, int16_t *cs, int p, int X, int Y, uint2 x, int lane) {
     if (Y > X) {
         const int eX = cs[X + 1] - 1;
-        const int vX = cu[eX];
-        if (lane == 0 && p != eX) cu[p] = (int16_t)vX;
+        const uint2 vX = cu[eX];
+        if (lane == 0 && p != eX) cu[p] = vX;
         for (int c0 = X + 1; c0 < Y; c0 += 64) {
             const int c = c0 + lane;
-            int v = 0, dst = -1;
+            uint2 v = {0u, 0u};
+            int dst = -1;
             if (c < Y) {
                 const int b = cs[c], e = cs[c + 1];
                 if (e > b) {
@@ -391,21 +364,22 @@ __device__ void csr_move(int16_t *cu, int16_t *cs, int p, int X, int Y, int x, i
                 }
             }
             __builtin_amdgcn_wave_barrier();
-            if (dst >= 0) cu[dst] = (int16_t)v;
+            if (dst >= 0) cu[dst] = v;
         }
         __builtin_amdgcn_wave_barrier();
-        if (lane == 0) cu[cs[Y] - 1] = (int16_t)x;
+        if (lane == 0) cu[cs[Y] - 1] = x;
         __builtin_amdgcn_wave_barrier();
         for (int c = X + 1 + lane; c <= Y; c += 64) cs[c] = (int16_t)(cs[c] - 1);
     } else {
         const int fX = cs[X];
-        const int vX = cu[fX];
-        if (lane == 0 && p != fX) cu[p] = (int16_t)vX;
+        const uint2 vX = cu[fX];
+        if (lane == 0 && p != fX) cu[p] = vX;
         // downwards, chunks from the top so that a chunk reads its slots before the chunk below
         // writes into them
         for (int c0 = X - 1; c0 > Y; c0 -= 64) {
             const int c = c0 - lane;
-            int v = 0, dst = -1;
+            uint2 v = {0u, 0u};
+            int dst = -1;
             if (c > Y) {
                 const int b = cs[c], e = cs[c + 1];
                 if (e > b) {
@@ -414,45 +388,54 @@ __device__ void csr_move(int16_t *cu, int16_t *cs, int p, int X, int Y, int x, i
                 }
             }
             __builtin_amdgcn_wave_barrier();
-            if (dst >= 0) cu[dst] = (int16_t)v;
+            if (dst >= 0) cu[dst] = v;
         }
         __builtin_amdgcn_wave_barrier();
-        if (lane == 0) cu[cs[Y + 1]] = (int16_t)x;
+        if (lane == 0) cu[cs[Y + 1]] = x;
         __builtin_amdgcn_wave_barrier();
         for (int c = Y + 1 + lane; c <= X; c += 64) cs[c] = (int16_t)(cs[c] + 1);
     }
 }
 
-// candidate idx -> unit (binary search over the 27 prefix sums, or all units but `a`)
-__device__ __forceinline__ int candidate_unit(int idx, int cps, int a, const int *pref, const int *start,
-                                              const int16_t *cu) {
-    if (!cps) return idx < a ? idx : idx + 1;
+// candidate idx -> slot (binary search over the 27 prefix sums; without cells the slots themselves)
+__device__ __forceinline__ int candidate_slot(int idx, bool whole_box, const int *pref, const int *start) {
+    if (whole_box) return idx;
     int lo = 0, hi = 27;  // pref[lo] <= idx < pref[hi]
     while (hi - lo > 1) {
         int mid = (lo + hi) >> 1;
         if (pref[mid] <= idx) lo = mid;
         else hi = mid;
     }
-    return cu[start[lo] + (idx - pref[lo])];
+    return start[lo] + (idx - pref[lo]);
 }
 
-// Three candidates at once (indices i0, i1, i2 < M with cells): a fixed five-step search over
-// the 28 prefix sums (largest lo with pref[lo] <= idx, pref[27] = M), branch-free, so that the
-// three chains of LDS reads interleave.
-__device__ __forceinline__ void candidate_units3(int i0, int i1, int i2, const int *pref, const int *start,
-                                                 const int16_t *cu, int &j0, int &j1, int &j2) {
-    int lo0 = 0, lo1 = 0, lo2 = 0;
+// The nearby cells as runs of slots.  Cells are numbered along x first, so the three nearby cells
+// of a row (one y and z) are one run of slots where the row does not wrap and two where it does:
+// 9 or 18 runs, run k holding candidates first[k] <= idx < first[k + 1] at slots idx + shift[k].
+// (Culled cells count as empty; a row's live cells always include its middle one or none, so the
+// run's shift is the middle cell's.)  A candidate's run is found by comparing with every first
+// in order: eight comparisons and selects without memory, against five dependent LDS reads of a
+// binary search over 27 cells.
+struct Runs {
+    alignas(16) int first[20];
+    alignas(16) int shift[20];
+};
+// Slots of the candidates idx[0 .. C) over R runs, in place.  (Every run is read once, before its
+// compare: arrays of registers indexed by a select would end in scratch memory.)
+template <int R, int C>
+__device__ __forceinline__ void run_slots(const Runs &s, int (&idx)[C]) {
+    int v[C];
+    const int v0 = s.shift[0];
 #pragma unroll
-    for (int st = 16; st > 0; st >>= 1) {
-        const int t0 = min(lo0 + st, 27), t1 = min(lo1 + st, 27), t2 = min(lo2 + st, 27);
-        const int p0 = pref[t0], p1 = pref[t1], p2 = pref[t2];
-        lo0 = p0 <= i0 ? t0 : lo0;
-        lo1 = p1 <= i1 ? t1 : lo1;
-        lo2 = p2 <= i2 ? t2 : lo2;
+    for (int c = 0; c < C; c++) v[c] = v0;
+#pragma unroll
+    for (int k = 1; k < R; k++) {
+        const int first = s.first[k], shift = s.shift[k];
+#pragma unroll
+        for (int c = 0; c < C; c++) v[c] = idx[c] >= first ? shift : v[c];
     }
-    j0 = cu[start[lo0] + (i0 - pref[lo0])];
-    j1 = cu[start[lo1] + (i1 - pref[lo1])];
-    j2 = cu[start[lo2] + (i2 - pref[lo2])];
+#pragma unroll
+    for (int c = 0; c < C; c++) idx[c] += v[c];
 }
 
 // LDS bytes of the dynamic part for a class (fixed-point positions, cell lists, contenders and
@@ -461,7 +444,7 @@ __host__ __device__ inline size_t batched_lds_bytes(int nmax, int cellmax, int w
     size_t b = 8ull * nmax + 2ull * (cellmax + 1);
     b = (b + 7) & ~7ull;
     b += (24ull + 8ull + 4ull) * B_CONTENDERS;     // positions, random words, identifiers
-    b += 4ull * B_QUEUE * wpr;
+    b += 2ull * B_QUEUE * wpr;
     return (b + 15) & ~15ull;
 }
 
@@ -482,18 +465,19 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NTH = 64 * WPR;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    uint16_t *qx = (uint16_t *)smem, *qy = qx + A.nmax, *qz = qy + A.nmax;
-    int16_t *cu = (int16_t *)(qz + A.nmax);    // units sorted by cell, the active unit left out
-    int16_t *cs = cu + A.nmax;                 // cell c holds cu[cs[c] .. cs[c + 1])
+    uint2 *cu = (uint2 *)smem;                    // records sorted by cell, the active unit left out
+    int16_t *cs = (int16_t *)(cu + A.nmax);       // cell c holds cu[cs[c] .. cs[c + 1])
     size_t off = (8ull * A.nmax + 2ull * (A.cellmax + 1) + 7) & ~7ull;
     int32_t *ccount = (int32_t *)(smem + off);                        // 24 B x B_CONTENDERS: chunk-start cell counts
     uint32_t *cont_w = (uint32_t *)(smem + off + 24 * B_CONTENDERS);  // B_CONTENDERS x 2
-    int32_t *cont_id = (int32_t *)(cont_w + 2 * B_CONTENDERS);       // (j << 1) | f
-    int32_t *queue = cont_id + B_CONTENDERS + wave * B_QUEUE;
+    int32_t *cont_id = (int32_t *)(cont_w + 2 * B_CONTENDERS);       // (slot << 1) | f
+    uint16_t *queue = (uint16_t *)(cont_id + B_CONTENDERS) + wave * B_QUEUE;   // slots
     __shared__ BKey sk[B_MAX_WPR];
     __shared__ int s_item, s_chunk, s_nc, s_overflow, s_nearby[27], s_pref[28], s_M, s_Mfull;
     __shared__ int s_preff[28];   // audit mode: prefix sums over every unit of the 27 cells (none culled)
     __shared__ double s_ap[3], s_newpos[3 * B_MAX_WPR], s_h, s_cb, s_bounds[B_MAX_CPS + 1];
+    __shared__ int s_newslot[B_MAX_WPR];
+    __shared__ Runs s_runs;
     __shared__ ReplicaDev R;
     __shared__ unsigned long long s_geo;   // geometric survivors of the other wavefronts (several per replica)
 
@@ -547,11 +531,9 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         const double L = R.L, side = R.side;
         const double *P = A.pos64 + R.off;
         const double inv_step = 0x1p16 / L;
-        for (int i = tid; i < n; i += NTH) {
-            qx[i] = quant1(P[i], inv_step);
-            qy[i] = quant1(P[(size_t)n + i], inv_step);
-            qz[i] = quant1(P[2 * (size_t)n + i], inv_step);
-        }
+        auto record = [&](int i, double x, double y, double z) {
+            return make_uint2(quant1(x, inv_step) | (quant1(y, inv_step) << 16), quant1(z, inv_step) | ((uint32_t)i << 16));
+        };
         const int ncell = cps ? cps * cps * cps : 0;
         // counting sort of the units by cell; the counts and cursors live in the contender
         // area, which is idle here (4 * 512 bytes fit in it)
@@ -595,7 +577,10 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             }
             bsync();
             for (int i = tid; i < n; i += NTH)
-                if (i != R.active) cu[atomicAdd(&ccount[unit_cell(i)], 1)] = (int16_t)i;
+                if (i != R.active) cu[atomicAdd(&ccount[unit_cell(i)], 1)] = record(i, P[i], P[(size_t)n + i], P[2 * (size_t)n + i]);
+        } else {
+            for (int i = tid; i < n; i += NTH)
+                if (i != R.active) cu[i < R.active ? i : i - 1] = record(i, P[i], P[(size_t)n + i], P[2 * (size_t)n + i]);
         }
         const float Lf = (float)L;
         const float step = (float)(L * 0x1p-16);
@@ -611,9 +596,11 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         const float kf0 = (float)pk0, kf1 = (float)pk1;
         const int pf0 = (int)pw0, pf1 = (int)pw1;
         const float inv_beta_lo = (float)(1.0 / A.beta) * (1.f - 0x1p-22f);
-        // pre-filter constants (cand_near): (rc + 2E)^2 rounded up, half the box
+        // pre-filter constants (cand_near), in steps: (rc + 2E)^2 rounded up
         const float RB = ((float)R.cutoff * (1.f + 0x1p-22f) + 2.f * E) * (1.f + 0x1p-20f);
-        const float RB2 = RB * RB * (1.f + 0x1p-20f);
+        const float inv_stepf = (float)inv_step * (1.f + 0x1p-22f);
+        const float RQ = RB * inv_stepf * (1.f + 0x1p-20f);
+        const float RQ2 = RQ * RQ * (1.f + 0x1p-20f) + 0x1p11f;
         const float halfL = 0.5f * Lf, E2 = 2.f * E;
         // A separation within 2E of +-L/2 on some axis has |s_q| >= L/2 - 2E.  When that exceeds
         // the capsule's reach rc + 2E ahead of the largest horizon (the chain length, rounded
@@ -621,8 +608,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         // pass needs the ambiguity test.
         const float hf_max = (float)A.chain_length * (1.f + 0x1p-22f) + 0x1p-60f;
         const bool check_amb = !(halfL - E2 > (hf_max + RB) * (1.f + 0x1p-20f));
-        // with 3 cells per side the 27 nearby cells are the whole box: candidate idx is unit idx
-        // or idx + 1, past the active unit
+        // with 3 cells per side the 27 nearby cells are the whole box: candidate idx is slot idx
         const bool whole_box = cps == 0 || cps == 3;
         // Replica state through the chunk, in registers (with one wavefront per replica the LDS
         // copy R is only read at the start and written at the end; with several, wavefront 0
@@ -633,6 +619,14 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         double st_ap[3] = {s_ap[0], s_ap[1], s_ap[2]};
         double st_h = 0.0, st_cb = 0.0;
         int st_M = 0, st_pc[3] = {0, 0, 0};
+        bool st_wrap = false;           // the rows of nearby cells wrap (18 runs)
+        int ncell_at = 0, ncell_n = 0;  // lane k < 27: first slot and units of nearby cell k, its coordinates
+        int ncell_c = 0;
+        const int off0 = lane % 3 - 1, off1 = (lane / 3) % 3 - 1, off2 = lane / 9 - 1;
+        if (cps && wave == 0) {
+#pragma unroll
+            for (int q = 0; q < 3; q++) st_pc[q] = bcell1(st_ap[q], side, cps);
+        }
         // Nearby cells that cannot meet the capsule of the next leg are left out of its candidate
         // list (their count is taken as zero): the box distance from the segment [0, h] (h
         // widened to cover hf) must be at least rc + 2E rounded up, plus 2E for the position
@@ -650,81 +644,80 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         // they are the whole box), its cell, horizon and candidate count, and cleared contender
         // counters: wavefront 0, before the first leg and right after each commit (so that no
         // separate barrier precedes pass 1)
-        auto prepare_leg = [&](const double *pa, int dn_, double cl) {
-            int pc[3] = {0, 0, 0};
-            if (cps) {
-#pragma unroll
-                for (int q = 0; q < 3; q++) pc[q] = bcell1(pa[q], side, cps);
-            }
+        auto prepare_leg = [&](double pa0, double pa1, double pa2, int pc0, int pc1, int pc2, int dn_, double cl) {
             double hh = cl, cb = INFINITY;
             if (cps) {
-                cb = s_bounds[pc[dn_] + 1] - pa[dn_];
+                const int pcd = dn_ == 0 ? pc0 : (dn_ == 1 ? pc1 : pc2);
+                cb = s_bounds[pcd + 1] - (dn_ == 0 ? pa0 : (dn_ == 1 ? pa1 : pa2));
                 if (cb < hh) hh = cb;
             }
             int Mv = n - 1, Mf = n - 1;
+            bool wrap = false;
+            if (cps) {
+                const int lim = lane < 27 ? 1 : 0;
+                const int u0 = pc0 + off0, u1 = pc1 + off1, u2 = pc2 + (lane < 27 ? off2 : 0);
+                const int c0 = u0 < 0 ? u0 + cps : (u0 >= cps ? u0 - cps : u0), c1 = u1 < 0 ? u1 + cps : (u1 >= cps ? u1 - cps : u1),
+                          c2 = u2 < 0 ? u2 + cps : (u2 >= cps ? u2 - cps : u2);
+                const int c = c0 + cps * (c1 + cps * c2);
+                ncell_at = cs[c];
+                ncell_n = (cs[c + 1] - ncell_at) * lim;
+                ncell_c = c0 | (c1 << 4) | (c2 << 8);
+            }
             if (cps && !whole_box) {
-                int cnt = 0, cntf = 0;
-                if (lane < 27) {
-                    const int off[3] = {lane % 3 - 1, (lane / 3) % 3 - 1, lane / 9 - 1};
-                    int cc[3];
+                bool live = true;
+                if (cull) {
+                    const float rb = ((float)R.cutoff * (1.f + 0x1p-22f) + 2.f * E) * (1.f + 0x1p-20f);
+                    const float cull_r = (rb * (1.f + 0x1p-20f) + 2.f * E + Lf * 0x1p-18f) * (1.f + 0x1p-20f);
+                    const float cull_r2 = cull_r * cull_r * (1.f + 0x1p-20f);
+                    // the cell's box relative to the active unit (not wrapped: its image on that
+                    // side), against the point 0 across the motion and the segment [0, h] along it
+                    const float top = (float)hh * (1.f + 0x1p-20f) + 0x1p-50f, sidef = (float)side;
+                    float g2 = 0.f;
 #pragma unroll
-                    for (int q = 0; q < 3; q++) cc[q] = (pc[q] + off[q] + cps) % cps;
-                    const int c = cc[0] + cps * (cc[1] + cps * cc[2]);
-                    s_nearby[lane] = cs[c];
-                    cntf = cs[c + 1] - cs[c];
-                    bool live = true;
-                    if (cull) {
-                        const float rb = ((float)R.cutoff * (1.f + 0x1p-22f) + 2.f * E) * (1.f + 0x1p-20f);
-                        const float cull_r = (rb * (1.f + 0x1p-20f) + 2.f * E + Lf * 0x1p-18f) * (1.f + 0x1p-20f);
-                        const float cull_r2 = cull_r * cull_r * (1.f + 0x1p-20f);
-                        // the cell's box relative to the active unit (shifted by L where the
-                        // neighbour wraps), against the point 0 across the motion and the
-                        // segment [0, h] along it
-                        const float top = (float)hh * (1.f + 0x1p-20f) + 0x1p-50f;
-                        float g2 = 0.f;
-#pragma unroll
-                        for (int q = 0; q < 3; q++) {
-                            const double shift = (off[q] < 0 && pc[q] == 0) ? -L : ((off[q] > 0 && pc[q] == cps - 1) ? L : 0.0);
-                            const float lo = (float)(s_bounds[cc[q]] - pa[q] + shift);
-                            const float hi = (float)(s_bounds[cc[q] + 1] - pa[q] + shift);
-                            const float gap = fmaxf(fmaxf(lo - (q == dn_ ? top : 0.f), -hi), 0.f);
-                            g2 += gap * gap;
-                        }
-                        live = g2 < cull_r2;
+                    for (int q = 0; q < 3; q++) {
+                        const float lo = fmaf((float)(q == 0 ? pc0 + off0 : (q == 1 ? pc1 + off1 : pc2 + off2)), sidef,
+                                              -(float)(q == 0 ? pa0 : (q == 1 ? pa1 : pa2)));
+                        float gap = fmaxf(fmaxf(lo - (q == dn_ ? top : 0.f), -(lo + sidef)), 0.f);
+                        // (a row's middle cell never is farther than its neighbours, see Runs)
+                        if (q == 0) gap = off0 == 0 ? 0.f : gap;
+                        g2 = fmaf(gap, gap, g2);
                     }
-                    cnt = live ? cntf : 0;
+                    live = g2 < cull_r2;
                 }
-                // inclusive scans of the 27 counts (kept and all): within each 16-lane row by DPP
-                // row shifts (a lane whose source is outside the row adds 0), then lanes 16-26
-                // add row 0's sum
-                int incl = cnt, inclf = cntf;
-                incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xF, 0xF, false);
-                inclf += __builtin_amdgcn_update_dpp(0, inclf, 0x111, 0xF, 0xF, false);
-                incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, false);
-                inclf += __builtin_amdgcn_update_dpp(0, inclf, 0x112, 0xF, 0xF, false);
-                incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xF, false);
-                inclf += __builtin_amdgcn_update_dpp(0, inclf, 0x114, 0xF, 0xF, false);
-                incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xF, 0xF, false);
-                inclf += __builtin_amdgcn_update_dpp(0, inclf, 0x118, 0xF, 0xF, false);
-                const int row0 = __builtin_amdgcn_readlane(incl, 15), row0f = __builtin_amdgcn_readlane(inclf, 15);
-                if (lane >= 16) {
-                    incl += row0;
-                    inclf += row0f;
+                // inclusive scans of the counts kept (low half) and of all (high half) in one word,
+                // each sum below 2^15: within each 16-lane row by DPP row shifts (a lane whose
+                // source is outside the row adds 0), then lanes 16-26 add row 0's sum
+                const uint32_t own = (live ? (uint32_t)ncell_n : 0u) | ((uint32_t)ncell_n << 16);
+                uint32_t incl = own;
+                incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x111, 0xF, 0xF, false);
+                incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x112, 0xF, 0xF, false);
+                incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x114, 0xF, 0xF, false);
+                incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x118, 0xF, 0xF, false);
+                const uint32_t row0 = (uint32_t)__builtin_amdgcn_readlane((int)incl, 15);
+                incl += lane >= 16 ? row0 : 0u;
+                const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)incl, 26);
+                Mv = (int)(all & 0xFFFFu);
+                Mf = (int)(all >> 16);
+                const int first = (int)((incl - own) & 0xFFFFu), shift = ncell_at - first;
+                // the runs: column 0 of a row begins one, and so does a column after a wrap
+                const bool wrap_lo = pc0 == 0, wrap_hi = pc0 == cps - 1;
+                wrap = wrap_lo || wrap_hi;
+                if (lane < 27) {
+                    s_nearby[lane] = ncell_at;
+                    s_pref[lane + 1] = (int)(incl & 0xFFFFu);
+                    if (A.mode == 2) s_preff[lane + 1] = (int)(incl >> 16);
+                    const int row = lane / 3, col = off0 + 1;
+                    const int run = wrap ? 2 * row + (wrap_lo ? (col > 0) : (col > 1)) : row;
+                    const bool begins = col == 0 || (wrap_lo && col == 1) || (wrap_hi && col == 2);
+                    const bool speaks = col == 1 || (wrap_lo && col == 0) || (wrap_hi && col == 2);
+                    if (begins) s_runs.first[run] = first;
+                    if (speaks) s_runs.shift[run] = shift;
                 }
-                if (lane < 27) s_pref[lane + 1] = incl;
-                if (lane == 0) s_pref[0] = 0;
-                if (A.mode == 2) {
-                    if (lane < 27) s_preff[lane + 1] = inclf;
-                    if (lane == 0) s_preff[0] = 0;
-                }
-                Mv = __builtin_amdgcn_readlane(incl, 26);
-                Mf = __builtin_amdgcn_readlane(inclf, 26);
             }
             st_h = hh;
             st_cb = cb;
             st_M = Mv;
-#pragma unroll
-            for (int q = 0; q < 3; q++) st_pc[q] = pc[q];
+            st_wrap = wrap;
             if (lane == 0) {
                 s_nc = 0;
                 s_overflow = 0;
@@ -732,16 +725,18 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 if (WPR > 1) {
                     s_h = hh;
                     s_cb = cb;
-                    s_M = Mv;
+                    s_M = Mv | (wrap ? 1 << 20 : 0);
                 }
             }
         };
-        if (wave == 0) prepare_leg(st_ap, st_d, st_cl);
+        if (tid == 0) s_pref[0] = s_preff[0] = 0;
+        if (wave == 0) prepare_leg(st_ap[0], st_ap[1], st_ap[2], st_pc[0], st_pc[1], st_pc[2], st_d, st_cl);
         bsync();
         if (WPR > 1) {
             st_h = s_h;
             st_cb = s_cb;
-            st_M = s_M;
+            st_M = s_M & 0xFFFFF;
+            st_wrap = s_M >> 20;
         }
         for (int leg_i = 0; leg_i < legs_now && !st_err; leg_i++) {
             const int a = st_a, d = st_d;
@@ -749,36 +744,33 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             const double ap[3] = {st_ap[0], st_ap[1], st_ap[2]};
             const int M = st_M;
             const double h = st_h;
-            const uint32_t qa0 = quant1(ap[0], inv_step), qa1 = quant1(ap[1], inv_step), qa2 = quant1(ap[2], inv_step);
+            const uint32_t qa01 = quant1(ap[0], inv_step) | (quant1(ap[1], inv_step) << 16), qa2 = quant1(ap[2], inv_step);
             const float hf = (float)h * (1.f + 0x1p-22f) + 0x1p-60f;
+            const float hq = hf * inv_stepf * (1.f + 0x1p-22f);
             BKey best = {INFINITY, 3, 0x7ffffff, 0};   // j < 2^27: the reduction packs (rank, j, f)
             double bestpos[3] = {0.0, 0.0, 0.0};
+            int bestslot = 0;
             unsigned geo_pass = 0;   // geometric survivors of this wavefront (uniform)
             if (A.mode != 1) {
                 // ---- pass 1b: bounds of the queued candidates of this wavefront
                 int nc = 0;   // contenders so far (one wavefront per replica: uniform register)
-                auto bound_queue = [&](int cnt) {
+                auto bound_queue = [&](const uint16_t *from, int cnt) {
                     const bool act = lane < cnt;
                     int j = 0;
                     uint32_t w[4] = {0u, 0u, 0u, 0u};
                     bool con[2] = {false, false};
                     if (act) {
-                        j = queue[lane];
-                        Geo g;
-                        const bool amb = cand_geometry(qsep(qx[j], qa0, step), qsep(qy[j], qa1, step), qsep(qz[j], qa2, step),
-                                                       d, Lf, E, check_amb, g);
-                        philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), (uint32_t)j, 0u, (uint32_t)r, A.seed_lo, w);
+                        j = from[lane];
+                        const uint2 rec = cu[j];
+                        const Sep s = qsep(rec, qa01, qa2);
+                        const bool amb = check_amb && qsep_ambiguous(s);
+                        const Reach g = cand_reach(s, d, step, E);
+                        philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), rec.y >> 16, 0u, (uint32_t)r, A.seed_lo, w);
 #pragma unroll
                         for (int f = 0; f < 2; f++) {
                             if (f >= nf) break;
-                            float t = 0.f;
-                            if (!amb) {
-                                if (g.perp2_lo >= rc2_hi) continue;
-                                if (factor_geometric_floor(g, pick(f, kf0, kf1), rc2_hi) > hf) continue;
-                                t = factor_lower_bound(g, pick(f, kf0, kf1), pick(f, pf0, pf1), rc2_hi, pick(f, vrc0, vrc1),
-                                                       dU_lower(pick(f, w[0], w[2]), inv_beta_lo));
-                            }
-                            con[f] = t <= hf;
+                            con[f] = amb | !factor_surely_later(g, pick(f, kf0, kf1), pick(f, pf0, pf1) == 12, rc2_hi, pick(f, vrc0, vrc1),
+                                                                hf, dU_lower_flat(pick(f, w[0], w[2]), inv_beta_lo));
                         }
                     }
                     // contender slots: with one wavefront per replica from ballots over the whole
@@ -808,45 +800,43 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 // chunks of 64 per wavefront and iteration, so that their LDS reads (cell search,
                 // unit, position) overlap
                 int qn = 0;
-                auto append = [&](bool surv, int j) {
-                    const unsigned long long m = __ballot(surv);
-                    const int before = __popcll(m & ((1ull << lane) - 1ull));
-                    if (surv) queue[qn + before] = j;
-                    qn += __popcll(m);
-                    if (qn >= 64) {
-                        bound_queue(64);
-                        const int rem = qn - 64;
-                        const int v = lane < rem ? queue[64 + lane] : 0;
-                        if (lane < rem) queue[lane] = v;
-                        qn = rem;
+                // C chunks of 64 candidates (a place past the end reads the last candidate again)
+                auto near_chunks = [&](int base, auto chunks) {
+                    constexpr int C = decltype(chunks)::value;
+                    int j[C];
+                    bool s[C];
+#pragma unroll
+                    for (int k = 0; k < C; k++) j[k] = min(base + k * NTH + lane, M - 1);
+                    if (!whole_box) {
+                        if (!st_wrap) run_slots<9, C>(s_runs, j);
+                        else run_slots<18, C>(s_runs, j);
                     }
-                    geo_pass += (unsigned)__popcll(m);
+#pragma unroll
+                    for (int k = 0; k < C; k++)
+                        s[k] = cand_near(qsep(cu[j[k]], qa01, qa2), d, RQ2, hq, check_amb) & (base + k * NTH + lane < M);
+#pragma unroll
+                    for (int k = 0; k < C; k++) {
+                        const unsigned long long m = __ballot(s[k]);
+                        const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                        if (s[k]) queue[qn + before] = (uint16_t)j[k];
+                        qn += __popcll(m);
+                        geo_pass += (unsigned)__popcll(m);
+                    }
                 };
-                for (int base = wave * 64; base < M; base += 3 * NTH) {
-                    const int i0 = base + lane, i1 = base + NTH + lane, i2 = base + 2 * NTH + lane;
-                    int j0, j1, j2;
-                    if (whole_box) {
-                        j0 = i0 < a ? i0 : i0 + 1;
-                        j1 = i1 < a ? i1 : i1 + 1;
-                        j2 = i2 < a ? i2 : i2 + 1;
-                    } else {
-                        candidate_units3(min(i0, M - 1), min(i1, M - 1), min(i2, M - 1), s_pref, s_nearby, cu, j0, j1, j2);
-                    }
-                    bool s0 = false, s1 = false, s2 = false;
-                    if (i0 < M)
-                        s0 = cand_near(qsep(qx[j0], qa0, step), qsep(qy[j0], qa1, step), qsep(qz[j0], qa2, step), d, halfL,
-                                       E2, RB2, hf, check_amb);
-                    if (i1 < M)
-                        s1 = cand_near(qsep(qx[j1], qa0, step), qsep(qy[j1], qa1, step), qsep(qz[j1], qa2, step), d, halfL,
-                                       E2, RB2, hf, check_amb);
-                    if (i2 < M)
-                        s2 = cand_near(qsep(qx[j2], qa0, step), qsep(qy[j2], qa1, step), qsep(qz[j2], qa2, step), d, halfL,
-                                       E2, RB2, hf, check_amb);
-                    append(s0, j0);
-                    append(s1, j1);
-                    append(s2, j2);
+                for (int base = wave * 64;;) {
+                    if (base + 2 * NTH < M) near_chunks(base, std::integral_constant<int, 3>{});
+                    else if (base + NTH < M) near_chunks(base, std::integral_constant<int, 2>{});
+                    else if (base < M) near_chunks(base, std::integral_constant<int, 1>{});
+                    base += 3 * NTH;
+                    const bool last = base >= M;
+                    int done = 0;
+                    for (; qn - done >= (last ? 1 : 64); done += 64) bound_queue(queue + done, min(qn - done, 64));
+                    if (last) break;
+                    const int rem = max(qn - done, 0);
+                    const uint16_t v = queue[done + min(lane, 63)];
+                    if (lane < rem) queue[lane] = v;
+                    qn = rem;
                 }
-                if (qn > 0) bound_queue(qn);
                 if (WPR == 1 && lane == 0) s_nc = nc;
                 bsync();
             }
@@ -854,21 +844,23 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             // ---- pass 2: exact FP64 inversion of the contenders (or of every candidate)
             const int nwork = all_exact ? M * nf : min(s_nc, B_CONTENDERS);
             for (int w = tid; w < nwork; w += NTH) {
-                int j, f;
+                int j, f, slot;
                 double pj[3];
                 uint32_t wa, wb;
                 if (all_exact) {
                     f = w % nf;
                     const int idx = w / nf;
-                    j = whole_box ? (idx < a ? idx : idx + 1) : candidate_unit(idx, cps, a, s_pref, s_nearby, cu);
+                    slot = candidate_slot(idx, whole_box, s_pref, s_nearby);
+                    j = (int)(cu[slot].y >> 16);
                     pj[0] = P[j]; pj[1] = P[(size_t)n + j]; pj[2] = P[2 * (size_t)n + j];
                     uint32_t ww[4];
                     philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), (uint32_t)j, 0u, (uint32_t)r, A.seed_lo, ww);
                     wa = pick(f, ww[0], ww[2]);
                     wb = pick(f, ww[1], ww[3]);
                 } else {
-                    j = cont_id[w] >> 1;
+                    slot = cont_id[w] >> 1;
                     f = cont_id[w] & 1;
+                    j = (int)(cu[slot].y >> 16);
                     // the FP64 position from global memory (its latency overlaps the log of
                     // the draw inside exact_event)
                     pj[0] = P[j]; pj[1] = P[(size_t)n + j]; pj[2] = P[2 * (size_t)n + j];
@@ -882,6 +874,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 if (bkey_lt(c, best)) {
                     best = c;
                     bestpos[0] = pj[0]; bestpos[1] = pj[1]; bestpos[2] = pj[2];
+                    bestslot = slot;
                 }
             }
             if (A.mode == 2) {
@@ -893,7 +886,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 for (int idx = tid; idx < Ma * nf; idx += NTH) {
                     const int f = idx % nf;
                     const int ci = idx / nf;
-                    const int j = whole_box ? (ci < a ? ci : ci + 1) : candidate_unit(ci, cps, a, s_preff, s_nearby, cu);
+                    const int slot = candidate_slot(ci, whole_box, s_preff, s_nearby), j = (int)(cu[slot].y >> 16);
                     uint32_t ww[4];
                     philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), (uint32_t)j, 0u, (uint32_t)r, A.seed_lo, ww);
                     const double dx = exact_event(pick(f, ww[0], ww[2]), pick(f, ww[1], ww[3]), A.beta,
@@ -903,7 +896,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     if (dx <= h) {
                         bool found = false;
                         for (int q = 0; q < min(s_nc, B_CONTENDERS); q++)
-                            if (cont_id[q] == ((j << 1) | f)) found = true;
+                            if (cont_id[q] == ((slot << 1) | f)) found = true;
                         if (!found && !s_overflow) atomicAdd(A.audit, 1ull);
                     }
                 }
@@ -915,7 +908,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 BKey c2k = {st_cl, 2, 0, 0};
                 if (bkey_lt(c2k, best)) best = c2k;
             }
-            const int wbest = block_min<WPR>(best, mine, bestpos, sk, s_newpos, nwork);
+            const int wbest = block_min<WPR>(best, mine, bestpos, bestslot, sk, s_newpos, s_newslot, nwork);
             if (wave == 0) {
                 dst[0] += (unsigned long long)s_Mfull;   // every candidate of the 27 cells
                 dst[2] += (unsigned long long)min(s_nc, B_CONTENDERS);
@@ -928,18 +921,27 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             // wavefront, a ballot finds the new active unit's slot in its cell list, lane 0 writes
             if (wave == 0) {
                 double *Pw = A.pos64 + R.off;
+                // the cell on axis d after the move, from the cell's upper bound (the least double
+                // whose quotient by the side lies in the next cell)
                 double x;
+                const int pc0 = st_pc[0], pc1 = st_pc[1], pc2 = st_pc[2];
+                const double ap0 = ap[0], ap1 = ap[1], ap2 = ap[2], apd = d == 0 ? ap0 : (d == 1 ? ap1 : ap2);
+                int pcd = d == 0 ? pc0 : (d == 1 ? pc1 : pc2);
                 if (best.rank == 1) {
-                    int c = st_pc[d];
-                    x = c + 1 < cps ? s_bounds[c + 1] : 0.0;
+                    x = pcd + 1 < cps ? s_bounds[pcd + 1] : 0.0;
+                    pcd = pcd + 1 < cps ? pcd + 1 : 0;
                 } else {
-                    x = ap[d] + best.d;
-                    if (x >= L) x -= L;
+                    x = apd + best.d;
+                    const bool round = x >= L;
+                    if (round) x -= L;
+                    if (cps) pcd = round ? 0 : (x >= s_bounds[pcd + 1] ? pcd + 1 : pcd);
                 }
                 int newa = a;
-                double np[3] = {ap[0], ap[1], ap[2]};
-                np[d] = x;
+                double np[3] = {d == 0 ? x : ap0, d == 1 ? x : ap1, d == 2 ? x : ap2};
+                int pc[3] = {d == 0 ? pcd : pc0, d == 1 ? pcd : pc1, d == 2 ? pcd : pc2};
                 const double pold[3] = {np[0], np[1], np[2]};
+                const int ca = pc[0] + cps * (pc[1] + cps * pc[2]);
+                int cn = 0, q = -1;
                 if (best.rank == 0) {
                     newa = best.j;
                     if (WPR == 1) {
@@ -947,8 +949,18 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                         for (int k = 0; k < 3; k++)
                             np[k] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(bestpos[k]), wbest),
                                                      __builtin_amdgcn_readlane(__double2loint(bestpos[k]), wbest));
+                        q = __builtin_amdgcn_readlane(bestslot, wbest);
                     } else {
                         np[0] = s_newpos[3 * wbest]; np[1] = s_newpos[3 * wbest + 1]; np[2] = s_newpos[3 * wbest + 2];
+                        q = __builtin_amdgcn_readfirstlane(s_newslot[wbest]);
+                    }
+                    if (cps) {
+                        // the nearby cell whose slots hold the new active unit
+                        const unsigned long long in = __ballot((unsigned)(q - ncell_at) < (unsigned)ncell_n);
+                        const int k = in ? __ffsll((long long)in) - 1 : 0;
+                        const int c = __builtin_amdgcn_readlane(ncell_c, k);
+                        pc[0] = c & 15; pc[1] = (c >> 4) & 15; pc[2] = c >> 8;
+                        if (!in) q = -1;
                     }
                 } else if (best.rank == 2) {
                     uint32_t w[4];
@@ -956,23 +968,26 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     newa = (int)(((uint64_t)w[0] * (uint64_t)n) >> 32);
                     if (newa != a) {
                         np[0] = Pw[newa]; np[1] = Pw[(size_t)n + newa]; np[2] = Pw[2 * (size_t)n + newa];
+                        int from = 0, to = n - 1;
+                        if (cps) {
+#pragma unroll
+                            for (int k = 0; k < 3; k++) pc[k] = __builtin_amdgcn_readfirstlane(bcell1(np[k], side, cps));
+                            const int c = pc[0] + cps * (pc[1] + cps * pc[2]);
+                            from = cs[c];
+                            to = cs[c + 1];
+                        }
+                        for (int base = from; base < to && q < 0; base += 64) {
+                            const unsigned long long mask = __ballot(base + lane < to && (int)(cu[min(base + lane, to - 1)].y >> 16) == newa);
+                            if (mask) q = base + __ffsll((long long)mask) - 1;
+                        }
                     }
                 }
-                int ca = 0, cn = 0, q = -1;
-                if (newa != a && cps) {
-                    ca = bcell1(pold[0], side, cps) + cps * (bcell1(pold[1], side, cps) + cps * bcell1(pold[2], side, cps));
-                    cn = bcell1(np[0], side, cps) + cps * (bcell1(np[1], side, cps) + cps * bcell1(np[2], side, cps));
-                    // the new active unit's slot in its cell's segment
-                    const int b1 = cs[cn + 1];
-                    for (int base = cs[cn]; base < b1 && q < 0; base += 64) {
-                        const unsigned long long mask = __ballot(base + lane < b1 && cu[base + lane] == newa);
-                        if (mask) q = base + __ffsll((long long)mask) - 1;
-                    }
-                }
+                cn = pc[0] + cps * (pc[1] + cps * pc[2]);
                 // the replica's state, alike in every lane of wavefront 0
+                const double np0 = np[0], np1 = np[1], np2 = np[2], npd = d == 0 ? np0 : (d == 1 ? np1 : np2);
                 dest[1] += best.d;
                 if (best.rank == 0) {
-                    dest[0] += bmin_image(np[d] - ap[d], L) - best.d;
+                    dest[0] += bmin_image(npd - apd, L) - best.d;
                     dest[2] += 1.0;
                     dest[4] += 1.0;
                     st_cl -= best.d;
@@ -984,19 +999,20 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     st_cl = A.chain_length;
                     st_d = (d + 1) % 3;
                 }
-                if (newa != a && cps && q < 0) st_err = 2;
+                if (newa != a && q < 0) st_err = 2;
                 st_a = newa;
                 st_leg = leg + 1;
 #pragma unroll
-                for (int k = 0; k < 3; k++) st_ap[k] = np[k];
+                for (int k = 0; k < 3; k++) {
+                    st_ap[k] = np[k];
+                    st_pc[k] = pc[k];
+                }
+                const uint2 old = record(a, pold[0], pold[1], pold[2]);
                 if (lane == 0) {
                     Pw[(size_t)d * n + a] = x;
-                    qx[a] = quant1(pold[0], inv_step);
-                    qy[a] = quant1(pold[1], inv_step);
-                    qz[a] = quant1(pold[2], inv_step);
                     // the old active unit takes the new one's slot (and is moved to the cell it
                     // ended in below)
-                    if (newa != a && cps && q >= 0) cu[q] = (int16_t)a;
+                    if (newa != a && q >= 0) cu[q] = old;
                     if (A.log && leg < (uint64_t)A.log_legs) {
                         ecmc_batch_event ev;
                         ev.kind = best.rank;
@@ -1021,11 +1037,11 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 if (newa != a && cps && q >= 0 && ca != cn) {
-                    csr_move(cu, cs, q, cn, ca, a, lane);
+                    csr_move(cu, cs, q, cn, ca, old, lane);
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
                 }
-                prepare_leg(st_ap, st_d, st_cl);
+                prepare_leg(st_ap[0], st_ap[1], st_ap[2], st_pc[0], st_pc[1], st_pc[2], st_d, st_cl);
             }
             bsync();
             if (WPR > 1) {
@@ -1037,7 +1053,8 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 st_ap[0] = s_ap[0]; st_ap[1] = s_ap[1]; st_ap[2] = s_ap[2];
                 st_h = s_h;
                 st_cb = s_cb;
-                st_M = s_M;
+                st_M = s_M & 0xFFFFF;
+                st_wrap = s_M >> 20;
             }
         }
         if (tid == 0) {

@@ -320,6 +320,62 @@ ECMC_FN double root_pow_fast(double x, bool six, double &lo) {
     return r.h;
 }
 
+// FP32 seeds: log2 of a double in the normal float range and 2 ** y, each within 2^-20
+// (relative to max(|log2 x|, 1) and to 2 ** y), and the reciprocal to about 2^-46.
+ECMC_FN float seed_log2(double x) {
+#if defined(__HIPCC__) && !defined(ECMC_HOST_BUILD)
+    return __builtin_amdgcn_logf((float)x);
+#else
+    return log2f((float)x);
+#endif
+}
+ECMC_FN float seed_exp2(float y) {
+#if defined(__HIPCC__) && !defined(ECMC_HOST_BUILD)
+    return __builtin_amdgcn_exp2f(y);
+#else
+    return exp2f(y);
+#endif
+}
+ECMC_FN double seed_rcp(double x) {
+#if defined(__HIPCC__) && !defined(ECMC_HOST_BUILD)
+    const double r = __builtin_amdgcn_rcp(x);
+    return fma(r, fma(-x, r, 1.0), r);
+#else
+    return 1.0 / x;
+#endif
+}
+
+// t0 (1 + u) ** (-1/k) for u = t0^k / X - 1 (ik = 1/k), the k-th root of X from a seed t0 within
+// 2^-17: the third-order series leaves below 2^-56, the roundings 2^-50.
+ECMC_FN double root_refine(double t0, double u, double ik) {
+    const double c2 = 0.5 * (1.0 + ik), c3 = c2 * (1.0 / 3.0) * (1.0 + ik + ik);
+    return fma(-t0 * ik * u, fma(u, fma(u, c3, -c2), 1.0), t0);
+}
+
+// x ** y for y the double nearest 1/k, k = 3 or 6, and 2^-100 < x < 2^100, as hi + lo with
+// relative error below 2^-68: a root t of about 2^-49 from FP32 seeds and one third-order step,
+// one Newton step on t^k - x in double-double (t^k and x agree to 2^-46, so the difference of the
+// high parts is exact), which leaves (k - 1)/2 (t error)^2, and x^(y - 1/k) = 1 + delta log x with
+// |delta| < 2^-55 and log x from the seed (2^-20 |log2 x|).  About 75 instructions; the path
+// through cbrt, sqrt and the 2^-64 logarithm (root_pow_fast) takes 230.
+ECMC_FN double root36_seeded(double x, bool six, double &lo) {
+    const double ik = six ? 1.0 / 6.0 : 1.0 / 3.0;
+    const float l2 = seed_log2(x);
+    const double t0 = (double)seed_exp2(l2 * (six ? 1.f / 6.f : 1.f / 3.f));
+    const double rx = seed_rcp(x);
+    const double a3 = t0 * t0 * t0;
+    const double t = root_refine(t0, ((six ? a3 * a3 : a3) - x) * rx, ik);
+    const dd t3 = dd_mul_d(two_prod(t, t), t);
+    const dd t6 = dd_mul(t3, t3);
+    const dd tk = six ? t6 : t3;
+    const double corr = t * (((tk.h - x) + tk.l) * (rx * ik));
+    // (y - 1/k) ln 2: the doubles nearest 1/3 and 1/6 are below them by 2^-54 / 3 and 2^-55 / 3
+    const double c = (double)l2 * ((six ? -0x1p-55 : -0x1p-54) * (1.0 / 3.0) * 0x1.62e42fefa39efp-1);
+    const dd r = quick_two_sum(t, fma(t, c, -corr));
+    lo = r.l;
+    return r.h;
+}
+
 // x ** n for an integer 3 <= n <= 32 by binary powering in double-double (each product
 // carries about 2^-104 relative error), rounded once.
 ECMC_FN double dd_pow_int(double x, int n) {
@@ -382,6 +438,30 @@ ECMC_FN double rational_pow_fast(double x, double y, int num, int den, double &l
     return r.h;
 }
 
+// The same from FP32 seeds and one third-order step, for 2^-60 < x < 2^60 and odd den (so that
+// x^num and t^den stay in range), relative error below 2^-66: delta = y - num/den is below
+// 2^-54 and log x comes from the seed.  About 150 instructions for num / den = 2/9 against 420
+// through pow and the 2^-64 logarithm.
+ECMC_FN double rational_pow_seeded(double x, double y, int num, int den, double &lo) {
+    const double id = 1.0 / den;
+    const float l2 = seed_log2(x);
+    const double t0 = (double)seed_exp2(l2 * (float)y);
+    const dd xn = num == 1 ? dd{x, 0.0} : two_prod(x, x);
+    const double rx = seed_rcp(xn.h);
+    double a = 1.0, b = t0;
+    for (int n = den; n > 0; n >>= 1) {
+        a = (n & 1) ? a * b : a;
+        b *= b;
+    }
+    const double t = root_refine(t0, (a - xn.h) * rx, id);
+    const dd tk = dd_pow_int_dd(dd{t, 0.0}, den);
+    const double corr = t * (((tk.h - xn.h) + (tk.l - xn.l)) * (rx * id));
+    const double c = (double)l2 * (fma(y, (double)den, -(double)num) * id * 0x1.62e42fefa39efp-1);
+    const dd r = quick_two_sum(t, fma(t, c, -corr));
+    lo = r.l;
+    return r.h;
+}
+
 // Correctly rounded x ** y for the arguments the potentials use (x > 0): the cases that need
 // more than one operation.  Fast paths with a rounding test first (integer powers, half-integer
 // powers r^(p/2) of odd p, and 2/p for the inversion of an integer power p), then the
@@ -439,10 +519,10 @@ ECMC_FN double pow36(double x, bool six) {
 
 // Correctly rounded x ** (1/3) or x ** (1/6) for the double exponents 1.0/3.0 and 1.0/6.0.
 ECMC_FN double root36(double x, bool six) {
-    if (x > 0x1p-900 && x < 0x1p900) {
+    if (x > 0x1p-100 && x < 0x1p100) {
         double lo;
-        const double hi = root_pow_fast(x, six, lo);
-        if (rounding_settled(hi, lo, 0x1p-92)) return hi + lo;
+        const double hi = root36_seeded(x, six, lo);
+        if (rounding_settled(hi, lo, 0x1p-68)) return hi + lo;   // all but about one call in 10^4
     }
     return cr_pow_slow(x, six ? 1.0 / 6.0 : 1.0 / 3.0);
 }

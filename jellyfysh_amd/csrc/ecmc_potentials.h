@@ -97,10 +97,10 @@ ECMC_FN double pow_half_power(double r2, double power) {
 ECMC_FN double root_two_over_power(double x, double power) {
     if (power == 12.0 || power == 6.0) return root36(x, power == 12.0);
     const double y = 2.0 / power;
-    if (power >= 3.0 && power <= 31.0 && power == rint(power) && ((int)power & 1) && x > 0x1p-300 && x < 0x1p300) {
+    if (power >= 3.0 && power <= 31.0 && power == rint(power) && ((int)power & 1) && x > 0x1p-60 && x < 0x1p60) {
         double lo;
-        const double hi = rational_pow_fast(x, y, 2, (int)power, lo);
-        if (rounding_settled(hi, lo, 0x1p-88)) return hi + lo;
+        const double hi = rational_pow_seeded(x, y, 2, (int)power, lo);
+        if (rounding_settled(hi, lo, 0x1p-66)) return hi + lo;   // else cr_pow's own fast path
     }
     return cr_pow(x, y);
 }
