@@ -129,11 +129,12 @@ static int launch_class(ecmc_batch *b, int c, int legs, hipStream_t st) {
     int per_cu = 1;
 #define ECMC_LAUNCH(W)                                                                                     \
     {                                                                                                      \
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batched_kernel<W>, 64 * W, lds);              \
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batched_kernel<W, false>, 64 * W, lds);       \
         if (per_cu < 1) return ecmc_fail(ECMC_ERR_CONFIGURATION, "replica does not fit in LDS");           \
         int grid = std::min(A.count, per_cu * std::max(cus, 1));                                           \
         if (b->max_blocks > 0) grid = std::min(grid, b->max_blocks);                                       \
-        hipLaunchKernelGGL(batched_kernel<W>, dim3(grid), dim3(64 * W), lds, st, A);                       \
+        if (A.mode) hipLaunchKernelGGL((batched_kernel<W, true>), dim3(grid), dim3(64 * W), lds, st, A);   \
+        else hipLaunchKernelGGL((batched_kernel<W, false>), dim3(grid), dim3(64 * W), lds, st, A);         \
     }
     switch (wpr) {
     case 1: ECMC_LAUNCH(1); break;

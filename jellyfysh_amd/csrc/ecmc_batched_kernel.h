@@ -139,6 +139,22 @@ __device__ __forceinline__ float dU_lower_flat(uint32_t a, float inv_beta_lo) {
     return fmaxf((u24 < 0x1p-10f ? u24 : l) * inv_beta_lo * (1.f - 0x1p-20f), 0.f);
 }
 
+// A value that is alike in all lanes, as a scalar.
+__device__ __forceinline__ int buni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t buni(uint64_t v) {
+    return (uint64_t)(uint32_t)buni((int)(uint32_t)v) | ((uint64_t)(uint32_t)buni((int)(uint32_t)(v >> 32)) << 32);
+}
+
+// The launch arguments, read again from the kernel's argument segment: what a leg needs of them
+// seldom is then not held in scalar registers (or spilled to lanes) through the leg.
+typedef double __attribute__((address_space(1))) gdouble;   // global memory
+typedef const BatchArgs __attribute__((address_space(4))) BatchArgsRef;
+__device__ __forceinline__ BatchArgsRef &again() {
+    uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(BatchArgsRef *)p;
+}
+
 struct BKey {
     double d;
     int32_t rank, j, f;
@@ -251,7 +267,17 @@ __device__ __forceinline__ T pick(int f, T v0, T v1) { return f ? v1 : v0; }
 #ifndef ECMC_BATCHED_WAVES_PER_SIMD
 #define ECMC_BATCHED_WAVES_PER_SIMD 2   // waves per SIMD the register allocation must allow (VGPRs <= 256)
 #endif
-__device__ __forceinline__ double exact_ipt(double s0, double s1, double s2, int d, bool six, double prefactor,
+struct SlowMath {   // correctly rounded for every argument
+    __device__ __forceinline__ double pow36(double x, bool six) { return ecmc::pow36(x, six); }
+    __device__ __forceinline__ double root36(double x, bool six) { return ecmc::root36(x, six); }
+};
+struct FastMath {   // the fast paths alone: ok turns false where they do not settle the rounding
+    bool ok = true;
+    __device__ __forceinline__ double pow36(double x, bool six) { return pow36_settled(x, six, ok); }
+    __device__ __forceinline__ double root36(double x, bool six) { return root36_settled(x, six, ok); }
+};
+template <class Math>
+__device__ __forceinline__ double exact_ipt(Math &m, double s0, double s1, double s2, int d, bool six, double prefactor,
                                             double rc2, double urc, double dU) {
     const double perp2 = d == 0 ? s1 * s1 + s2 * s2 : (d == 1 ? s0 * s0 + s2 * s2 : s0 * s0 + s1 * s1);
     const bool rep = prefactor > 0.0;
@@ -263,10 +289,10 @@ __device__ __forceinline__ double exact_ipt(double s0, double s1, double s2, int
     const double c0 = d == 0 ? sdd : s0, c1 = d == 1 ? sdd : s1, c2 = d == 2 ? sdd : s2;
     const double sn2 = (0.0 + c0 * c0 + c1 * c1) + c2 * c2;
     bool live = perp2 < rc2 && (rep ? sd > 0.0 : sn2 < rc2);
-    const double cur = (rep && !(sn2 < rc2)) ? urc : prefactor / pow36(live ? sn2 : 1.0, six);
-    const double maxp = prefactor / pow36(rep && live ? perp2 : 1.0, six);
+    const double cur = (rep && !(sn2 < rc2)) ? urc : prefactor / m.pow36(live ? sn2 : 1.0, six);
+    const double maxp = prefactor / m.pow36(rep && live ? perp2 : 1.0, six);
     live = live && (rep ? dU < maxp - cur : !(cur + dU >= urc));
-    const double nsq = root36(live ? prefactor / (cur + dU) : 1.0, six);
+    const double nsq = m.root36(live ? prefactor / (cur + dU) : 1.0, six);
     const double a = nsq - perp2;
     const double sq = sqrt(fmax(a, 0.0));
     const double res = a < 0.0 ? NAN : (rep ? sdd - sq : disp + (sdd + sq));
@@ -274,17 +300,22 @@ __device__ __forceinline__ double exact_ipt(double s0, double s1, double s2, int
 }
 
 // The exact FP64 event displacement of one contender: the exponential draw dU = -log(1 - u) /
-// beta from its two words (correctly rounded log), then exact_ipt.  A call, not inlined: the
-// leg loop keeps its state in registers, and inlining this chain pushes the kernel past 256
-// VGPRs into spills (measured slower than the call).
-#ifndef ECMC_BATCHED_EXACT_ATTR
-#define ECMC_BATCHED_EXACT_ATTR __noinline__
-#endif
-__device__ ECMC_BATCHED_EXACT_ATTR double exact_event(uint32_t wa, uint32_t wb, double beta, double s0, double s1,
-                                                      double s2, int d, bool six, double prefactor, double rc2,
-                                                      double urc) {
+// beta from its two words (correctly rounded log), then exact_ipt.  The fast paths of the
+// correctly rounded functions run inlined; the few arguments that they leave open (about one in
+// 500, by the logarithm) take the call, whose registers the leg loop does not hold.
+__device__ __noinline__ double exact_event_slow(uint32_t wa, uint32_t wb, double beta, double s0, double s1, double s2, int d,
+                                                bool six, double prefactor, double rc2, double urc) {
     const double dU = -cr_log(1.0 - unit53(wa, wb)) / beta;
-    return exact_ipt(s0, s1, s2, d, six, prefactor, rc2, urc, dU);
+    SlowMath m;
+    return exact_ipt(m, s0, s1, s2, d, six, prefactor, rc2, urc, dU);
+}
+__device__ __forceinline__ double exact_event(uint32_t wa, uint32_t wb, double beta, double s0, double s1, double s2, int d,
+                                              bool six, double prefactor, double rc2, double urc) {
+    FastMath m;
+    const double dU = -log_settled(1.0 - unit53(wa, wb), m.ok) / beta;
+    double dx = exact_ipt(m, s0, s1, s2, d, six, prefactor, rc2, urc, dU);
+    if (__builtin_expect(!m.ok, 0)) dx = exact_event_slow(wa, wb, beta, s0, s1, s2, d, six, prefactor, rc2, urc);
+    return dx;
 }
 
 // Positions in LDS: 16-bit fixed point per coordinate, q = round(x 2^16 / L) mod 2^16 (x in
@@ -460,8 +491,12 @@ __host__ __device__ inline size_t batched_lds_bytes(int nmax, int cellmax, int w
 //      inversion with correctly rounded pow/log, workgroup min-reduce over (displacement,
 //      kind, target, factor);
 //   5. thread 0 commits.
-template <int WPR>
+//
+// CHECK: modes 1 and 2 (their own instance, so that the filtered mode's registers hold nothing of
+// them).
+template <int WPR, bool CHECK>
 __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched_kernel(BatchArgs A) {
+    const int mode = CHECK ? A.mode : 0;
     extern __shared__ __align__(16) unsigned char smem[];
     constexpr int NTH = 64 * WPR;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -517,19 +552,19 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             }
         }
         bsync();
-        const int member = s_item;
+        const int member = buni(s_item);
         if (member < 0) break;
-        const int r = A.order[member];
+        const int r = buni(A.order[member]);
         if (tid == 0) {
             R = A.rep[r];
             s_geo = 0;
         }
         bsync();
-        const int chunk = s_chunk;
+        const int chunk = buni(s_chunk);
         const int legs_now = min(A.chunk_legs, A.legs - chunk * A.chunk_legs);
-        const int n = R.n, cps = R.cps;
+        const int n = buni(R.n), cps = buni(R.cps);
         const double L = R.L, side = R.side;
-        const double *P = A.pos64 + R.off;
+        gdouble *P = (gdouble *)buni((uint64_t)(A.pos64 + R.off));
         const double inv_step = 0x1p16 / L;
         auto record = [&](int i, double x, double y, double z) {
             return make_uint2(quant1(x, inv_step) | (quant1(y, inv_step) << 16), quant1(z, inv_step) | ((uint32_t)i << 16));
@@ -613,8 +648,8 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         // Replica state through the chunk, in registers (with one wavefront per replica the LDS
         // copy R is only read at the start and written at the end; with several, wavefront 0
         // publishes it to LDS after each commit and every wavefront reloads it)
-        int st_a = R.active, st_d = R.direction, st_err = R.err;
-        uint64_t st_leg = R.leg;
+        int st_a = buni(R.active), st_d = buni(R.direction), st_err = buni(R.err);
+        uint64_t st_leg = buni(R.leg);
         double st_cl = R.chain_left;
         double st_ap[3] = {s_ap[0], s_ap[1], s_ap[2]};
         double st_h = 0.0, st_cb = 0.0;
@@ -625,7 +660,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         const int off0 = lane % 3 - 1, off1 = (lane / 3) % 3 - 1, off2 = lane / 9 - 1;
         if (cps && wave == 0) {
 #pragma unroll
-            for (int q = 0; q < 3; q++) st_pc[q] = bcell1(st_ap[q], side, cps);
+            for (int q = 0; q < 3; q++) st_pc[q] = buni(bcell1(st_ap[q], side, cps));
         }
         // Nearby cells that cannot meet the capsule of the next leg are left out of its candidate
         // list (their count is taken as zero): the box distance from the segment [0, h] (h
@@ -636,7 +671,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         // are on; the audit mode keeps it and checks every candidate of the 27 cells, culled
         // or not.  (The radius is recomputed in each call from the cutoff in LDS, so that it
         // does not hold a register through the leg.)
-        const bool cull = A.mode != 1 && !check_amb;
+        const bool cull = mode != 1 && !check_amb;
         // the estimators, summed leg by leg in the oracle's order (wavefront 0)
         double dest[6] = {R.est[0], R.est[1], R.est[2], R.est[3], R.est[4], R.est[5]};
         unsigned long long dst[4] = {0ull, 0ull, 0ull, 0ull};  // statistics increments (wavefront 0)
@@ -705,7 +740,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 if (lane < 27) {
                     s_nearby[lane] = ncell_at;
                     s_pref[lane + 1] = (int)(incl & 0xFFFFu);
-                    if (A.mode == 2) s_preff[lane + 1] = (int)(incl >> 16);
+                    if (mode == 2) s_preff[lane + 1] = (int)(incl >> 16);
                     const int row = lane / 3, col = off0 + 1;
                     const int run = wrap ? 2 * row + (wrap_lo ? (col > 0) : (col > 1)) : row;
                     const bool begins = col == 0 || (wrap_lo && col == 1) || (wrap_hi && col == 2);
@@ -735,8 +770,8 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
         if (WPR > 1) {
             st_h = s_h;
             st_cb = s_cb;
-            st_M = s_M & 0xFFFFF;
-            st_wrap = s_M >> 20;
+            st_M = buni(s_M) & 0xFFFFF;
+            st_wrap = buni(s_M) >> 20;
         }
         for (int leg_i = 0; leg_i < legs_now && !st_err; leg_i++) {
             const int a = st_a, d = st_d;
@@ -751,7 +786,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             double bestpos[3] = {0.0, 0.0, 0.0};
             int bestslot = 0;
             unsigned geo_pass = 0;   // geometric survivors of this wavefront (uniform)
-            if (A.mode != 1) {
+            if (mode != 1) {
                 // ---- pass 1b: bounds of the queued candidates of this wavefront
                 int nc = 0;   // contenders so far (one wavefront per replica: uniform register)
                 auto bound_queue = [&](const uint16_t *from, int cnt) {
@@ -765,7 +800,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                         const Sep s = qsep(rec, qa01, qa2);
                         const bool amb = check_amb && qsep_ambiguous(s);
                         const Reach g = cand_reach(s, d, step, E);
-                        philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), rec.y >> 16, 0u, (uint32_t)r, A.seed_lo, w);
+                        philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), rec.y >> 16, 0u, (uint32_t)r, again().seed_lo, w);
 #pragma unroll
                         for (int f = 0; f < 2; f++) {
                             if (f >= nf) break;
@@ -840,9 +875,10 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                 if (WPR == 1 && lane == 0) s_nc = nc;
                 bsync();
             }
-            const bool all_exact = (A.mode == 1) || s_overflow;
+            const int listed = buni(s_nc);
+            const bool all_exact = mode == 1 || buni(s_overflow);
             // ---- pass 2: exact FP64 inversion of the contenders (or of every candidate)
-            const int nwork = all_exact ? M * nf : min(s_nc, B_CONTENDERS);
+            const int nwork = all_exact ? M * nf : min(listed, B_CONTENDERS);
             for (int w = tid; w < nwork; w += NTH) {
                 int j, f, slot;
                 double pj[3];
@@ -854,7 +890,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     j = (int)(cu[slot].y >> 16);
                     pj[0] = P[j]; pj[1] = P[(size_t)n + j]; pj[2] = P[2 * (size_t)n + j];
                     uint32_t ww[4];
-                    philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), (uint32_t)j, 0u, (uint32_t)r, A.seed_lo, ww);
+                    philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), (uint32_t)j, 0u, (uint32_t)r, again().seed_lo, ww);
                     wa = pick(f, ww[0], ww[2]);
                     wb = pick(f, ww[1], ww[3]);
                 } else {
@@ -867,7 +903,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     wa = cont_w[2 * w];
                     wb = cont_w[2 * w + 1];
                 }
-                const double dx = exact_event(wa, wb, A.beta, bmin_image(pj[0] - ap[0], L), bmin_image(pj[1] - ap[1], L),
+                const double dx = exact_event(wa, wb, again().beta, bmin_image(pj[0] - ap[0], L), bmin_image(pj[1] - ap[1], L),
                                               bmin_image(pj[2] - ap[2], L), d, pick(f, pf0, pf1) == 12, pick(f, pk0, pk1),
                                               rc2, pick(f, urc0, urc1));
                 BKey c = {dx, 0, j, f};
@@ -877,7 +913,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     bestslot = slot;
                 }
             }
-            if (A.mode == 2) {
+            if (mode == 2) {
                 // audit: every candidate of the 27 cells (or of the whole box), including those in
                 // cells culled from the leg's list, whose exact displacement is <= h must be a
                 // contender (before the selection's barrier: after it, wavefront 0 already
@@ -888,8 +924,8 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     const int ci = idx / nf;
                     const int slot = candidate_slot(ci, whole_box, s_preff, s_nearby), j = (int)(cu[slot].y >> 16);
                     uint32_t ww[4];
-                    philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), (uint32_t)j, 0u, (uint32_t)r, A.seed_lo, ww);
-                    const double dx = exact_event(pick(f, ww[0], ww[2]), pick(f, ww[1], ww[3]), A.beta,
+                    philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), (uint32_t)j, 0u, (uint32_t)r, again().seed_lo, ww);
+                    const double dx = exact_event_slow(pick(f, ww[0], ww[2]), pick(f, ww[1], ww[3]), again().beta,
                                                   bmin_image(P[j] - ap[0], L), bmin_image(P[(size_t)n + j] - ap[1], L),
                                                   bmin_image(P[2 * (size_t)n + j] - ap[2], L), d, pick(f, pf0, pf1) == 12,
                                                   pick(f, pk0, pk1), rc2, pick(f, urc0, urc1));
@@ -897,7 +933,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                         bool found = false;
                         for (int q = 0; q < min(s_nc, B_CONTENDERS); q++)
                             if (cont_id[q] == ((slot << 1) | f)) found = true;
-                        if (!found && !s_overflow) atomicAdd(A.audit, 1ull);
+                        if (!found && !s_overflow) atomicAdd(again().audit, 1ull);
                     }
                 }
             }
@@ -910,8 +946,8 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             }
             const int wbest = block_min<WPR>(best, mine, bestpos, bestslot, sk, s_newpos, s_newslot, nwork);
             if (wave == 0) {
-                dst[0] += (unsigned long long)s_Mfull;   // every candidate of the 27 cells
-                dst[2] += (unsigned long long)min(s_nc, B_CONTENDERS);
+                dst[0] += (unsigned long long)buni(s_Mfull);   // every candidate of the 27 cells
+                dst[2] += (unsigned long long)min(listed, B_CONTENDERS);
                 dst[3] += (unsigned long long)nwork;
             }
             if (WPR == 1) dst[1] += geo_pass;
@@ -920,7 +956,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             // or, with several wavefronts, in s_newpos): the values below are uniform across the
             // wavefront, a ballot finds the new active unit's slot in its cell list, lane 0 writes
             if (wave == 0) {
-                double *Pw = A.pos64 + R.off;
+                gdouble *Pw = P;
                 // the cell on axis d after the move, from the cell's upper bound (the least double
                 // whose quotient by the side lies in the next cell)
                 double x;
@@ -964,7 +1000,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     }
                 } else if (best.rank == 2) {
                     uint32_t w[4];
-                    philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), 0xFFFFFFFFu, 1u, (uint32_t)r, A.seed_lo, w);
+                    philox4x32_10((uint32_t)leg, (uint32_t)(leg >> 32), 0xFFFFFFFFu, 1u, (uint32_t)r, again().seed_lo, w);
                     newa = (int)(((uint64_t)w[0] * (uint64_t)n) >> 32);
                     if (newa != a) {
                         np[0] = Pw[newa]; np[1] = Pw[(size_t)n + newa]; np[2] = Pw[2 * (size_t)n + newa];
@@ -996,7 +1032,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     st_cl -= best.d;
                 } else {
                     dest[5] += 1.0;
-                    st_cl = A.chain_length;
+                    st_cl = again().chain_length;
                     st_d = (d + 1) % 3;
                 }
                 if (newa != a && q < 0) st_err = 2;
@@ -1005,7 +1041,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
                     st_ap[k] = np[k];
-                    st_pc[k] = pc[k];
+                    st_pc[k] = buni(pc[k]);
                 }
                 const uint2 old = record(a, pold[0], pold[1], pold[2]);
                 if (lane == 0) {
@@ -1013,7 +1049,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                     // the old active unit takes the new one's slot (and is moved to the cell it
                     // ended in below)
                     if (newa != a && q >= 0) cu[q] = old;
-                    if (A.log && leg < (uint64_t)A.log_legs) {
+                    if (leg < (uint64_t)again().log_legs) {
                         ecmc_batch_event ev;
                         ev.kind = best.rank;
                         ev.active = a;
@@ -1021,7 +1057,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
                         ev.factor = best.rank == 0 ? best.f : 0;
                         ev.displacement = best.d;
                         ev.x = x;
-                        A.log[(size_t)r * A.log_legs + leg] = ev;
+                        again().log[(size_t)r * again().log_legs + leg] = ev;
                     }
                     if (WPR > 1) {
                         R.active = st_a;
@@ -1045,16 +1081,16 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             }
             bsync();
             if (WPR > 1) {
-                st_a = R.active;
-                st_d = R.direction;
-                st_leg = R.leg;
+                st_a = buni(R.active);
+                st_d = buni(R.direction);
+                st_leg = buni(R.leg);
                 st_cl = R.chain_left;
-                st_err = R.err;
+                st_err = buni(R.err);
                 st_ap[0] = s_ap[0]; st_ap[1] = s_ap[1]; st_ap[2] = s_ap[2];
                 st_h = s_h;
                 st_cb = s_cb;
-                st_M = s_M & 0xFFFFF;
-                st_wrap = s_M >> 20;
+                st_M = buni(s_M) & 0xFFFFF;
+                st_wrap = buni(s_M) >> 20;
             }
         }
         if (tid == 0) {
@@ -1068,7 +1104,7 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             R.stats[1] += (int64_t)(dst[1] + s_geo);
             R.stats[2] += (int64_t)dst[2];
             R.stats[3] += (int64_t)dst[3];
-            A.rep[r] = R;
+            again().rep[r] = R;
         }
         bsync();   // every store of this chunk (positions, log, state) has completed
         if (tid == 0) {
@@ -1076,9 +1112,9 @@ __global__ __launch_bounds__(64 * WPR, ECMC_BATCHED_WAVES_PER_SIMD) void batched
             // one more chunk done
             // (an exchange, whose return is awaited, so this block's next probe sees the update)
             __threadfence();
-            const int prev = __hip_atomic_exchange(A.state + member, (chunk + 1) << 1, __ATOMIC_RELAXED,
+            const int prev = __hip_atomic_exchange(again().state + member, (chunk + 1) << 1, __ATOMIC_RELAXED,
                                                    __HIP_MEMORY_SCOPE_AGENT);
-            if (prev != ((chunk << 1) | 1)) A.rep[r].err = 3;   // the claim protocol was broken
+            if (prev != ((chunk << 1) | 1)) again().rep[r].err = 3;   // the claim protocol was broken
         }
     }
 }

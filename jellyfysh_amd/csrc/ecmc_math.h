@@ -283,6 +283,15 @@ ECMC_SLOW double cr_log_slow(double x) { return dd_log(x).h; }
 // log of zero, negative, infinite, NaN and subnormal arguments
 ECMC_SLOW double log_special(double x) { return log(x); }
 
+// The fast path alone: ok turns false where cr_log would go on (the value is then not to be used).
+ECMC_FN double log_settled(double x, bool &ok) {
+    const bool in = x >= 0x1p-1022 && x < 0x1p1023 && x != 1.0;
+    double lo;
+    const double hi = log_fast(in ? x : 0.5, lo);
+    ok = ok && in && rounding_settled(hi, lo, 0x1p-64);
+    return hi + lo;
+}
+
 // Correctly rounded natural logarithm: the fast path when its rounding is settled (all but
 // about one call in 500), else the double-double path.
 ECMC_FN double cr_log(double x) {
@@ -515,6 +524,21 @@ ECMC_FN double pow36(double x, bool six) {
     const dd x3 = dd_mul_d(x2, x);
     const dd x6 = dd_mul(x3, x3);
     return six ? x6.h : x3.h;
+}
+
+// The fast paths of pow36 and root36 alone, as log_settled.
+ECMC_FN double pow36_settled(double x, bool six, bool &ok) {
+    ok = ok && x > 0x1p-30 && x < 0x1p30;
+    const dd x2 = two_prod(x, x);
+    const dd x3 = dd_mul_d(x2, x);
+    const dd x6 = dd_mul(x3, x3);
+    return six ? x6.h : x3.h;
+}
+ECMC_FN double root36_settled(double x, bool six, bool &ok) {
+    double lo;
+    const double hi = root36_seeded(x, six, lo);
+    ok = ok && x > 0x1p-100 && x < 0x1p100 && rounding_settled(hi, lo, 0x1p-68);
+    return hi + lo;
 }
 
 // Correctly rounded x ** (1/3) or x ** (1/6) for the double exponents 1.0/3.0 and 1.0/6.0.
