@@ -641,6 +641,7 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
     a.ewald.f = s->d_ewald;
     a.ewald_codes = s->d_ewald_codes;
     a.ewald_ncodes = (int32_t)ewald_codes.size();
+    for (int32_t c : ewald_codes) a.ewald_nreal += (c >> 24) == 0;
     a.n_out = s->d_nout;
     a.max_occ = desc->max_occupants;
     a.layers = desc->neighbor_layers;

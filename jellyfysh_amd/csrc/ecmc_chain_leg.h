@@ -129,7 +129,7 @@ struct ChainArgs {
     // a launch and back at its end, and so do the first occ_cols occupants of every cell (16-bit);
     // 0 keeps everything in global memory
     int32_t resident, lds_ring_off, lds_charge_off, lds_occ_off, lds_occn_off, lds_sur_off, occ_cols;
-    int32_t ewald_ncodes;
+    int32_t ewald_ncodes, ewald_nreal;
     // the terms of the merged-image Coulomb derivative in the sequential loop's order (real-space
     // images by k, j, i, then Fourier terms by i, j, k): kind << 24 | (i + 128) << 16 |
     // (j + 128) << 8 | (k + 128), built on the host
@@ -620,6 +620,15 @@ struct SlotTime {
     int64_t seq;
     int32_t valid, pad;
 };
+// The terms of the merged-image Coulomb derivative as the FP32 form takes them: a real-space image and
+// two Fourier terms per lane, where no more are needed (ok).
+struct EwaldTerms {
+    int32_t code[3][64];         // image, Fourier terms (-1: none), as ChainArgs::ewald_codes
+    float f[2][64];
+    double L, inv_l;
+    float aol, aol2, two_aol_rpi;
+    int32_t ok;
+};
 template <int NT>
 struct ChainShared {
     static constexpr int NW = NT / 64;
@@ -631,6 +640,7 @@ struct ChainShared {
     Winner win[NW];
     alignas(16) int32_t nb_cell[NW][32];     // nearby cells and exclusive prefix sums of their occupants
     alignas(16) int32_t nb_pref[NW][32];
+    EwaldTerms ewald;
     uint32_t far_word[NW][64], far_pref[NW][64];
     uint32_t occupied[64];       // one bit per occupied cell (cell bounding, grids of at most FAR_BLOCK cells)
     int32_t qn[NW];
@@ -1626,6 +1636,78 @@ __device__ __noinline__ static double ewald_derivative_wave(const Ewald &e, cons
     return sum;
 }
 
+// The same derivative in FP32 with a bound on its error, for the thinning of an event: the factor's
+// real rate is compared with a draw, and about one comparison in 10^4 is closer than the bound (the
+// FP64 sum above then decides).  Lane terms: one real-space image (creal) and two Fourier terms (cf0,
+// cf1; -1: none).  Separations are reduced in FP64, then per term
+//   real     exp by the hardware's exp2, erfc = exp erfcx (a polynomial of (1 + 2x) erfcx in
+//            (x - 2.5) / (x + 2.5), 2.2e-7 off with its roundings), relative error below
+//            2^-19 + 2^-20 z for the exponent z = a^2 v^2 (z's own relative error is 8 x 2^-24);
+//   Fourier  sines of fractions of a period by the 2e-9 polynomial 4.3.97 of Abramowitz and Stegun,
+//            each within 4e-7, a product of three within 2^-19;
+// and the sum over the lanes adds 9 roundings of partial sums: 2^-18 + 2^-20 z of a real term and
+// 2^-18 |f| of a Fourier term bound it, terms that underflow are 1e-38 of it.  2100 cycles against
+// 9700 of the FP64 sum (an exp, an erfc and two divisions in one chain, three rounds of terms).
+__device__ __forceinline__ float sin_turn(float f) {   // sin(2 pi f) for |f| <= 1/4
+    const float y = f * 6.2831853f, y2 = y * y;
+    return y * fmaf(y2, fmaf(y2, fmaf(y2, fmaf(y2, fmaf(y2, -2.39e-8f, 2.7526e-6f), -1.98409e-4f), 8.3333315e-3f), -0.1666666664f), 1.f);
+}
+__device__ __forceinline__ float wave_total(float v) {   // the sum over the lanes, by DPP
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xF, 0xF, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x112, 0xF, 0xF, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x114, 0xF, 0xF, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x118, 0xF, 0xF, true));
+    const int l = __float_as_int(v);
+    return (__int_as_float(__builtin_amdgcn_readlane(l, 15)) + __int_as_float(__builtin_amdgcn_readlane(l, 31))) +
+           (__int_as_float(__builtin_amdgcn_readlane(l, 47)) + __int_as_float(__builtin_amdgcn_readlane(l, 63)));
+}
+struct EwaldBound {
+    float value, error;
+};
+__device__ __noinline__ static EwaldBound ewald_derivative_fp32(double sx, double sy, double sz, double L, double inv_l, float aol,
+                                                                float aol2, float two_aol_rpi, int creal, int cf0, int cf1, float f0,
+                                                                float f1) {
+    const double px = sx * inv_l, py = sy * inv_l, pz = sz * inv_l;
+    auto fourier = [&](int c, float f) {
+        const double i = (double)(((c >> 16) & 255) - 128), j = (double)(((c >> 8) & 255) - 128), k = (double)((c & 255) - 128);
+        const double ti = i * px, tj = j * py, tk = k * pz;
+        const float a = (float)(ti - rint(ti)), b = fabsf((float)(tj - rint(tj))), d = fabsf((float)(tk - rint(tk)));
+        const float af = fabsf(a);
+        return f * copysignf(sin_turn(af > 0.25f ? 0.5f - af : af), a) * sin_turn(0.25f - b) * sin_turn(0.25f - d);
+    };
+    float sum = 0.f, err = 0.f;
+    if (cf0 >= 0) {
+        sum += fourier(cf0, f0);
+        err += fabsf(f0) * 0x1p-18f;
+    }
+    if (cf1 >= 0) {
+        sum += fourier(cf1, f1);
+        err += fabsf(f1) * 0x1p-18f;
+    }
+    if (creal >= 0) {
+        const float vx = (float)fma((double)(((creal >> 16) & 255) - 128), L, sx), vy = (float)fma((double)(((creal >> 8) & 255) - 128), L, sy),
+                    vz = (float)fma((double)((creal & 255) - 128), L, sz);
+        const float v2 = fmaf(vx, vx, fmaf(vy, vy, vz * vz)), rv = __builtin_amdgcn_rsqf(v2), x = aol * (v2 * rv), z = aol2 * v2;
+        const float E = __builtin_amdgcn_exp2f(-1.4426950f * z);
+        const float hi = fmaf(2.f, x, 1.f), lo = x + 2.5f, r = __builtin_amdgcn_rcpf(lo * hi), t = (x - 2.5f) * hi * r;
+        float p = -0x1.14e136p-14f;
+        p = fmaf(p, t, 0x1.a8737ep-12f);
+        p = fmaf(p, t, 0x1.eb5800p-12f);
+        p = fmaf(p, t, -0x1.11da4ep-8f);
+        p = fmaf(p, t, 0x1.edf72cp-11f);
+        p = fmaf(p, t, 0x1.0baf52p-5f);
+        p = fmaf(p, t, -0x1.a5c2b6p-4f);
+        p = fmaf(p, t, 0x1.42db30p-3f);
+        p = fmaf(p, t, -0x1.959aa8p-4f);
+        p = fmaf(p, t, -0x1.f52d20p-4f);
+        p = fmaf(p, t, 0x1.43cc70p+0f);
+        const float v = vx * (E * fmaf(p * (lo * r), rv, two_aol_rpi)) * (rv * rv);
+        sum += v;
+        err += fabsf(v) * (0x1p-18f + 0x1p-20f * z);
+    }
+    return EwaldBound{wave_total(sum), wave_total(err) * (1.f + 0x1p-10f)};
+}
+
 // ---- commit -------------------------------------------------------------------------------
 // The event to commit: a stored one (from the wavefront's LDS copy) or one of this leg's.
 template <int D>
@@ -1723,16 +1805,29 @@ __device__ __forceinline__ void commit_event(const ChainArgs &a, const Geo<D> &q
                     } else if ((FM & FEAT_COULOMB) && eh == ECMC_EH_TWO_LEAF_BOUNDING) {
                         bound = ipcb_derivative(T.bpar[0] * c1 * c2, q3[0], q3[1], q3[2]) * e.aspeed;
                     }
-                    const double der = ewald_derivative_wave(a.ewald, a.ewald_codes, a.ewald_ncodes, q3[0], q3[1], q3[2]);
-                    const double real = T.par[3] * c1 * c2 * der * e.aspeed;
-                    if (ub(real > 0)) {
-                        // lifting with probability real / bound
-                        const uint32_t w = (uint32_t)g.cursor;
-                        double u = words_to_random(ring_word<RES>(a, q, w), ring_word<RES>(a, q, w + 1));
-                        g.cursor += 2;
-                        u = 0 + (bound - 0) * u;
-                        lift = ub(u < real);
+                    // lifting with probability real / bound (two words, drawn where real > 0)
+                    const uint32_t w = (uint32_t)g.cursor;
+                    double u = words_to_random(ring_word<RES>(a, q, w), ring_word<RES>(a, q, w + 1));
+                    u = 0 + (bound - 0) * u;
+                    bool drawn = false, settled = false;
+                    if (uni(sh.ewald.ok)) {
+                        const EwaldTerms &x = sh.ewald;
+                        const int l = threadIdx.x & 63;
+                        const EwaldBound b = ewald_derivative_fp32(q3[0], q3[1], q3[2], x.L, x.inv_l, x.aol, x.aol2, x.two_aol_rpi,
+                                                                   x.code[0][l], x.code[1][l], x.code[2][l], x.f[0][l], x.f[1][l]);
+                        const double rate = T.par[3] * c1 * c2 * e.aspeed, real = rate * (double)b.value,
+                                     off = fabs(rate) * (double)b.error;
+                        drawn = ub(real - off > 0.0);
+                        lift = drawn & ub(u < real - off);
+                        settled = ub(real + off < 0.0) | (drawn & (lift | ub(u > real + off)));
                     }
+                    if (!settled) {
+                        const double der = ewald_derivative_wave(a.ewald, a.ewald_codes, a.ewald_ncodes, q3[0], q3[1], q3[2]);
+                        const double real = T.par[3] * c1 * c2 * der * e.aspeed;
+                        drawn = ub(real > 0);
+                        lift = drawn & ub(u < real);
+                    }
+                    if (drawn) g.cursor += 2;
                 }
                 if (!lift) add_est(sh, 6, 1.0);
             }
@@ -1856,6 +1951,26 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
     q.leaves = a.leaves; q.max_occ = a.max_occ;
     q.o_ring = a.lds_ring_off; q.o_charge = a.lds_charge_off; q.o_occn = a.lds_occn_off; q.o_occ = a.lds_occ_off;
     q.o_sur = a.lds_sur_off;
+    {
+        EwaldTerms &x = sh.ewald;
+        const int nr = a.ewald_nreal, nf = a.ewald_ncodes - nr, nn = a.ewald.fc + 1;
+        const bool ok = a.ewald_ncodes > 0 && nr <= 64 && nf <= 128 && a.L > 1e-6 && a.L < 1e6;
+        for (int i = threadIdx.x; ok && i < 192; i += NT) {
+            const int t = i < 64 ? (i < nr ? i : -1) : (i - 64 < nf ? nr + i - 64 : -1), c = t >= 0 ? a.ewald_codes[t] : -1;
+            x.code[i >> 6][i & 63] = c;
+            if (i >= 64)
+                x.f[(i >> 6) - 1][i & 63] =
+                    c >= 0 ? (float)a.ewald.f[((((c >> 16) & 255) - 128) * nn + ((c >> 8) & 255) - 128) * nn + (c & 255) - 128] : 0.f;
+        }
+        if (threadIdx.x == 0) {
+            x.L = a.L;
+            x.inv_l = 1.0 / a.L;
+            x.aol = (float)a.ewald.aol;
+            x.aol2 = (float)a.ewald.aol2;
+            x.two_aol_rpi = (float)a.ewald.two_aol_rpi;
+            x.ok = ok;
+        }
+    }
     q.L = a.L; q.half = a.half; q.beta = a.beta;
     q.inv_beta = (float)(1.0 / a.beta) * (1.f - 0x1p-20f);
     q.nb_cells = a.nb_table ? 0 : a.nb_stride;
