@@ -609,6 +609,7 @@ struct HotList {
     uint32_t tags;          // 4 bits per pair tagger
     int32_t boundary, veto; // taggers, -1: none
     int32_t before;         // pair taggers created before the cell boundary
+    int32_t veto_before;    // and before the cell veto
     uint32_t mask;          // all of them
     uint32_t creators;      // bit t: tagger t creates this list
     uint32_t prefixed;      // bit t: tagger t creates other taggers, then this list
@@ -1899,7 +1900,7 @@ __device__ __forceinline__ HotList hot_list(const ChainShared<NT> &sh, uint64_t 
     l.items = -1;
     l.tags = l.mask = l.creators = l.prefixed = l.trashers = 0;
     l.boundary = l.veto = -1;
-    l.before = 0;
+    l.before = l.veto_before = 0;
     int first = 0;
     while (first < n_taggers && !pair_kind(kind_of(kinds, first))) first++;
     if (first == n_taggers) return l;
@@ -1916,8 +1917,9 @@ __device__ __forceinline__ HotList hot_list(const ChainShared<NT> &sh, uint64_t 
         } else if (kind == ECMC_TAG_CELL_BOUNDARY && l.boundary < 0) {
             l.boundary = t;
             l.before = items;
-        } else if (kind == ECMC_TAG_CELL_VETO && i == 0) {
+        } else if (kind == ECMC_TAG_CELL_VETO && l.veto < 0) {
             l.veto = t;
+            l.veto_before = items;
         } else {
             return l;
         }
@@ -2372,17 +2374,6 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
     };
     // ---- creates: the earliest event known before the pairs is S
     Pick S = stored;
-    if ((FM & FEAT_CELL_VETO) && hot.veto >= 0) {
-        create_cell_veto<D, NT, RES>(a, q, g, sh, hot.veto);
-        if (g.err) { g.err = 0; return general(); }
-        Pick v;
-        v.t.q = lane_d(g.lt.q, hot.veto);
-        v.t.r = lane_d(g.lt.r, hot.veto);
-        v.w = hot.veto;
-        if (S.w < 0 || ub(time_lt(v.t, S.t))) S = v;
-        else if (ub(time_eq(v.t, S.t))) return general();
-        lane_slot(g, hot.veto, v.t, 0, 0);   // its payload stays in LDS; only this leg may commit it
-    }
     Boundary B;
     B.p.w = -1;
     B.x = 0.0;
@@ -2395,10 +2386,9 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
     Counts cn;
     cn.nb = cn.far = -1;
     Items its = constants;
-    its.word = (uint32_t)(g.cursor - cursor0);
+    its.word = 0;
     its.rank = its.before = 0;
-    const int pre = (int)(g.seq - seq0) - (hot.boundary >= 0 ? 1 : 0);
-    uint32_t word = its.word;
+    uint32_t word = 0, veto_word = 0;
     int M0 = 0, ncand = 0;
 #pragma unroll
     for (int i = 0; i < HOT_ITEMS; i++) {
@@ -2407,15 +2397,33 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
         const int M = candidate_count<D, FM, NT, RES>(a, q, g, sh, t, kind_of(q.kinds, t), cn);
         if (i == 0) M0 = M;
         its.word = lane == i ? word : its.word;
-        its.rank = lane == i ? pre + ncand + (hot.boundary >= 0 && i >= hot.before ? 1 : 0) : its.rank;
+        its.rank = lane == i ? ncand + (hot.boundary >= 0 && i >= hot.before ? 1 : 0) : its.rank;
         its.before = lane == i ? ncand : its.before;
         if ((q.draws >> t) & 1u) word += 2u * (uint32_t)M;
         ncand += M;
+        if (i + 1 == hot.veto_before) veto_word = word;
+    }
+    if ((int)word + 512 + 2 * RING_STEP > q.ring_mask + 1) return general();   // more words than the ring holds
+    if ((FM & FEAT_CELL_VETO) && hot.veto >= 0) {
+        // the veto draws its words between the pair taggers' created before and after it
+        g.cursor = cursor0 + veto_word;
+        create_cell_veto<D, NT, RES>(a, q, g, sh, hot.veto);
+        if (g.err) { g.err = 0; return general(); }
+        const uint32_t took = (uint32_t)(g.cursor - cursor0) - veto_word;
+        word += took;
+        its.word += lane >= hot.veto_before ? took : 0u;
+        its.rank += lane >= hot.veto_before ? 1 : 0;
+        Pick v;
+        v.t.q = lane_d(g.lt.q, hot.veto);
+        v.t.r = lane_d(g.lt.r, hot.veto);
+        v.w = hot.veto;
+        if (S.w < 0 || ub(time_lt(v.t, S.t))) S = v;
+        else if (ub(time_eq(v.t, S.t))) return general();
+        lane_slot(g, hot.veto, v.t, 0, 0);   // its payload stays in LDS; only this leg may commit it
     }
     g.cursor = cursor0 + word;
     g.seq += ncand;
     g.ncand = ncand;
-    if ((int)word + 512 + 2 * RING_STEP > q.ring_mask + 1) return general();   // more words than the ring holds
     ring_ensure<RES, D, NT>(a, q, g, g.cursor);
     if (hashed) {
         g.chash = 0;
@@ -2569,6 +2577,7 @@ __device__ __forceinline__ void chain_body(const ChainArgs &a) {
     hot.boundary = uni(sh.hot.boundary);
     hot.veto = uni(sh.hot.veto);
     hot.before = uni(sh.hot.before);
+    hot.veto_before = uni(sh.hot.veto_before);
     hot.mask = (uint32_t)uni((int)sh.hot.mask);
     hot.creators = (uint32_t)uni((int)sh.hot.creators);
     hot.prefixed = (uint32_t)uni((int)sh.hot.prefixed);
