@@ -278,6 +278,7 @@ static void plan_lds(ecmc_system *s) {
     };
     place((size_t)s->dim * s->n * sizeof(double));
     a.lds_ring_off = place((size_t)s->ring_words * sizeof(uint32_t));
+    a.lds_tg_off = place((size_t)s->desc.n_taggers * sizeof(ecmc_tagger_desc));
     if (charged) a.lds_charge_off = place((size_t)s->n * sizeof(double));
     if (a.occupancy) {
         a.lds_occn_off = place((size_t)s->ncells * sizeof(int32_t));

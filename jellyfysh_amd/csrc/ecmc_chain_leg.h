@@ -39,6 +39,11 @@ static_assert(ECMC_MAX_TAGGERS == 16, "the stored events are selected over one 1
 
 // The dynamic LDS of a leg-loop launch: a resident system's state (ChainArgs::lds_*_off).
 extern __shared__ __align__(16) unsigned char chain_dyn_lds[];
+// The taggers of a launch without it.
+__device__ __forceinline__ ecmc_tagger_desc *static_taggers() {
+    __shared__ ecmc_tagger_desc tg[ECMC_MAX_TAGGERS];
+    return tg;
+}
 
 constexpr uint32_t MT_UPPER = 0x80000000u, MT_LOWER = 0x7fffffffu, MT_MATRIX = 0x9908b0dfu;
 
@@ -128,7 +133,7 @@ struct ChainArgs {
     // and surplus lists live in the launch's dynamic LDS at these offsets, copied in at the start of
     // a launch and back at its end, and so do the first occ_cols occupants of every cell (16-bit);
     // 0 keeps everything in global memory
-    int32_t resident, lds_ring_off, lds_charge_off, lds_occ_off, lds_occn_off, lds_sur_off, occ_cols;
+    int32_t resident, lds_ring_off, lds_charge_off, lds_occ_off, lds_occn_off, lds_sur_off, lds_tg_off, occ_cols;
     int32_t ewald_ncodes, ewald_nreal;
     // the terms of the merged-image Coulomb derivative in the sequential loop's order (real-space
     // images by k, j, i, then Fourier terms by i, j, k): kind << 24 | (i + 128) << 16 |
@@ -166,6 +171,7 @@ __device__ __forceinline__ void wave_sync() {
 template <int D>
 struct Geo {
     unsigned char *dyn;        // the launch's dynamic LDS
+    ecmc_tagger_desc *tg;      // the taggers, in LDS (a resident system's beside its state, as many as it has)
     int n, ncells, occ_cols, occ_cap, ring_mask, leaves, max_occ, o_ring, o_charge, o_occn, o_occ, o_sur;
     float inv_beta;            // 1 / beta rounded down
     double L, half, beta;
@@ -176,6 +182,7 @@ struct Geo {
     int nb_cells;              // nearby cells (0: read from the table)
     uint64_t kinds;            // 4 bits per tagger: its kind
     uint32_t tests;            // 2 bits per tagger: its quick test
+    uint32_t inversions;       // 2 bits per tagger: 0 an inverse power inverted, 1 the Coulomb bound, 2 a rate or another potential
     uint32_t draws, charged;   // 1 bit per tagger
 };
 __device__ __forceinline__ int kind_of(uint64_t kinds, int t) { return (int)((kinds >> (4 * t)) & 15u); }
@@ -293,9 +300,58 @@ __device__ __forceinline__ void ring_make(uint32_t *ring, uint32_t mask, uint64_
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // the next step reads these words from other lanes
     }
 }
+// The same in LDS, where a wavefront's operations are in order: nothing waits for a step's writes, the
+// words 624 and 623 back of the next step (older than this step's) are read while this one waits
+// for its words 227 back, and the mask is left out where none of the four runs wraps.  570 -> 330
+// cycles a step.
+__device__ __forceinline__ void ring_make_lds(uint32_t *ring, uint32_t mask, uint64_t from, int steps) {
+    constexpr int U = RING_STEP / 64;
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t at = (uint32_t)uni((int)(uint32_t)from);
+    uint32_t x[U], y[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        x[u] = ring[(at + lane + 64u * u - 624u) & mask];
+        y[u] = ring[(at + lane + 64u * u - 623u) & mask];
+    }
+#pragma unroll 1
+    for (int s = 0; s < steps; s++, at += RING_STEP) {
+        uint32_t z[U], nx[U], ny[U];
+        const uint32_t o = at & mask, r = (at - 227u) & mask, n = (at + RING_STEP - 624u) & mask;
+        const bool wraps = max(max(o, r), n) + RING_STEP + 1u > mask + 1u;   // (uniform)
+        if (!wraps) {
+            const uint32_t *const pr = ring + r + lane, *const pn = ring + n + lane;
+#pragma unroll
+            for (int u = 0; u < U; u++) z[u] = pr[64 * u];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                nx[u] = pn[64 * u];
+                ny[u] = pn[64 * u + 1];
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                z[u] = ring[(r + lane + 64u * u) & mask];
+                nx[u] = ring[(n + lane + 64u * u) & mask];
+                ny[u] = ring[(n + lane + 64u * u + 1u) & mask];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) z[u] = mt_next(x[u], y[u], z[u]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (!wraps) ring[o + lane + 64u * u] = z[u];
+            else ring[(o + lane + 64u * u) & mask] = z[u];
+            x[u] = nx[u];
+            y[u] = ny[u];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the next step reads these words from other lanes
+    }
+}
 template <bool RES, int D>
 __device__ __forceinline__ void ring_make(const ChainArgs &a, const Geo<D> &q, uint64_t from, int steps) {
-    if (RES) ring_make(reinterpret_cast<uint32_t *>(q.dyn + q.o_ring), (uint32_t)q.ring_mask, from, steps);
+    if (RES) ring_make_lds(reinterpret_cast<uint32_t *>(q.dyn + q.o_ring), (uint32_t)q.ring_mask, from, steps);
     else ring_make(a.ring, (uint32_t)q.ring_mask, from, steps);
 }
 // Word `off` after the leg's first word `keep` (32-bit: the ring's mask drops the rest).
@@ -431,8 +487,22 @@ constexpr int VARIANT_DIPOLES = (1 << ECMC_POT_INVERSE_POWER) | (1 << ECMC_POT_D
 // run two paths: the same operations on the same values.  urc = U(rc) and rc2 = rc^2 of the
 // truncated form, 0 and +inf without a cutoff (then current >= urc is the reference's test
 // against zero).
-template <int D>
-__device__ __forceinline__ double ip_time(int dir, double speed, const double *sep, double pp, double power, double rc2,
+//
+// SettledPowers takes the powers through the fast paths alone, without a branch or a call between
+// them (ok turns false where they do not settle a rounding, about one time in 10^4): the two
+// powers, the logarithm of the draw and the root's parts then overlap in one instruction stream.
+// 6300 -> 3900 cycles for the contenders of a Lennard-Jones leg.
+struct AnyPowers {
+    __device__ __forceinline__ double half(double r2, double power) { return pow_half_power(r2, power); }
+    __device__ __forceinline__ double root(double x, double power) { return root_two_over_power(x, power); }
+};
+struct SettledPowers {   // powers 6 and 12
+    bool ok = true;
+    __device__ __forceinline__ double half(double r2, double power) { return pow36_settled(r2, power == 12.0, ok); }
+    __device__ __forceinline__ double root(double x, double power) { return root36_settled(x, power == 12.0, ok); }
+};
+template <int D, class Powers>
+__device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, const double *sep, double pp, double power, double rc2,
                                           double urc, double dU) {
     const bool rep = pp > 0.0;
     const double perp2 = others_sq<D>(sep, dir);
@@ -444,10 +514,10 @@ __device__ __forceinline__ double ip_time(int dir, double speed, const double *s
     for (int d = 0; d < D; d++) c[d] = d == dir ? sdd : sep[d];
     const double sn2 = norm_sq<D>(c);
     bool live = perp2 < rc2 && (rep ? sd > 0.0 : sn2 < rc2);
-    const double cur = (rep && !(sn2 < rc2)) ? urc : pp / pow_half_power(live ? sn2 : 1.0, power);
-    const double maxp = pp / pow_half_power(rep && live ? perp2 : 1.0, power);
+    const double cur = (rep && !(sn2 < rc2)) ? urc : pp / m.half(live ? sn2 : 1.0, power);
+    const double maxp = pp / m.half(rep && live ? perp2 : 1.0, power);
     live = live && (rep ? dU < maxp - cur : !(cur + dU >= urc));
-    const double nsq = root_two_over_power(live ? pp / (cur + dU) : 1.0, power);
+    const double nsq = m.root(live ? pp / (cur + dU) : 1.0, power);
     const double a = nsq - perp2;
     const double sq = sqrt(fmax(a, 0.0));
     const double res = a < 0.0 ? NAN : (rep ? sdd - sq : disp + (sdd + sq)) / speed;
@@ -469,12 +539,21 @@ __device__ __noinline__ static double pair_time(int how, double p0, double p1, d
     s[0] = s0;
     s[1] = s1;
     if (D > 2) s[D - 1] = s2;
+    if ((FM & FEAT_IP) && (how == ECMC_POT_INVERSE_POWER || how == ECMC_POT_INVERSE_POWER_TRUNC) && (p0 == 12.0 || p0 == 6.0)) {
+        const bool trunc = how == ECMC_POT_INVERSE_POWER_TRUNC;
+        const double pp = (c1 * c2) * p1;
+        SettledPowers m;
+        const double change = -log_settled(1.0 - words_to_random(w0, w1), m.ok) / beta;
+        const double dt = ip_time<D>(m, dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, change);
+        if (m.ok) return dt;
+    }
     // hard potentials draw nothing (beta = 0 marks them)
     const double dU = beta != 0.0 ? -cr_log(1.0 - words_to_random(w0, w1)) / beta : 0.0;
     if ((FM & FEAT_IP) && (how == ECMC_POT_INVERSE_POWER || how == ECMC_POT_INVERSE_POWER_TRUNC)) {
         const bool trunc = how == ECMC_POT_INVERSE_POWER_TRUNC;
         const double pp = (c1 * c2) * p1;
-        return ip_time<D>(dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, dU);
+        AnyPowers m;
+        return ip_time<D>(m, dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, dU);
     }
     if ((FM & FEAT_COULOMB) && how == TIME_COULOMB_BOUND) {
         // two_leaf_unit_bounding_potential_event_handler.py:138-143 with the Coulomb bound
@@ -635,7 +714,6 @@ struct ChainShared {
     static constexpr int NW = NT / 64;
     Slot slot[ECMC_MAX_TAGGERS];             // payloads of the stored events, written by thread 0
     SlotTime time[NW][ECMC_MAX_TAGGERS];     // their times as every wavefront sees them, around a rare step
-    ecmc_tagger_desc tg[ECMC_MAX_TAGGERS];
     TaggerPlan plan[ECMC_MAX_TAGGERS];
     Contender queue[NW][QCAP];
     Winner win[NW];
@@ -705,6 +783,7 @@ __device__ __forceinline__ void nearby_offsets(const ChainArgs &a, Geo<D> &q) {
 template <int D>
 __device__ __forceinline__ void geo_load(const Geo<3> &m, const ChainArgs &a, Geo<D> &q) {
     q.dyn = reinterpret_cast<unsigned char *>(uni((uint64_t)m.dyn));
+    q.tg = reinterpret_cast<ecmc_tagger_desc *>(uni((uint64_t)m.tg));
     q.n = uni(m.n); q.ncells = uni(m.ncells); q.occ_cols = uni(m.occ_cols); q.occ_cap = uni(m.occ_cap);
     q.ring_mask = uni(m.ring_mask); q.leaves = uni(m.leaves); q.max_occ = uni(m.max_occ);
     q.o_ring = uni(m.o_ring); q.o_charge = uni(m.o_charge); q.o_occn = uni(m.o_occn); q.o_occ = uni(m.o_occ); q.o_sur = uni(m.o_sur);
@@ -715,6 +794,7 @@ __device__ __forceinline__ void geo_load(const Geo<3> &m, const ChainArgs &a, Ge
         q.cps[d] = uni(m.cps[d]); q.cum[d] = uni(m.cum[d]);
     }
     q.nb_cells = uni(m.nb_cells); q.kinds = uni(m.kinds); q.tests = (uint32_t)uni((int)m.tests);
+    q.inversions = (uint32_t)uni((int)m.inversions);
     q.draws = (uint32_t)uni((int)m.draws); q.charged = (uint32_t)uni((int)m.charged);
     nearby_offsets<D>(a, q);
 }
@@ -1041,7 +1121,7 @@ template <int D, int FM, int NT, bool RES>
 __device__ __forceinline__ int candidate_count(const ChainArgs &a, const Geo<D> &q, const Leg<D> &g, ChainShared<NT> &sh, int t,
                                                int kind, Counts &n) {
     if (g.active < 0) return 0;
-    if ((FM & FEAT_FMAP) && kind == ECMC_TAG_FACTOR_MAP) return uni(fmap_count(sh.tg[t], q.leaves, q.n, g.active));
+    if ((FM & FEAT_FMAP) && kind == ECMC_TAG_FACTOR_MAP) return uni(fmap_count(q.tg[t], q.leaves, q.n, g.active));
     if (kind == ECMC_TAG_PAIR_ALL) return q.n - 1;
     if (kind == ECMC_TAG_SURPLUS) return g.nsur;
     if ((FM & FEAT_CELL_BOUNDING) && kind == ECMC_TAG_CELL_BOUNDING) {
@@ -1067,7 +1147,7 @@ struct Candidates {
     int kind, act, wave, M, m, k, fn, first;
     __device__ __forceinline__ Candidates(const ChainArgs &a_, const Geo<D> &q_, ChainShared<NT> &s_, int t, int kind_, int act_, int M_,
                                           const Counts &n_)
-        : a(a_), q(q_), sh(s_), tg(s_.tg[t]), n(n_), kind(kind_), act(act_), wave(wave_index<NT>()), M(M_), m(0), k(0), fn(1), first(0) {
+        : a(a_), q(q_), sh(s_), tg(q_.tg[t]), n(n_), kind(kind_), act(act_), wave(wave_index<NT>()), M(M_), m(0), k(0), fn(1), first(0) {
         if ((FM & FEAT_FMAP) && kind == ECMC_TAG_FACTOR_MAP) {
             m = act / q.leaves;
             k = act % q.leaves;
@@ -1291,7 +1371,7 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
 template <int D, int FM, int NT, bool RES>
 __device__ __forceinline__ double candidate_dt(const ChainArgs &a, const Geo<D> &q, const Leg<D> &g, ChainShared<NT> &sh, int tag,
                                                uint32_t word, int target, int cell) {
-    const ecmc_tagger_desc &tg = sh.tg[tag];
+    const ecmc_tagger_desc &tg = q.tg[tag];
     double tp[D], s[D];
     load_pos<RES>(a, q, target, tp);
     separation_vector<D>(q, g.ap, tp, s);
@@ -1437,7 +1517,7 @@ __device__ __forceinline__ void store_boundary(Leg<D> &g, ChainShared<NT> &sh, c
 // composite objects the root's randint, then the leaf's.
 template <int D, int NT, bool RES>
 __device__ __forceinline__ void create_end_of_chain(const ChainArgs &a, const Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh, int t) {
-    const double value = sh.tg[t].value;
+    const double value = q.tg[t].value;
     const double since = time_sub(g.at, g.eoc_last);
     if (ub(!(0.0 <= since && since <= value))) { g.err = ECMC_ERR_CONFIGURATION; return; }
     const double chain = time_sub(g.eoc_last, g.at) + value;
@@ -1471,7 +1551,7 @@ __device__ __forceinline__ void create_end_of_chain(const ChainArgs &a, const Ge
 // words), uniform(0, mean) for item or alias, then expovariate / (total rate * speed).
 template <int D, int NT, bool RES>
 __device__ __forceinline__ void create_cell_veto(const ChainArgs &a, const Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh, int t) {
-    const ecmc_tagger_desc &tg = sh.tg[t];
+    const ecmc_tagger_desc &tg = q.tg[t];
     const int dir = g.adir;
     double cf = (((q.charged >> t) & 1u) ? charge_of<RES>(a, q, g.active) : 1.0) * 1.0 / tg.bpar[2];
     const int b = ub(!(cf > 0.0)) ? 1 : 0;
@@ -1532,7 +1612,7 @@ __device__ __forceinline__ void create_cell_veto(const ChainArgs &a, const Geo<D
 // Creates of one tagger other than the pair and cell-boundary taggers (collective for the words).
 template <int D, int FM, int NT, bool RES>
 __device__ __forceinline__ void create_single(const ChainArgs &a, const Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh, int t, int kind) {
-    const ecmc_tagger_desc &tg = sh.tg[t];
+    const ecmc_tagger_desc &tg = q.tg[t];
     Time time = {0.0, 0.0};
     if (kind == ECMC_TAG_END_OF_CHAIN || kind == ECMC_TAG_CELL_VETO) {
         lane_slot(g, t, time, 0, 0);
@@ -1778,7 +1858,7 @@ __device__ __forceinline__ void commit_event(const ChainArgs &a, const Geo<D> &q
         if (target >= 0) separation_vector_u<D>(q, e.apos, tp, s);
         bool lift = true, thins = false;
         if (FM & FEAT_EWALD) {
-            const ecmc_tagger_desc &T = sh.tg[e.tagger];
+            const ecmc_tagger_desc &T = q.tg[e.tagger];
             const int eh = uni(T.event_handler);
             thins = veto || eh == ECMC_EH_CELL_BOUNDING || eh == ECMC_EH_TWO_LEAF_BOUNDING;
             if (thins) {
@@ -1852,7 +1932,7 @@ __device__ __forceinline__ void commit_event(const ChainArgs &a, const Geo<D> &q
             g.at = e.t;
             add_est(sh, 3, 1.0);
         } else if (kind == ECMC_TAG_START_OF_RUN) {
-            const ecmc_tagger_desc &T = sh.tg[e.tagger];
+            const ecmc_tagger_desc &T = q.tg[e.tagger];
             next = uni(T.ivalue2);
             g.adir = uni(T.ivalue);
             g.aspeed = T.value;
@@ -1870,7 +1950,7 @@ __device__ __forceinline__ void commit_event(const ChainArgs &a, const Geo<D> &q
             if (kind == ECMC_TAG_END_OF_CHAIN) {
                 g.eoc_last = e.t;
                 ev.target = e.target;
-                add_est(sh, 1, sh.tg[e.tagger].value * g.aspeed);
+                add_est(sh, 1, q.tg[e.tagger].value * g.aspeed);
                 add_est(sh, 5, 1.0);
                 g.adir = g.adir + 1 == D ? 0 : g.adir + 1;
                 if (e.target != act) ev.flags |= 1;
@@ -1949,6 +2029,7 @@ template <int D, int NT, bool RES>
 __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh) {
     const int tid = threadIdx.x, lane = tid & 63;
     q.dyn = chain_dyn_lds;
+    q.tg = RES ? reinterpret_cast<ecmc_tagger_desc *>(chain_dyn_lds + a.lds_tg_off) : static_taggers();
     q.n = a.n; q.ncells = a.ncells; q.occ_cols = a.occ_cols; q.occ_cap = a.occ_cap; q.ring_mask = a.ring_words - 1;
     q.leaves = a.leaves; q.max_occ = a.max_occ;
     q.o_ring = a.lds_ring_off; q.o_charge = a.lds_charge_off; q.o_occn = a.lds_occn_off; q.o_occ = a.lds_occ_off;
@@ -2021,7 +2102,7 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
     }
     {
         const uint32_t *src = reinterpret_cast<const uint32_t *>(a.tg);
-        uint32_t *dst = reinterpret_cast<uint32_t *>(sh.tg);
+        uint32_t *dst = reinterpret_cast<uint32_t *>(q.tg);
         for (int i = tid; i < (int)(sizeof(ecmc_tagger_desc) / 4) * a.n_taggers; i += NT) dst[i] = src[i];
         const uint32_t *ss = reinterpret_cast<const uint32_t *>(s.slot);
         const int words = (int)sizeof(Slot) / 4 * ECMC_MAX_TAGGERS;
@@ -2042,9 +2123,9 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
         sh.occupied[tid] = w;
     }
     // every wavefront derives the bit fields of its own; wavefront 0 writes the plans
-    int kind = 0, test = QT_DIRECT, draws = 0, charged = 0;
+    int kind = 0, test = QT_DIRECT, draws = 0, charged = 0, inversion = 0;
     if (lane < a.n_taggers) {
-        const ecmc_tagger_desc &tg = sh.tg[lane];
+        const ecmc_tagger_desc &tg = q.tg[lane];
         kind = tg.kind;
         draws = pair_kind(kind) && pot_draws(tg);
         charged = tg.use_charge != 0;
@@ -2059,6 +2140,10 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
         pl.powrc = 1.0;
         pl.set_key = 16 + lane;
         if (pair_kind(kind)) {
+            inversion = tg.event_handler == ECMC_EH_TWO_LEAF_BOUNDING                                                          ? 1
+                        : tg.event_handler == ECMC_EH_CELL_BOUNDING                                                            ? 2
+                        : tg.potential == ECMC_POT_INVERSE_POWER || tg.potential == ECMC_POT_INVERSE_POWER_TRUNC               ? 0
+                                                                                                                               : 2;
             if (tg.event_handler == ECMC_EH_TWO_LEAF_BOUNDING) test = QT_COULOMB_BOUND;
             else if (tg.event_handler == ECMC_EH_CELL_BOUNDING) test = QT_CELL;
             else if (tg.potential == ECMC_POT_INVERSE_POWER || tg.potential == ECMC_POT_INVERSE_POWER_TRUNC) {
@@ -2076,7 +2161,7 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
                 // the first tagger with the same map stands for all of them
                 pl.set_key = 16 + lane;
                 for (int o = lane - 1; o >= 0; o--) {
-                    const ecmc_tagger_desc &og = sh.tg[o];
+                    const ecmc_tagger_desc &og = q.tg[o];
                     bool same = og.kind == ECMC_TAG_FACTOR_MAP && og.fmap_local == tg.fmap_local;
                     for (int k = 0; same && k < ECMC_MAX_LEAVES; k++) {
                         same = og.fmap_n[k] == tg.fmap_n[k];
@@ -2089,11 +2174,12 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
         if (tid < 64) sh.plan[lane] = pl;
     }
     q.kinds = 0;
-    q.tests = q.draws = q.charged = 0;
+    q.tests = q.draws = q.charged = q.inversions = 0;
 #pragma unroll
     for (int t = 0; t < ECMC_MAX_TAGGERS; t++) {
         q.kinds |= (uint64_t)(uint32_t)__builtin_amdgcn_readlane(kind, t) << (4 * t);
         q.tests |= (uint32_t)__builtin_amdgcn_readlane(test, t) << (2 * t);
+        q.inversions |= (uint32_t)__builtin_amdgcn_readlane(inversion, t) << (2 * t);
     }
     q.draws = (uint32_t)__ballot(draws) & 0xffffu;
     q.charged = (uint32_t)__ballot(charged) & 0xffffu;
@@ -2101,13 +2187,14 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
     if (tid == 0) {
         Geo<3> &m = sh.geo;
         m.dyn = q.dyn;
+        m.tg = q.tg;
         m.n = q.n; m.ncells = q.ncells; m.occ_cols = q.occ_cols; m.occ_cap = q.occ_cap; m.ring_mask = q.ring_mask;
         m.leaves = q.leaves; m.max_occ = q.max_occ;
         m.o_ring = q.o_ring; m.o_charge = q.o_charge; m.o_occn = q.o_occn; m.o_occ = q.o_occ; m.o_sur = q.o_sur;
         m.L = q.L; m.half = q.half; m.beta = q.beta; m.inv_beta = q.inv_beta;
 #pragma unroll
         for (int d = 0; d < D; d++) { m.side[d] = q.side[d]; m.inv[d] = q.inv[d]; m.cps[d] = q.cps[d]; m.cum[d] = q.cum[d]; }
-        m.nb_cells = q.nb_cells; m.kinds = q.kinds; m.tests = q.tests; m.draws = q.draws; m.charged = q.charged;
+        m.nb_cells = q.nb_cells; m.kinds = q.kinds; m.tests = q.tests; m.inversions = q.inversions; m.draws = q.draws; m.charged = q.charged;
         sh.hot = hot_list<NT>(sh, q.kinds, a.n_taggers);
     }
     __syncthreads();
@@ -2480,7 +2567,11 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
         }
         Winner m = no_winner();
         const int workers = NW > 1 && !direct ? NW - 1 : NW;
-        int b = direct ? wave * 64 : (NW > 1 ? (wave == 0 ? 0 : (wave == maker ? total : (wave - 1) * 64)) : 0);
+        // few contenders: each kind of inversion on a wavefront of its own, so that they run side by
+        // side and not one after the other in one wavefront
+        const bool by_kind = NW > 1 && !direct && total <= 64;
+        const int kind_here = wave == 0 ? 0 : wave - 1;
+        int b = by_kind ? (wave == maker ? total : 0) : direct ? wave * 64 : (NW > 1 ? (wave == 0 ? 0 : (wave == maker ? total : (wave - 1) * 64)) : 0);
         const int count = direct ? M0 : total;
         Candidates<D, FM, NT, RES> cs(a, q, sh, tag0, kind_of(q.kinds, tag0), g.active, M0, cn);
         const uint32_t word0 = item_word(its, 0);
@@ -2488,7 +2579,13 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
 #pragma unroll 1
         for (; b < count; b += workers * 64) {
             const int idx = b + lane;
-            if (idx < count) {
+            bool here = idx < count;
+            if (by_kind && here) {
+                const bool b0 = idx >= q0, b1 = idx >= q0 + q1, b2 = idx >= q0 + q1 + q2;
+                const int w = (int)b0 + (int)b1 + (int)b2, k = idx - (b2 ? q0 + q1 + q2 : (b1 ? q0 + q1 : (b0 ? q0 : 0)));
+                here = (int)((q.inversions >> (2 * (sh.queue[w][k].tag_cell & 15))) & 3u) == kind_here;
+            }
+            if (here) {
                 Contender c;
                 if (direct) {
                     int j, cell;
@@ -2589,7 +2686,7 @@ __device__ __forceinline__ void chain_body(const ChainArgs &a) {
     its.rank = its.before = 0;
     {
         const int i = min((int)(threadIdx.x & 63), HOT_ITEMS - 1), t = item_tag(its, i);
-        const ecmc_tagger_desc &tg = sh.tg[t];
+        const ecmc_tagger_desc &tg = q.tg[t];
         const int test = (q.tests >> (2 * t)) & 3;
         its.p = sh.plan[t].p;
         its.rc2_hi = sh.plan[t].rc2_hi;

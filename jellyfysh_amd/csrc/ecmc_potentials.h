@@ -383,37 +383,26 @@ ECMC_FN double ipcb_displacement(double pp, double sx, double sy, double sz, dou
     double cur = ipcb_potential(pp, sx, sy, sz);
     double p0 = ipcb_potential(pp, 0.0, sy, sz);
     double ph = ipcb_potential(pp, half, sy, sz);
-    double per = fabs(p0 - ph);
+    const double per = fabs(p0 - ph);
     double disp = floor(dU / per) * L;
     dU = fmod_near(dU, per);
-    double nn;
-    if (pp > 0.0) {
-        if (sx <= 0.0) {
-            disp += half + sx;
-            sx = half;
-            cur = ph;
-        } else if (dU >= p0 - cur) {
-            dU -= (p0 - cur);
-            disp += sx + half;
-            sx = half;
-            cur = ph;
-        }
-        nn = pp / (cur + dU);
-        disp += (sx - sqrt(nn * nn - (sy * sy + sz * sz)));
-    } else {
-        if (sx > 0.0) {
-            disp += sx;
-            sx = 0.0;
-            cur = p0;
-        } else if (dU >= ph - cur) {
-            dU -= (ph - cur);
-            disp += sx + L;
-            sx = 0.0;
-            cur = p0;
-        }
-        nn = pp / (cur + dU);
-        disp += (sx + sqrt(nn * nn - (sy * sy + sz * sz)));
+    // the remainder of one period, repulsive and attractive as one instruction stream: first to the
+    // far side (half a box ahead) or past the closest approach where the energy does not rise before
+    // it or the draw reaches over the maximum
+    const bool rep = pp > 0.0;
+    const double gap = (rep ? p0 : ph) - cur;
+    const bool flat = rep ? sx <= 0.0 : sx > 0.0;
+    const bool over = !flat && dU >= gap;
+    if (over) dU -= gap;
+    const double step = rep ? sx + half : (flat ? sx : sx + L);
+    if (flat || over) {
+        disp += step;
+        sx = rep ? half : 0.0;
+        cur = rep ? ph : p0;
     }
+    const double nn = pp / (cur + dU);
+    const double root = sqrt(nn * nn - (sy * sy + sz * sz));
+    disp += rep ? sx - root : sx + root;
     return disp;
 }
 
