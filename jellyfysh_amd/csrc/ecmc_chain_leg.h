@@ -203,6 +203,26 @@ __device__ __forceinline__ int32_t occ_get(const ChainArgs &a, const Geo<D> &q, 
     if (RES && k < q.occ_cols) return reinterpret_cast<uint16_t *>(q.dyn + q.o_occ)[c * q.occ_cols + k];
     return a.occ[(size_t)c * q.occ_cap + k];
 }
+// Occupants place[u] of cells c[u]: the LDS reads together, memory only where some lane needs it.
+template <bool RES, int U, int D>
+__device__ __forceinline__ void occ_get_all(const ChainArgs &a, const Geo<D> &q, const int (&c)[U], const int (&place)[U], int (&v)[U]) {
+    if (RES && q.occ_cols > 0) {
+        const uint16_t *const lo = reinterpret_cast<const uint16_t *>(q.dyn + q.o_occ);
+        bool beyond = false;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            v[u] = lo[c[u] * q.occ_cols + min(place[u], q.occ_cols - 1)];
+            beyond |= place[u] >= q.occ_cols;
+        }
+        if (!ub(beyond)) return;
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (place[u] >= q.occ_cols) v[u] = a.occ[(size_t)c[u] * q.occ_cap + place[u]];
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = a.occ[(size_t)c[u] * q.occ_cap + place[u]];
+    }
+}
 template <bool RES, int D>
 __device__ __forceinline__ void occ_set(const ChainArgs &a, const Geo<D> &q, int c, int k, int32_t v) {
     if (RES && k < q.occ_cols) reinterpret_cast<uint16_t *>(q.dyn + q.o_occ)[c * q.occ_cols + k] = (uint16_t)v;
@@ -1156,33 +1176,68 @@ struct Candidates {
     }
     __device__ __forceinline__ bool far() const { return (FM & FEAT_CELL_BOUNDING) && kind == ECMC_TAG_CELL_BOUNDING; }
     __device__ __forceinline__ int span() const { return far() ? min(q.ncells - first, FAR_BLOCK) : M; }
-    __device__ __forceinline__ bool get(int idx, int &j, int &target, int &cell) const {
-        j = idx;
-        cell = 0;
-        if (far()) {
-            const uint32_t w = sh.far_word[wave][idx >> 5], bit = 1u << (idx & 31);
-            j = (int)sh.far_pref[wave][idx >> 5] + __popc(w & (bit - 1u));
-            cell = first + idx;
-            const bool live = (w & bit) != 0;
-            target = live ? occ_get<RES>(a, q, cell, 0) : act;
-            return live;
+    // U indices at once, so that their loads overlap (one branch on the kind for all of them).
+    template <int U>
+    __device__ __forceinline__ void get(const int (&idx)[U], int (&j)[U], int (&target)[U], int (&cell)[U], bool (&live)[U]) const {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            j[u] = idx[u];
+            cell[u] = 0;
+            live[u] = true;
         }
-        if ((FM & FEAT_FMAP) && kind == ECMC_TAG_FACTOR_MAP) target = fmap_target(tg, q.leaves, m, k, fn, idx);
-        else if (kind == ECMC_TAG_PAIR_ALL) target = idx < act ? idx : idx + 1;
-        else if (kind == ECMC_TAG_SURPLUS) target = sur_id<RES>(a, q, idx);
-        else {
+        if (far()) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const uint32_t w = sh.far_word[wave][idx[u] >> 5], bit = 1u << (idx[u] & 31);
+                j[u] = (int)sh.far_pref[wave][idx[u] >> 5] + __popc(w & (bit - 1u));
+                cell[u] = first + idx[u];
+                live[u] = (w & bit) != 0;
+            }
+            int zero[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) zero[u] = 0;
+            occ_get_all<RES, U>(a, q, cell, zero, target);
+#pragma unroll
+            for (int u = 0; u < U; u++) target[u] = live[u] ? target[u] : act;
+        } else if ((FM & FEAT_FMAP) && kind == ECMC_TAG_FACTOR_MAP) {
+#pragma unroll
+            for (int u = 0; u < U; u++) target[u] = fmap_target(tg, q.leaves, m, k, fn, idx[u]);
+        } else if (kind == ECMC_TAG_PAIR_ALL) {
+#pragma unroll
+            for (int u = 0; u < U; u++) target[u] = idx[u] < act ? idx[u] : idx[u] + 1;
+        } else if (kind == ECMC_TAG_SURPLUS) {
+#pragma unroll
+            for (int u = 0; u < U; u++) target[u] = sur_id<RES>(a, q, idx[u]);
+        } else {
             // the nearby cell holding candidate idx: the largest c with pref[c] <= idx (empty cells
             // repeat a prefix, and so do the places after the last cell)
-            int k4 = 0;
+            int4 p[U], c[U];
 #pragma unroll
-            for (int i = 0; i < 7; i++) k4 += n.group[i] <= idx ? 1 : 0;
-            const int4 p = *reinterpret_cast<const int4 *>(&sh.nb_pref[wave][4 * k4]);
-            const int4 c = *reinterpret_cast<const int4 *>(&sh.nb_cell[wave][4 * k4]);
-            const bool b1 = p.y <= idx, b2 = p.z <= idx, b3 = p.w <= idx;
-            const int at = b3 ? p.w : (b2 ? p.z : (b1 ? p.y : p.x)), in = b3 ? c.w : (b2 ? c.z : (b1 ? c.y : c.x));
-            target = occ_get<RES>(a, q, in, idx - at);
+            for (int u = 0; u < U; u++) {
+                int k4 = 0;
+#pragma unroll
+                for (int i = 0; i < 7; i++) k4 += n.group[i] <= idx[u] ? 1 : 0;
+                p[u] = *reinterpret_cast<const int4 *>(&sh.nb_pref[wave][4 * k4]);
+                c[u] = *reinterpret_cast<const int4 *>(&sh.nb_cell[wave][4 * k4]);
+            }
+            int in[U], place[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool b1 = p[u].y <= idx[u], b2 = p[u].z <= idx[u], b3 = p[u].w <= idx[u];
+                place[u] = idx[u] - (b3 ? p[u].w : (b2 ? p[u].z : (b1 ? p[u].y : p[u].x)));
+                in[u] = b3 ? c[u].w : (b2 ? c[u].z : (b1 ? c[u].y : c[u].x));
+            }
+            occ_get_all<RES, U>(a, q, in, place, target);
         }
-        return true;
+    }
+    __device__ __forceinline__ bool get(int idx, int &j, int &target, int &cell) const {
+        int ii[1] = {idx}, jj[1], tt[1], cc[1];
+        bool ll[1];
+        get<1>(ii, jj, tt, cc, ll);
+        j = jj[0];
+        target = tt[0];
+        cell = cc[0];
+        return ll[0];
     }
 };
 
@@ -1196,15 +1251,16 @@ struct Candidates {
 // the cutoff sphere.  FP32 rounding (a few 2^-24 per operation, at most 20 of them) lies far
 // inside the 2^-15 margins; hf is the horizon widened by 2^-16 relative and 2^-18 L, which covers
 // the rounding of the exact inversion (a root near the closest approach is off by up to
-// 2^-26 of the separation).  perp2: squared perpendicular separation, rounded down; sd: the
-// component along the motion; edge: the sign of sd is not certain (at +-L / 2).
+// 2^-26 of the separation).  perp2: squared perpendicular separation, from below; sd: the component
+// along the motion to 2^-23 L, which the slacks cover; behind: surely negative; edge: the sign of sd
+// is not certain (at +-L / 2).
 __device__ __forceinline__ bool quick_cull(int test, int p, float rc2_hi, float pp, float perp2, float sd, bool behind, bool edge,
                                            float hf, float L, float dU_lo) {
     const float K = fabsf(pp);
     const bool sure = (K >= 0x1p-100f) & (K <= 0x1p100f) & !edge;
     bool none;
     if (test == QT_INVERSE_POWER) {
-        const float slack = (fabsf(sd) + hf) * 0x1p-17f;
+        const float slack = (fabsf(sd) + hf) * 0x1p-17f + L * 0x1p-20f;
         const float e = fmaxf(fmaxf(sd - hf, -sd) - slack, 0.f);
         const float r2 = (perp2 + e * e) * (1.f - 0x1p-16f);
         none = pp > 0.f ? behind : sd - slack > hf;
@@ -1251,7 +1307,7 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
     const float Lf = (float)q.L;
     const float hf = (float)(h * g.aspeed) * (1.f + 0x1p-16f) + Lf * 0x1p-18f;
     const float ibf = q.inv_beta;
-    const double edge_at = q.half * (1.0 - 0x1p-40), behind_at = -q.L * 0x1p-40;
+    const float inv_L = __builtin_amdgcn_rcpf(Lf);
     const int act = g.active, dir = g.adir;
     const float caf = (FM & FEAT_EWALD) && q.charged ? (float)charge_of<RES>(a, q, act) : 1.f;
     float cell_rate_max = 0.f;
@@ -1279,10 +1335,13 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
                 int j[U], target[U], cell[U];
                 bool live[U], edge[U], behind[U];
                 float perp2[U], sd[U];
+                int idx[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) idx[u] = min(base + u * NT + lane, span - 1);
+                cs.template get<U>(idx, j, target, cell, live);
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const int idx = base + u * NT + lane;
-                    live[u] = cs.get(min(idx, span - 1), j[u], target[u], cell[u]) && idx < span;
+                    live[u] = live[u] & (base + u * NT + lane < span);
                     edge[u] = behind[u] = false;
                     perp2[u] = sd[u] = 0.f;
                 }
@@ -1290,23 +1349,22 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
                     double tp[U][D];
 #pragma unroll
                     for (int u = 0; u < U; u++) load_pos<RES>(a, q, target[u], tp[u]);
+                    // minimum image in FP32: within 2^-23 L of the exact separation (the difference's
+                    // conversion, the product with L), except within that of +-L / 2
 #pragma unroll
                     for (int u = 0; u < U; u++) {
+                        float f[D], lo[D];
 #pragma unroll
                         for (int d = 0; d < D; d++) {
-                            double v = tp[u][d] - g.ap[d];
-                            const double w = v - (v >= q.half ? q.L : 0.0);   // one of the two corrections is zero
-                            v = w + (v < -q.half ? q.L : 0.0);
-                            const float f = (float)v;
-                            const float lo = fmaxf(fabsf(f) * (1.f - 0x1p-17f) - 0x1p-100f, 0.f);
-                            if (d == dir) {
-                                sd[u] = f;
-                                edge[u] = !(fabs(v) < edge_at);
-                                behind[u] = v < behind_at;
-                            } else {
-                                perp2[u] += lo * lo;
-                            }
+                            const float v = (float)(tp[u][d] - g.ap[d]);
+                            f[d] = fmaf(-Lf, rintf(v * inv_L), v);
+                            lo[d] = fmaxf(fabsf(f[d]) - Lf * 0x1p-21f, 0.f);
                         }
+                        sd[u] = pick_axis<D>(f, dir);
+                        const float p = dir == 0 ? lo[1] : lo[0], p2 = D > 2 ? (dir == 2 ? lo[1] : lo[D - 1]) : 0.f;
+                        perp2[u] = fmaf(p, p, p2 * p2);
+                        edge[u] = !(fabsf(sd[u]) < (0.5f - 0x1p-20f) * Lf);
+                        behind[u] = sd[u] < -0x1p-20f * Lf;
                     }
                 }
 #pragma unroll 1
