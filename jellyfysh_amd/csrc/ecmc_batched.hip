@@ -122,10 +122,25 @@ static int launch_class(ecmc_batch *b, int c, int legs, hipStream_t st) {
     A.log = b->d_log;
     A.audit = b->d_audit;
     int wpr = b->class_wpr[c];
-    size_t lds = batched_lds_bytes(A.nmax, A.cellmax, wpr);
     int dev = 0, cus = 0;
     hipGetDevice(&dev);
     hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    // One wavefront per replica is the best use of a full card; replicas too few to fill it are run by
+    // the idle wavefronts too (the events are the same).  Beyond 27 cells' worth of candidates the
+    // leg's first pass is long enough: 64 to 256 replicas of 2048 units 14.3 -> 12.2 ms with four,
+    // 1024 replicas 15.9 -> 14.3 ms with two, 64 replicas of 512 units 12.8 -> 11.6 ms with four; 64
+    // replicas of 128 units lose (9.3 against 11.1 ms), and so does every size where the workgroups
+    // no longer are resident at once (1024 replicas with four: 22.6 ms).
+    constexpr int WIDE_UNITS = 384;
+    if (wpr == 1 && b->max_blocks == 0 && A.nmax >= WIDE_UNITS) {
+        if (A.count <= 2 * cus) wpr = 4;
+        else if (A.count <= 4 * cus) wpr = 2;
+        int fit = 0;
+        if (wpr == 4) hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<4, false>, 256, batched_lds_bytes(A.nmax, A.cellmax, 4));
+        if (wpr == 2) hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<2, false>, 128, batched_lds_bytes(A.nmax, A.cellmax, 2));
+        if (fit * cus < A.count) wpr = 1;
+    }
+    size_t lds = batched_lds_bytes(A.nmax, A.cellmax, wpr);
     int per_cu = 1;
 #define ECMC_LAUNCH(W)                                                                                     \
     {                                                                                                      \

@@ -550,11 +550,11 @@ enum { TIME_COULOMB_BOUND = 16, TIME_RATE = 17 };
 // Candidate time displacement (send_event_time of the pair event handlers): the potential change
 // dU = -log(1 - u) / beta of the words (w0, w1), inverted for separation (s0, s1, s2), parameters
 // p0 .. p2 and charges c1, c2; x is rc^p of a truncated inverse power or the box length of the
-// Coulomb bound.  A call, not inlined: everything comes in registers, and inside the leg loop the
+// Coulomb bound; p2, x and y are the minimum and the two factors of a Lennard-Jones potential.  A call, not inlined: everything comes in registers, and inside the leg loop the
 // constants and temporaries of these chains would push the loop's own state out of them.
 template <int D, int FM>
-__device__ __noinline__ static double pair_time(int how, double p0, double p1, double p2, double x, int dir, double speed, double s0,
-                                                double s1, double s2, double c1, double c2, uint32_t w0, uint32_t w1, double beta) {
+__device__ __noinline__ static double pair_time(int how, double p0, double p1, double p2, double x, double y, int dir, double speed,
+                                                double s0, double s1, double s2, double c1, double c2, uint32_t w0, uint32_t w1, double beta) {
     double s[D];
     s[0] = s0;
     s[1] = s1;
@@ -587,7 +587,7 @@ __device__ __noinline__ static double pair_time(int how, double p0, double p1, d
     if (POT_BUILT(ECMC_POT_HARD_SPHERE) && how == ECMC_POT_HARD_SPHERE) return hs_displacement<D>(dir, speed, s, p0);
     if (POT_BUILT(ECMC_POT_HARD_DIPOLE) && how == ECMC_POT_HARD_DIPOLE) return hd_displacement<D>(dir, speed, s, p0, p1);
     if (POT_BUILT(ECMC_POT_LENNARD_JONES) && how == ECMC_POT_LENNARD_JONES)
-        return mh_displacement<D>(mh_lennard_jones(p0, p1), dir, speed, s, dU);
+        return mh_displacement<D>(MexicanHat{1, p0, p1, p2, p2 * p2, x, y, 0.0, 0.0}, dir, speed, s, dU);
     if (POT_BUILT(ECMC_POT_DISPLACED_EVEN_POWER) && how == ECMC_POT_DISPLACED_EVEN_POWER)
         return mh_displacement<D>(mh_displaced_even_power(p0, p1, p2), dir, speed, s, dU);
     return NAN;
@@ -660,6 +660,7 @@ struct TaggerPlan {
     int32_t set_key;     // taggers with one key enumerate the same candidates
     float rc2_hi;        // squared cutoff rounded up (+inf: none)
     double powrc;        // rc^p of a truncated inverse power
+    double r0, k6, k12;  // Lennard-Jones: the minimum and the factors of r^-6 and r^-12
 };
 // A candidate to invert exactly: its first random word and push rank (both from the leg's first),
 // its unit, and tagger | target cell << 4 (the cell of a cell-bounding candidate).
@@ -1447,7 +1448,12 @@ __device__ __forceinline__ double candidate_dt(const ChainArgs &a, const Geo<D> 
     }
     const int eh = tg.event_handler;
     int how = tg.potential;
-    double p0 = tg.par[0], p1 = tg.par[1], p2 = tg.par[2], x = sh.plan[tag].powrc;
+    double p0 = tg.par[0], p1 = tg.par[1], p2 = tg.par[2], x = sh.plan[tag].powrc, y = 0.0;
+    if (POT_BUILT(ECMC_POT_LENNARD_JONES) && how == ECMC_POT_LENNARD_JONES) {
+        p2 = sh.plan[tag].r0;
+        x = sh.plan[tag].k6;
+        y = sh.plan[tag].k12;
+    }
     if ((FM & FEAT_COULOMB) && eh == ECMC_EH_TWO_LEAF_BOUNDING) {
         how = TIME_COULOMB_BOUND;
         p0 = tg.bpar[0];
@@ -1457,7 +1463,7 @@ __device__ __forceinline__ double candidate_dt(const ChainArgs &a, const Geo<D> 
         how = TIME_RATE;
         p0 = cell_rate_of_cells<D>(a, q, tg, g.occ_cell, cell, g.adir, ca, ct);
     }
-    return pair_time<D, FM>(how, p0, p1, p2, x, g.adir, g.aspeed, s[0], s[1], s[D - 1], ca, ct, w0, w1, beta);
+    return pair_time<D, FM>(how, p0, p1, p2, x, y, g.adir, g.aspeed, s[0], s[1], s[D - 1], ca, ct, w0, w1, beta);
 }
 
 // Keeps the earlier of two candidates by (time, push rank).
@@ -2196,6 +2202,13 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
         pl.p = 1;
         pl.rc2_hi = INFINITY;
         pl.powrc = 1.0;
+        pl.r0 = pl.k6 = pl.k12 = 0.0;
+        if (pair_kind(kind) && tg.potential == ECMC_POT_LENNARD_JONES) {
+            const MexicanHat h = mh_lennard_jones(tg.par[0], tg.par[1]);
+            pl.r0 = h.r0;
+            pl.k6 = h.k6;
+            pl.k12 = h.k12;
+        }
         pl.set_key = 16 + lane;
         if (pair_kind(kind)) {
             inversion = tg.event_handler == ECMC_EH_TWO_LEAF_BOUNDING                                                          ? 1

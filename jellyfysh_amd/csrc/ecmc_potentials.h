@@ -257,7 +257,7 @@ ECMC_FN double mh_potential(const MexicanHat &h, const double *s) {
 ECMC_FN double mh_invert_inside(const MexicanHat &h, double u) {
     if (h.lj) {
         double so6 = (1 + cr_pow(1 + 4 * u / h.prefactor, 0.5)) / 2;
-        return h.sigma / cr_pow(so6, 1.0 / 6.0);
+        return h.sigma / root36(so6, true);
     }
     return h.r0 - cr_pow(u / h.prefactor, h.inverse_power);
 }
@@ -265,7 +265,7 @@ ECMC_FN double mh_invert_outside(const MexicanHat &h, double u) {
     if (h.lj) {
         if (u >= 0.0) return INFINITY;
         double so6 = (1 - cr_pow(1 + 4 * u / h.prefactor, 0.5)) / 2;
-        return h.sigma / cr_pow(so6, 1.0 / 6.0);
+        return h.sigma / root36(so6, true);
     }
     return h.r0 + cr_pow(u / h.prefactor, h.inverse_power);
 }
