@@ -433,8 +433,18 @@ __device__ __forceinline__ int pos_to_cell(const Geo<D> &q, const double *p, int
 
 template <int D>
 __device__ __forceinline__ void separation_vector(const Geo<D> &q, const double *ap, const double *tp, double *s) {
+    // within one period either way py_mod's value is x, x - L or x + L
+    bool far = false;
+    double x[D];
 #pragma unroll
-    for (int d = 0; d < D; d++) s[d] = py_mod((tp[d] - ap[d]) + q.half, q.L) - q.half;
+    for (int d = 0; d < D; d++) {
+        x[d] = (tp[d] - ap[d]) + q.half;
+        far |= !((x[d] > -q.L) & (x[d] < 2.0 * q.L));
+        s[d] = (x[d] < 0.0 ? x[d] + q.L : (x[d] >= q.L ? x[d] - q.L : x[d])) - q.half;
+    }
+    if (!far) return;
+#pragma unroll
+    for (int d = 0; d < D; d++) s[d] = py_mod(x[d], q.L) - q.half;
 }
 template <int D>
 __device__ __forceinline__ void separation_vector_u(const Geo<D> &q, const double *ap, const double *tp, double *s) {
@@ -521,6 +531,7 @@ struct SettledPowers {   // powers 6 and 12
     __device__ __forceinline__ double half(double r2, double power) { return pow36_settled(r2, power == 12.0, ok); }
     __device__ __forceinline__ double root(double x, double power) { return root36_settled(x, power == 12.0, ok); }
 };
+__device__ __forceinline__ double over_speed(double x, double speed) { return speed == 1.0 ? x : x / speed; }
 template <int D, class Powers>
 __device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, const double *sep, double pp, double power, double rc2,
                                           double urc, double dU) {
@@ -540,7 +551,7 @@ __device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, cons
     const double nsq = m.root(live ? pp / (cur + dU) : 1.0, power);
     const double a = nsq - perp2;
     const double sq = sqrt(fmax(a, 0.0));
-    const double res = a < 0.0 ? NAN : (rep ? sdd - sq : disp + (sdd + sq)) / speed;
+    const double res = a < 0.0 ? NAN : over_speed(rep ? sdd - sq : disp + (sdd + sq), speed);
     return live ? res : INFINITY;
 }
 
@@ -580,10 +591,10 @@ __device__ __noinline__ static double pair_time(int how, double p0, double p1, d
         double p[3] = {0, 0, 0};
 #pragma unroll
         for (int d = 0; d < D; d++) p[d] = pick_axis<D>(s, dir + d >= D ? dir + d - D : dir + d);
-        return ipcb_displacement(p0 * c1 * c2, p[0], p[1], p[2], dU, x) / speed;
+        return over_speed(ipcb_displacement(p0 * c1 * c2, p[0], p[1], p[2], dU, x), speed);
     }
     // two_leaf_unit_cell_bounding_potential_event_handler.py:171-177, p0 the rate
-    if ((FM & FEAT_CELL_BOUNDING) && how == TIME_RATE) return (p0 > 0 ? dU / p0 : INFINITY) / speed;
+    if ((FM & FEAT_CELL_BOUNDING) && how == TIME_RATE) return over_speed(p0 > 0 ? dU / p0 : INFINITY, speed);
     if (POT_BUILT(ECMC_POT_HARD_SPHERE) && how == ECMC_POT_HARD_SPHERE) return hs_displacement<D>(dir, speed, s, p0);
     if (POT_BUILT(ECMC_POT_HARD_DIPOLE) && how == ECMC_POT_HARD_DIPOLE) return hd_displacement<D>(dir, speed, s, p0, p1);
     if (POT_BUILT(ECMC_POT_LENNARD_JONES) && how == ECMC_POT_LENNARD_JONES)
@@ -714,6 +725,8 @@ struct HotList {
     uint32_t creators;      // bit t: tagger t creates this list
     uint32_t prefixed;      // bit t: tagger t creates other taggers, then this list
     uint32_t trashers;      // bit t: tagger t trashes all of this list
+    int32_t hard;           // its one pair tagger is a hard sphere's, of this radius
+    double radius;
 };
 
 struct SlotTime {
@@ -2039,8 +2052,10 @@ __device__ __forceinline__ void commit_event(const ChainArgs &a, const Geo<D> &q
 // ---- launch ---------------------------------------------------------------------------------
 // The hot list: the create list of the first pair tagger, if it has the form (one thread).
 template <int NT>
-__device__ __forceinline__ HotList hot_list(const ChainShared<NT> &sh, uint64_t kinds, int n_taggers) {
+__device__ __forceinline__ HotList hot_list(const ChainShared<NT> &sh, const ecmc_tagger_desc *tg, uint64_t kinds, int n_taggers) {
     HotList l;
+    l.hard = 0;
+    l.radius = 0.0;
     l.items = -1;
     l.tags = l.mask = l.creators = l.prefixed = l.trashers = 0;
     l.boundary = l.veto = -1;
@@ -2084,6 +2099,9 @@ __device__ __forceinline__ HotList hot_list(const ChainShared<NT> &sh, uint64_t 
         else l.prefixed |= 1u << t;
     }
     l.items = items;
+    const ecmc_tagger_desc &pair = tg[l.tags & 15u];
+    l.hard = items == 1 && pair.event_handler == ECMC_EH_TWO_LEAF && pair.potential == ECMC_POT_HARD_SPHERE;
+    l.radius = pair.par[0];
     return l;
 }
 
@@ -2266,7 +2284,7 @@ __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D
 #pragma unroll
         for (int d = 0; d < D; d++) { m.side[d] = q.side[d]; m.inv[d] = q.inv[d]; m.cps[d] = q.cps[d]; m.cum[d] = q.cum[d]; }
         m.nb_cells = q.nb_cells; m.kinds = q.kinds; m.tests = q.tests; m.inversions = q.inversions; m.draws = q.draws; m.charged = q.charged;
-        sh.hot = hot_list<NT>(sh, q.kinds, a.n_taggers);
+        sh.hot = hot_list<NT>(sh, q.tg, q.kinds, a.n_taggers);
     }
     __syncthreads();
     if (g.active >= 0) load_pos<RES>(a, q, g.active, g.ap);
@@ -2673,7 +2691,16 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
                     }
                     c = sh.queue[w][k];
                 }
-                const double dt = candidate_dt<D, FM, NT, RES>(a, q, g, sh, c.tag_cell & 15, c.word, c.target, c.tag_cell >> 4);
+                double dt;
+                if (POT_BUILT(ECMC_POT_HARD_SPHERE) && hot.hard) {
+                    // nothing is drawn or looked up: the call's generality costs more than the root
+                    double tp[D], s[D];
+                    load_pos<RES>(a, q, c.target, tp);
+                    separation_vector<D>(q, g.ap, tp, s);
+                    dt = hs_displacement<D>(g.adir, g.aspeed, s, hot.radius);
+                } else {
+                    dt = candidate_dt<D, FM, NT, RES>(a, q, g, sh, c.tag_cell & 15, c.word, c.target, c.tag_cell >> 4);
+                }
                 Winner v;
                 v.t = time_add(g.at, dt);
                 v.dt = dt;
@@ -2746,6 +2773,8 @@ __device__ __forceinline__ void chain_body(const ChainArgs &a) {
     hot.veto = uni(sh.hot.veto);
     hot.before = uni(sh.hot.before);
     hot.veto_before = uni(sh.hot.veto_before);
+    hot.hard = uni(sh.hot.hard);
+    hot.radius = uni(sh.hot.radius);
     hot.mask = (uint32_t)uni((int)sh.hot.mask);
     hot.creators = (uint32_t)uni((int)sh.hot.creators);
     hot.prefixed = (uint32_t)uni((int)sh.hot.prefixed);

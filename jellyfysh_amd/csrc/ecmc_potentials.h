@@ -53,7 +53,8 @@ ECMC_FN double hs_displacement(int dir, double speed, const double *s, double ra
 #pragma unroll
     for (int i = 0; i < D; i++) vs = vs + v[i] * s[i];
     double srt = vs * vs - v2 * (s2 - diam2);
-    return (srt >= 0.0 && vs >= 0.0) ? (vs - sqrt(srt)) / v2 : INFINITY;
+    const double t = vs - sqrt(fmax(srt, 0.0));
+    return (srt >= 0.0 && vs >= 0.0) ? (v2 == 1.0 ? t : t / v2) : INFINITY;
 }
 
 // HardDipolePotential.displacement (hard_dipole_potential.py:66-110): the time until the
