@@ -465,7 +465,7 @@ def main():
     launch_ms = dom_ms / max(dom_launches, 1)
     achieved = flops_per_launch / (launch_ms * 1e-3) / 1e12
     exact = float((s1["stats"][:, 3] - s0["stats"][:, 3]).sum())
-    dom_name = "ecmc::batched_kernel<%d, false>" % batch.classes[1][dom]
+    dom_name = "ecmc::batched_kernel<%d,false>" % batch.classes[1][dom]
     traffic = profiled_traffic(dom_name, args.legs)
     # pressure from untimed production steps after the timed region (each replica then has
     # (warmup + steps) x legs legs behind it)

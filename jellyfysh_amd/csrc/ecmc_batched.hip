@@ -2,18 +2,18 @@
 // persistent kernel per size class.
 //
 // Each workgroup (WPR wavefronts) pulls replicas from a queue sorted largest first (LPT)
-// and runs `legs` legs on each.  A replica's FP32 positions and its cell lists live in LDS;
+// and runs `legs` legs on each.  A replica's fixed-point positions, sorted by cell, live in LDS;
 // its FP64 positions stay in HBM, where only the active unit's row changes.  One leg:
 //   1. horizon h = min(displacement to the next cell wall, rest of the chain), FP64;
 //   2. every candidate (occupants of the 27 nearby cells, or all units when the box holds
-//      fewer than three cells per side) and factor gets an FP32 lower bound on its event
-//      displacement, with a proven downward margin; only those whose bound is <= h enter
-//      a contender list in LDS;
+//      fewer than three cells per side) and factor gets an FP32 upper bound on the rise of its
+//      energy within h, with a proven upward margin; only those whose bound reaches the draw
+//      enter a contender list in LDS;
 //   3. the contenders are inverted exactly in FP64 (correctly rounded pow/log) and a
 //      workgroup min-reduce over (displacement, kind, target, factor) picks the event;
 //   4. thread 0 commits it (lifting, wall snap, or end of chain with a Philox-drawn new
 //      active unit) and updates the cell lists.
-// Because every bound is <= the exact FP64 value, the committed event is the one a full
+// Because a factor left out has no event within h, the committed event is the one a full
 // FP64 evaluation of every candidate selects; the audit mode checks that on the device.
 #include <hip/hip_runtime.h>
 #include <math.h>

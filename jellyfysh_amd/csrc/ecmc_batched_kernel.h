@@ -116,7 +116,7 @@ struct Reach {
 //                      cutoff: rise = V(nearest) - max(V(at hf), V(rc)), V = |k| / r^p.
 // Bounded up with the nearest distance from below and the farther one from above; no power or
 // logarithm has to be inverted for it (a bound on the displacement itself takes two exp2/log2
-// pairs and a root per factor: 350 instead of 200 instructions per 64 candidates).  Infinite or
+// pairs and a root per factor).  Infinite or
 // NaN bounds (a nearest distance of zero) keep the candidate.
 __device__ __forceinline__ bool factor_surely_later(const Reach &g, float k, bool twelve, float rc2_hi, float vrc_lo, float hf,
                                                     float dU_lo) {
@@ -484,13 +484,17 @@ __host__ __device__ inline size_t batched_lds_bytes(int nmax, int cellmax, int w
 //   2. pass 1a over every candidate: the fixed-point separation against the capsule of
 //      radius rc about the segment of motion (cand_near); candidates outside are done, the
 //      others are appended to the wavefront's queue (ballot compaction);
-//   3. pass 1b over each full queue: FP32 geometry with the position slack, Philox draws,
-//      FP32 lower bounds of the event displacements (FP32 dU bound from the draw's leading
-//      bits); a factor whose bound is <= h is a contender;
+//   3. pass 1b over each full queue: FP32 geometry with the position slack, Philox draws (FP32
+//      bound of dU from the draw's leading bits); a factor whose energy may rise by the draw
+//      within h (factor_surely_later) is a contender;
 //   4. pass 2, one contender per thread: its FP64 position from global memory, exact FP64
 //      inversion with correctly rounded pow/log, workgroup min-reduce over (displacement,
 //      kind, target, factor);
 //   5. thread 0 commits.
+// Bound by the instructions it issues: with two wavefronts per SIMD (LDS for the largest replica
+// and 256 VGPRs) the VALU is busy 72% of the time.  1697 vector instructions a leg before the
+// cell-sorted records, the runs, the energy test, the division-free cells and the inlined
+// inversion, 1280 with them; 4096 replicas of 64 to 2048 units, 20 000 legs each: 343 -> 270 ms.
 //
 // CHECK: modes 1 and 2 (their own instance, so that the filtered mode's registers hold nothing of
 // them).

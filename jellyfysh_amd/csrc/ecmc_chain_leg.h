@@ -4,9 +4,19 @@
 // the chain's state (active unit, its position, time, random cursor, estimators) in registers
 // and runs the sequential part of a leg -- create lists, cell-boundary and end-of-chain events,
 // selection, commit -- redundantly on the same values, so nothing of it is broadcast.  Only
-// wavefront 0 writes the shared lists (cell occupants, positions, stored events) and memory.  A leg has at most three barriers: after
-// the occupancy update when the active unit changed, after the candidate tests, and after the
-// exact inversions.
+// wavefront 0 writes the shared lists (cell occupants, positions, stored events) and memory.  A leg
+// has at most three barriers: after the occupancy update when the active unit changed, after the
+// candidate tests, and after the exact inversions.
+//
+// Bound by latency: one wavefront per SIMD issues an instruction of the leg's dependent chain about
+// every seven cycles (4 to issue, the rest waits for results and LDS), whatever the chip could do
+// besides; HBM and the FP64 rate are idle.  So a leg costs what its chain of instructions is long.
+// Cycles per leg, one chain of 4096 Lennard-Jones units: occupancy 3400, nearby cells 2900, quick
+// test of 512 candidates 6000, inversion of 5.6 contenders 6400 (beside it 1000 random words), their
+// winner 1500, selection and event 2300, commit 1500, the loop 2300.  Leg times at the start of this
+// form's work and now: 34.6 -> 11.9 us here, 11.7 -> 5.4 us for 256 hard disks, 66.6 -> 22.4 us for
+// 256 systems of 512 charges with cell bounding, 51.7 -> 18.7 us with the cell veto, 53.6 -> 19.2 us for
+// 64 systems of 1000 dipole units.
 //
 // The pair candidates of all taggers of a create list are evaluated together:
 //   1. every candidate gets a cheap FP32 test (quick_cull) whether its factor can rise by the
@@ -322,8 +332,8 @@ __device__ __forceinline__ void ring_make(uint32_t *ring, uint32_t mask, uint64_
 }
 // The same in LDS, where a wavefront's operations are in order: nothing waits for a step's writes, the
 // words 624 and 623 back of the next step (older than this step's) are read while this one waits
-// for its words 227 back, and the mask is left out where none of the four runs wraps.  570 -> 330
-// cycles a step.
+// for its words 227 back, and the mask is left out where none of the four runs wraps.  575 -> 465
+// cycles a step of 192 words (21 steps a leg of 1000 dipole units).
 __device__ __forceinline__ void ring_make_lds(uint32_t *ring, uint32_t mask, uint64_t from, int steps) {
     constexpr int U = RING_STEP / 64;
     const uint32_t lane = threadIdx.x & 63;
@@ -517,23 +527,9 @@ constexpr int VARIANT_DIPOLES = (1 << ECMC_POT_INVERSE_POWER) | (1 << ECMC_POT_D
 // run two paths: the same operations on the same values.  urc = U(rc) and rc2 = rc^2 of the
 // truncated form, 0 and +inf without a cutoff (then current >= urc is the reference's test
 // against zero).
-//
-// SettledPowers takes the powers through the fast paths alone, without a branch or a call between
-// them (ok turns false where they do not settle a rounding, about one time in 10^4): the two
-// powers, the logarithm of the draw and the root's parts then overlap in one instruction stream.
-// 6300 -> 3900 cycles for the contenders of a Lennard-Jones leg.
-struct AnyPowers {
-    __device__ __forceinline__ double half(double r2, double power) { return pow_half_power(r2, power); }
-    __device__ __forceinline__ double root(double x, double power) { return root_two_over_power(x, power); }
-};
-struct SettledPowers {   // powers 6 and 12
-    bool ok = true;
-    __device__ __forceinline__ double half(double r2, double power) { return pow36_settled(r2, power == 12.0, ok); }
-    __device__ __forceinline__ double root(double x, double power) { return root36_settled(x, power == 12.0, ok); }
-};
 __device__ __forceinline__ double over_speed(double x, double speed) { return speed == 1.0 ? x : x / speed; }
-template <int D, class Powers>
-__device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, const double *sep, double pp, double power, double rc2,
+template <int D>
+__device__ __forceinline__ double ip_time(int dir, double speed, const double *sep, double pp, double power, double rc2,
                                           double urc, double dU) {
     const bool rep = pp > 0.0;
     const double perp2 = others_sq<D>(sep, dir);
@@ -545,10 +541,10 @@ __device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, cons
     for (int d = 0; d < D; d++) c[d] = d == dir ? sdd : sep[d];
     const double sn2 = norm_sq<D>(c);
     bool live = perp2 < rc2 && (rep ? sd > 0.0 : sn2 < rc2);
-    const double cur = (rep && !(sn2 < rc2)) ? urc : pp / m.half(live ? sn2 : 1.0, power);
-    const double maxp = pp / m.half(rep && live ? perp2 : 1.0, power);
+    const double cur = (rep && !(sn2 < rc2)) ? urc : pp / pow_half_power(live ? sn2 : 1.0, power);
+    const double maxp = pp / pow_half_power(rep && live ? perp2 : 1.0, power);
     live = live && (rep ? dU < maxp - cur : !(cur + dU >= urc));
-    const double nsq = m.root(live ? pp / (cur + dU) : 1.0, power);
+    const double nsq = root_two_over_power(live ? pp / (cur + dU) : 1.0, power);
     const double a = nsq - perp2;
     const double sq = sqrt(fmax(a, 0.0));
     const double res = a < 0.0 ? NAN : over_speed(rep ? sdd - sq : disp + (sdd + sq), speed);
@@ -570,21 +566,12 @@ __device__ __noinline__ static double pair_time(int how, double p0, double p1, d
     s[0] = s0;
     s[1] = s1;
     if (D > 2) s[D - 1] = s2;
-    if ((FM & FEAT_IP) && (how == ECMC_POT_INVERSE_POWER || how == ECMC_POT_INVERSE_POWER_TRUNC) && (p0 == 12.0 || p0 == 6.0)) {
-        const bool trunc = how == ECMC_POT_INVERSE_POWER_TRUNC;
-        const double pp = (c1 * c2) * p1;
-        SettledPowers m;
-        const double change = -log_settled(1.0 - words_to_random(w0, w1), m.ok) / beta;
-        const double dt = ip_time<D>(m, dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, change);
-        if (m.ok) return dt;
-    }
     // hard potentials draw nothing (beta = 0 marks them)
     const double dU = beta != 0.0 ? -cr_log(1.0 - words_to_random(w0, w1)) / beta : 0.0;
     if ((FM & FEAT_IP) && (how == ECMC_POT_INVERSE_POWER || how == ECMC_POT_INVERSE_POWER_TRUNC)) {
         const bool trunc = how == ECMC_POT_INVERSE_POWER_TRUNC;
         const double pp = (c1 * c2) * p1;
-        AnyPowers m;
-        return ip_time<D>(m, dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, dU);
+        return ip_time<D>(dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, dU);
     }
     if ((FM & FEAT_COULOMB) && how == TIME_COULOMB_BOUND) {
         // two_leaf_unit_bounding_potential_event_handler.py:138-143 with the Coulomb bound
@@ -1804,8 +1791,9 @@ __device__ __noinline__ static double ewald_derivative_wave(const Ewald &e, cons
 //   Fourier  sines of fractions of a period by the 2e-9 polynomial 4.3.97 of Abramowitz and Stegun,
 //            each within 4e-7, a product of three within 2^-19;
 // and the sum over the lanes adds 9 roundings of partial sums: 2^-18 + 2^-20 z of a real term and
-// 2^-18 |f| of a Fourier term bound it, terms that underflow are 1e-38 of it.  2100 cycles against
-// 9700 of the FP64 sum (an exp, an erfc and two divisions in one chain, three rounds of terms).
+// 2^-18 |f| of a Fourier term bound it, terms that underflow are 1e-38 of it.  The commit of a charged
+// leg took 11 700 cycles with the FP64 sum (an exp, an erfc and two divisions in one chain, three
+// rounds of terms) and takes 6300.
 __device__ __forceinline__ float sin_turn(float f) {   // sin(2 pi f) for |f| <= 1/4
     const float y = f * 6.2831853f, y2 = y * y;
     return y * fmaf(y2, fmaf(y2, fmaf(y2, fmaf(y2, fmaf(y2, -2.39e-8f, 2.7526e-6f), -1.98409e-4f), 8.3333315e-3f), -0.1666666664f), 1.f);
@@ -2657,7 +2645,8 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
         Winner m = no_winner();
         const int workers = NW > 1 && !direct ? NW - 1 : NW;
         // few contenders: each kind of inversion on a wavefront of its own, so that they run side by
-        // side and not one after the other in one wavefront
+        // side and not one after the other in one wavefront (12 000 -> 9000 cycles for the 33
+        // contenders of three kinds of a charged leg)
         const bool by_kind = NW > 1 && !direct && total <= 64;
         const int kind_here = wave == 0 ? 0 : wave - 1;
         int b = by_kind ? (wave == maker ? total : 0) : direct ? wave * 64 : (NW > 1 ? (wave == 0 ? 0 : (wave == maker ? total : (wave - 1) * 64)) : 0);

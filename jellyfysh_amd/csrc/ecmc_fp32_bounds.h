@@ -1,5 +1,6 @@
-// ecmc_fp32_bounds.h -- FP32 brackets of inverse-power event displacements, for the
-// candidate filters of the batched kernel and of the chain kernel.
+// ecmc_fp32_bounds.h -- FP32 brackets of inverse-power event displacements
+// (ecmc_pair_time_bounds), and the directed FP32 steps and draws under them that the batched
+// kernel's and the chain kernel's candidate tests use too.
 //
 // Every quantity is bracketed [lo, hi] and each FP32 operation is covered by a relative
 // margin (ETA for products/quotients/roots, ETA_POW or a logarithm-scaled margin for the
