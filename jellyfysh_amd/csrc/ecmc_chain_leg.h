@@ -527,9 +527,23 @@ constexpr int VARIANT_DIPOLES = (1 << ECMC_POT_INVERSE_POWER) | (1 << ECMC_POT_D
 // run two paths: the same operations on the same values.  urc = U(rc) and rc2 = rc^2 of the
 // truncated form, 0 and +inf without a cutoff (then current >= urc is the reference's test
 // against zero).
+//
+// SettledPowers takes the powers through the fast paths alone, without a branch or a call between
+// them (ok turns false where they do not settle a rounding, about one time in 500, by the logarithm of
+// the draw): the two powers, the logarithm and the root's parts then overlap in one instruction
+// stream.  1000 legs of 4096 Lennard-Jones units: 12.12 -> 11.90 ms.
+struct AnyPowers {
+    __device__ __forceinline__ double half(double r2, double power) { return pow_half_power(r2, power); }
+    __device__ __forceinline__ double root(double x, double power) { return root_two_over_power(x, power); }
+};
+struct SettledPowers {   // powers 6 and 12
+    bool ok = true;
+    __device__ __forceinline__ double half(double r2, double power) { return pow36_settled(r2, power == 12.0, ok); }
+    __device__ __forceinline__ double root(double x, double power) { return root36_settled(x, power == 12.0, ok); }
+};
 __device__ __forceinline__ double over_speed(double x, double speed) { return speed == 1.0 ? x : x / speed; }
-template <int D>
-__device__ __forceinline__ double ip_time(int dir, double speed, const double *sep, double pp, double power, double rc2,
+template <int D, class Powers>
+__device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, const double *sep, double pp, double power, double rc2,
                                           double urc, double dU) {
     const bool rep = pp > 0.0;
     const double perp2 = others_sq<D>(sep, dir);
@@ -541,10 +555,10 @@ __device__ __forceinline__ double ip_time(int dir, double speed, const double *s
     for (int d = 0; d < D; d++) c[d] = d == dir ? sdd : sep[d];
     const double sn2 = norm_sq<D>(c);
     bool live = perp2 < rc2 && (rep ? sd > 0.0 : sn2 < rc2);
-    const double cur = (rep && !(sn2 < rc2)) ? urc : pp / pow_half_power(live ? sn2 : 1.0, power);
-    const double maxp = pp / pow_half_power(rep && live ? perp2 : 1.0, power);
+    const double cur = (rep && !(sn2 < rc2)) ? urc : pp / m.half(live ? sn2 : 1.0, power);
+    const double maxp = pp / m.half(rep && live ? perp2 : 1.0, power);
     live = live && (rep ? dU < maxp - cur : !(cur + dU >= urc));
-    const double nsq = root_two_over_power(live ? pp / (cur + dU) : 1.0, power);
+    const double nsq = m.root(live ? pp / (cur + dU) : 1.0, power);
     const double a = nsq - perp2;
     const double sq = sqrt(fmax(a, 0.0));
     const double res = a < 0.0 ? NAN : over_speed(rep ? sdd - sq : disp + (sdd + sq), speed);
@@ -566,12 +580,21 @@ __device__ __noinline__ static double pair_time(int how, double p0, double p1, d
     s[0] = s0;
     s[1] = s1;
     if (D > 2) s[D - 1] = s2;
+    if ((FM & FEAT_IP) && (how == ECMC_POT_INVERSE_POWER || how == ECMC_POT_INVERSE_POWER_TRUNC) && (p0 == 12.0 || p0 == 6.0)) {
+        const bool trunc = how == ECMC_POT_INVERSE_POWER_TRUNC;
+        const double pp = (c1 * c2) * p1;
+        SettledPowers m;
+        const double change = -log_settled(1.0 - words_to_random(w0, w1), m.ok) / beta;
+        const double dt = ip_time<D>(m, dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, change);
+        if (m.ok) return dt;
+    }
     // hard potentials draw nothing (beta = 0 marks them)
     const double dU = beta != 0.0 ? -cr_log(1.0 - words_to_random(w0, w1)) / beta : 0.0;
     if ((FM & FEAT_IP) && (how == ECMC_POT_INVERSE_POWER || how == ECMC_POT_INVERSE_POWER_TRUNC)) {
         const bool trunc = how == ECMC_POT_INVERSE_POWER_TRUNC;
         const double pp = (c1 * c2) * p1;
-        return ip_time<D>(dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, dU);
+        AnyPowers m;
+        return ip_time<D>(m, dir, speed, s, pp, p0, trunc ? p2 * p2 : INFINITY, trunc ? pp / x : 0.0, dU);
     }
     if ((FM & FEAT_COULOMB) && how == TIME_COULOMB_BOUND) {
         // two_leaf_unit_bounding_potential_event_handler.py:138-143 with the Coulomb bound
