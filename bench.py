@@ -295,7 +295,7 @@ def charged_spheres_rate(replicas, legs, far="cell_bounding"):
                 chain_displacement_per_sec=float(est[:, 1].sum()) / wall,
                 note="plain chain kernel, one workgroup per replica in one launch; FP64 event times; Coulomb "
                      "far cells through %s (FP64 Ewald tables), nearby and surplus bounds with thinning; "
-                     "repulsion inverted exactly over all pairs" % far.replace("_", " "))
+                     "every candidate tested in FP32 first, the few left inverted exactly in FP64" % far.replace("_", " "))
 
 
 def flexible_dipoles_rate(replicas, legs):
@@ -336,8 +336,7 @@ def flexible_dipoles_rate(replicas, legs):
                 kernel_ms=ms, single_replica_events_per_sec=float(k1[0]) / (ms1 * 1e-3), create_s=create_s,
                 note="plain chain kernel, one workgroup per replica in one launch; leaf units of composite "
                      "objects with factor type maps; Coulomb through the inverse-power Coulomb bound with "
-                     "thinning (FP64 Ewald derivative), bond and repulsion inverted exactly (FP32 brackets "
-                     "first for the repulsion)")
+                     "thinning, every candidate tested in FP32 first and the few left inverted exactly in FP64")
 
 
 def cpu_baseline(n, lengths, pos, seconds, threads):
