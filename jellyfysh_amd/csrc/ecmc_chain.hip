@@ -31,6 +31,7 @@
 #include <math.h>
 #include <vector>
 #include <string>
+#include <atomic>
 #include <mutex>
 #include <utility>
 #include <cmath>
@@ -199,6 +200,7 @@ struct ecmc_system {
     int64_t log_cap = 0;
     int64_t *d_nout = nullptr;
     HostView *host = nullptr;          // pinned: what the last launch left for the host to read
+    std::atomic<uint32_t> began{0}, ended{0};   // calls that launch: begun and ended (see read_host)
     ecmc_event *d_step_ev = nullptr;   // the event of the last host-driven commit
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -742,7 +744,9 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
         }
     }
     plan_lds(s);
-    // the host view; a system without one (pinned memory exhausted) copies what it reads
+    // the host view; a system without one (pinned memory exhausted) copies what it reads.  The allocation
+    // takes 50 to 130 us of a system's creation (0.37 to 0.61 ms each where 256 are created), what the copies of
+    // one or two calls took.
     const bool res_positions = s->args.resident != 0;
     if (hipHostMalloc((void **)&s->host, sizeof(HostView) + (res_positions ? sizeof(double) * dim * n : 0),
                       hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
@@ -785,23 +789,45 @@ static int status_of_state(int err) {
     }
 }
 
+// A call that launches work of these systems, from before the launch to its end.
+struct InFlight {
+    ecmc_system *const *systems;
+    int32_t count;
+    InFlight(ecmc_system *const *systems_, int32_t count_) : systems(systems_), count(count_) {
+        for (int i = 0; i < count; i++) systems[i]->began++;
+    }
+    ~InFlight() {
+        for (int i = 0; i < count; i++) systems[i]->ended++;
+    }
+};
+
+// Copies from the host view, false if a launch may write it meanwhile: another thread's call is
+// under way (`own`: the caller's own, 1 within its InFlight) or began during the copy.  The reader
+// then takes a copy command, which waits for the launches before it.
+static bool read_host(const ecmc_system *s, void *to, const void *from, size_t bytes, uint32_t own) {
+    const uint32_t ended = s->ended.load(), began = s->began.load();
+    if (began - ended != own) return false;
+    memcpy(to, from, bytes);
+    std::atomic_thread_fence(std::memory_order_seq_cst);
+    return s->began.load() == began;
+}
+
 // The state that the last launch left (or the initial one): from the host view, else copied.
-static int read_state(const ecmc_system *s, ChainState &st) {
-    if (s->host) st = s->host->st;
-    else if (hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
+static int read_state(const ecmc_system *s, ChainState &st, uint32_t own = 0) {
+    if (s->host && read_host(s, &st, &s->host->st, sizeof(st), own)) return ECMC_OK;
+    if (hipMemcpy(&st, s->d_st, sizeof(ChainState), hipMemcpyDeviceToHost) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
     return ECMC_OK;
 }
 
 // The committed legs of the launch that just ended and its error code.
 static int read_launch(const ecmc_system *s, int64_t &k, int &err) {
-    if (s->host) {
-        k = s->host->n_out;
-        err = s->host->st.err;
-    } else if (hipMemcpy(&k, s->d_nout, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess ||
-               hipMemcpy(&err, (const char *)s->d_st + offsetof(ChainState, err), sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) {
+    if (s->host && read_host(s, &k, &s->host->n_out, sizeof(k), 1) &&
+        read_host(s, &err, &s->host->st.err, sizeof(err), 1))
+        return ECMC_OK;
+    if (hipMemcpy(&k, s->d_nout, sizeof(int64_t), hipMemcpyDeviceToHost) != hipSuccess ||
+               hipMemcpy(&err, (const char *)s->d_st + offsetof(ChainState, err), sizeof(int), hipMemcpyDeviceToHost) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy failed");
-    }
     return ECMC_OK;
 }
 
@@ -820,6 +846,7 @@ extern "C" int ecmc_system_run(ecmc_system *s, int64_t max_events, ecmc_event *h
     a.log = host_log ? s->d_log : nullptr;
     a.max_events = max_events;
     a.stop_mask = s->stop_mask;
+    const InFlight flight(&s, 1);
     hipEventRecord(s->ev0, s->stream);
     if (hipMemcpyAsync(s->d_args, &a, sizeof(ChainArgs), hipMemcpyHostToDevice, s->stream) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy of the launch arguments failed");
@@ -862,6 +889,7 @@ static int systems_run_staged(ecmc_system *const *systems, int32_t count, int64_
         if (n_committed) n_committed[i] = 0;
     }
     if (max_events == 0) return ECMC_OK;
+    const InFlight flight(systems, count);
     ecmc_system *s0 = systems[0];
     if (hipMemcpyAsync(d_args, host_args, sizeof(ChainArgs) * count, hipMemcpyHostToDevice, s0->stream) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy of the launch arguments failed");
@@ -966,6 +994,7 @@ extern "C" int ecmc_systems_run_noalloc(ecmc_system *const *systems, int32_t cou
 static int system_step(ecmc_system *s, int op, int tagger, ChainState &st) {
     if (!s) return ecmc_fail(ECMC_ERR_ARGUMENT, "null system");
     if (op != 0 && (tagger < 0 || tagger >= s->desc.n_taggers)) return ecmc_fail(ECMC_ERR_ARGUMENT, "no such tagger");
+    const InFlight flight(&s, 1);
     const ChainArgs &sa = s->args;   // one step works on global memory
     if (hipMemcpyAsync(s->d_args, &sa, sizeof(ChainArgs), hipMemcpyHostToDevice, s->stream) != hipSuccess)
         return ecmc_fail(ECMC_ERR_HIP, "hipMemcpy of the launch arguments failed");
@@ -973,7 +1002,7 @@ static int system_step(ecmc_system *s, int op, int tagger, ChainState &st) {
     else hipLaunchKernelGGL((chain_step_kernel<3, FEAT_ALL, 256>), dim3(1), dim3(256), 0, s->stream, s->d_args, op, tagger, s->d_step_ev);
     if (hipGetLastError() != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "kernel launch failed");
     if (hipStreamSynchronize(s->stream) != hipSuccess) return ecmc_fail(ECMC_ERR_HIP, "kernel execution failed");
-    const int rc = read_state(s, st);
+    const int rc = read_state(s, st, 1);
     if (rc) return rc;
     return status_of_state(st.err);
 }
@@ -1013,9 +1042,12 @@ extern "C" int ecmc_system_send_out_state(ecmc_system *s, int32_t tagger, ecmc_e
 
 extern "C" int ecmc_system_positions(const ecmc_system *s, double *out) {
     if (!s || !out) return ecmc_fail(ECMC_ERR_ARGUMENT, "null argument");
-    if (s->host && s->host->has_positions) {
-        memcpy(out, s->host + 1, sizeof(double) * s->dim * s->n);
-        return ECMC_OK;
+    if (s->host) {
+        int32_t filled = 0;
+        const uint32_t began = s->began.load();   // one launch's flag and positions
+        if (read_host(s, &filled, &s->host->has_positions, sizeof(filled), 0) && filled &&
+            read_host(s, out, s->host + 1, sizeof(double) * s->dim * s->n, 0) && s->began.load() == began)
+            return ECMC_OK;
     }
     std::vector<double> soa((size_t)s->dim * s->n);
     if (hipMemcpy(soa.data(), s->d_pos, sizeof(double) * soa.size(), hipMemcpyDeviceToHost) != hipSuccess)

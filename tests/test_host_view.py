@@ -50,3 +50,36 @@ def test_gpu_readers_agree_with_and_without_residency(device, legs):
     _same(a, b)
     assert a.run(legs, log=False) == legs and b.run(legs, log=False) == legs
     _same(a, b)
+
+
+@pytest.mark.parametrize("together", [False, True])
+def test_gpu_reader_on_another_thread_sees_whole_launches(device, together):
+    """A reader beside a running launch gets the state before it or after it, never a part of it."""
+    import threading
+    from jellyfysh_amd.chain import run_together
+    legs = 20000
+    a, b = _chain(3), _chain(3)
+    states = [_read(b)]
+    for _ in range(2):
+        b.run(legs, log=False)
+        states.append(_read(b))
+    keys = [[s[0].tobytes() for s in states], [s[1].tobytes() for s in states]]
+    done = []
+
+    def work():
+        for _ in range(2):
+            done.append(run_together([a], legs)[0][0] if together else a.run(legs, log=False))
+
+    t = threading.Thread(target=work)
+    print("reading beside two launches", flush=True)
+    t.start()
+    seen = [[], []]
+    for _ in range(20000):
+        seen[0].append(keys[0].index(a.positions().tobytes()))
+        seen[1].append(keys[1].index(a.estimators().tobytes()))
+        if not t.is_alive():
+            break
+    t.join(60)
+    assert done == [legs, legs]
+    assert all(s == sorted(s) for s in seen)
+    _same(a, b)
