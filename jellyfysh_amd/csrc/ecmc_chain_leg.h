@@ -4,9 +4,11 @@
 // the chain's state (active unit, its position, time, random cursor, estimators) in registers
 // and runs the sequential part of a leg -- create lists, cell-boundary and end-of-chain events,
 // selection, commit -- redundantly on the same values, so nothing of it is broadcast.  Only
-// wavefront 0 writes the shared lists (cell occupants, positions, stored events) and memory.  A leg
-// has at most three barriers: after the occupancy update when the active unit changed, after the
-// candidate tests, and after the exact inversions.
+// wavefront 0 writes the shared lists (cell occupants, positions, stored events) and memory.  A leg's
+// barriers: after the occupancy update when the active unit changed, after the candidate tests (none
+// where a single set is inverted without them), after the exact inversions, and before the thinning
+// of a cell veto.  Only the third is in every leg, so what wavefronts exchange around it is kept
+// twice (ChainShared::win).
 //
 // Bound by latency: one wavefront per SIMD issues an instruction of the leg's dependent chain about
 // every seven cycles (4 to issue, the rest waits for results and LDS), whatever the chip could do
@@ -760,7 +762,12 @@ struct ChainShared {
     SlotTime time[NW][ECMC_MAX_TAGGERS];     // their times as every wavefront sees them, around a rare step
     TaggerPlan plan[ECMC_MAX_TAGGERS];
     Contender queue[NW][QCAP];
-    Winner win[NW];
+    // The earliest candidate of every wavefront: of the legs in turn, and of the rare steps' full
+    // evaluations.  A leg may have no barrier after the one that its winners are read behind, and the
+    // next leg none before it writes its own: the slowest wavefront may still be reading one copy
+    // while the fastest fills the other, and the barrier of that leg lies before the first is
+    // written again.
+    Winner win[3][NW];
     alignas(16) int32_t nb_cell[NW][32];     // nearby cells and exclusive prefix sums of their occupants
     alignas(16) int32_t nb_pref[NW][32];
     EwaldTerms ewald;
@@ -2357,30 +2364,31 @@ __device__ __forceinline__ void launch_store(const ChainArgs &a, const Geo<D> &q
 }
 
 // The earliest candidate among the work of all wavefronts (each with its lanes' best in m), after
-// one barrier.  `again`: another evaluation of this leg may write sh.win before a barrier.
+// one barrier; `win`: a copy of ChainShared::win that no wavefront reads any more.  The rare steps
+// evaluate several sets one after the other into one copy: `again` ends with a second barrier.
 template <int NT>
-__device__ __forceinline__ Winner group_winner(ChainShared<NT> &sh, const Winner &m, bool again) {
+__device__ __forceinline__ Winner group_winner(Winner *win, const Winner &m, bool again) {
     constexpr int NW = NT / 64;
     Winner w = wave_winner(m);
     if (NW > 1) {
-        if ((threadIdx.x & 63) == 0) sh.win[wave_index<NT>()] = w;
+        if ((threadIdx.x & 63) == 0) win[wave_index<NT>()] = w;
         __syncthreads();
         w = no_winner();
 #pragma unroll
         for (int v = 0; v < NW; v++) {
             // read as uniform values: the comparison is then a scalar branch
             Winner o;
-            o.rank = uni(sh.win[v].rank);
-            w.bad |= uni(sh.win[v].bad);
+            o.rank = uni(win[v].rank);
+            w.bad |= uni(win[v].bad);
             if (o.rank == NO_RANK) continue;
-            o.t.q = uni(sh.win[v].t.q);
-            o.t.r = uni(sh.win[v].t.r);
+            o.t.q = uni(win[v].t.q);
+            o.t.r = uni(win[v].t.r);
             if (w.rank != NO_RANK && !ub(winner_lt(o, w))) continue;
             w.t = o.t;
             w.rank = o.rank;
-            w.dt = uni(sh.win[v].dt);
-            w.tag = uni(sh.win[v].tag);
-            w.target = uni(sh.win[v].target);
+            w.dt = uni(win[v].dt);
+            w.tag = uni(win[v].tag);
+            w.target = uni(win[v].target);
         }
         if (again) __syncthreads();
     }
@@ -2438,7 +2446,7 @@ __device__ __forceinline__ void create_pair_full(const ChainArgs &a, const Geo<D
             }
             if (!cs.far() || cs.first + FAR_BLOCK >= q.ncells) break;
         }
-        const Winner w = group_winner<NT>(sh, m, true);
+        const Winner w = group_winner<NT>(sh.win[2], m, true);
         const int bad = w.bad | acc.bad;
         if (w.rank != NO_RANK && (acc.rank == NO_RANK || ub(winner_lt(w, acc)))) acc = w;
         acc.bad = bad;
@@ -2542,11 +2550,12 @@ __device__ __noinline__ static void rare_step(const ChainArgs *args, ChainShared
 
 // A leg of the hot list: its creates and the choice of its event, in `e`.  Returns the outcome:
 // HOT_EVENT (commit e), HOT_STORED (the earliest stored event `stored` comes first and trashes the
-// list) or HOT_GENERAL (the general form has to run the leg: the leg's state is as before).
+// list) or HOT_GENERAL (the general form has to run the leg: the leg's state is as before).  `turn`: the
+// leg's parity, which copy of the winners it uses.
 enum { HOT_EVENT = 0, HOT_STORED = 1, HOT_GENERAL = 2 };
 template <int D, int FM, int NT, bool RES>
 __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh, const HotList &hot,
-                                          const Items &constants, const Pick &stored, bool hashed, Event<D> &e) {
+                                          const Items &constants, const Pick &stored, bool hashed, int turn, Event<D> &e) {
     constexpr int NW = NT / 64;
     const int lane = threadIdx.x & 63, wave = wave_index<NT>();
     const uint64_t cursor0 = g.cursor;
@@ -2724,7 +2733,7 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
                 else if (winner_lt(v, m)) m = v;
             }
         }
-        P = group_winner<NT>(sh, m, false);
+        P = group_winner<NT>(sh.win[turn], m, false);
         g.produced += (uint64_t)steps * RING_STEP;
         if (P.bad) return general();   // which reports it, unless another candidate set errs first
         const bool any = P.rank != NO_RANK;
@@ -2840,7 +2849,7 @@ __device__ __forceinline__ void chain_body(const ChainArgs &a) {
                     if ((hot.mask >> (threadIdx.x & 15)) & 1u) g.lvalid = 0;   // created anew
                     stored = pick_stored(g);
                 }
-                done = hot_events<D, FM, NT, RES>(a, q, g, sh, hot, its, stored, log != nullptr, e);
+                done = hot_events<D, FM, NT, RES>(a, q, g, sh, hot, its, stored, log != nullptr, (int)(k & 1), e);
             }
         }
         int w;
