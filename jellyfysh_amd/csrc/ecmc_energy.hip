@@ -39,13 +39,19 @@ constexpr int EROW = 9;   // a row's sums: energy, dU/dx_i (3), dU/dpar (4), dU/
 // wave vector instead of O(n^2), less the row's own term and the pairs out of scope.  Evaluated
 // pair by pair (three calls of the derivative and one of psi, each with its own erfc and its own
 // Fourier sum), 1000 units took 777 us forward and 1915 us backward.
+//
+// S(k) holds every charge of the system, so what a row takes off it again leaves rounding errors of
+// that size.  A row takes this form only where the charge to take off (its own and its units' out of
+// scope, by magnitude) is at most that of its partners, which bounds its error by twice the plain
+// sum's; the other rows add their pairs' Fourier parts one by one.
 struct CoulombWork {
-    int32_t on, fc, n_img, direct;     // direct: the Fourier part pair by pair (scope intra)
+    int32_t fc, n_img, direct;         // direct: the Fourier part pair by pair in every row (scope intra)
     double L, aol, aol2, two_aol_rpi, tpol, background;
     double2 *phase;                    // exp(2 pi i m x_d / L): [(d (fc + 1) + m) n + unit]
     double2 *S;                        // structure factors: wave vector of the half space (kvector)
     double *g;                         // Fourier weights of the octant [(i (fc + 1) + j) (fc + 1) + k]
     double *img;                       // image offsets, n_img x 3
+    int32_t *pairwise;                 // per row: not 0 where it adds its pairs' Fourier parts one by one
 };
 
 struct EnergyArgs {
@@ -126,10 +132,36 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// One wavefront per wave vector.
+// Whether unit j is a partner of a row of molecule mi (j not the row's own unit).
+__device__ __forceinline__ bool in_scope(const EnergyArgs &A, int mi, int j) {
+    return A.scope == ECMC_SCOPE_ALL || (A.mol[j] == mi) == (A.scope == ECMC_SCOPE_INTRA);
+}
+
+// The form of row i's Fourier part, by one wavefront.
+__device__ __forceinline__ void coulomb_row_form(const EnergyArgs &A, int i, int lane) {
+    const int mi = A.scope != ECMC_SCOPE_ALL ? A.mol[i] : 0;
+    double held = 0.0, excess = 0.0;   // the partners' charge, and the rest's
+    for (int j = lane; j < A.n; j += 64) {
+        const double q = A.use_charge ? fabs(A.charge[j]) : 1.0;
+        if (j == i) excess += q;
+        else if (in_scope(A, mi, j)) held += q;
+        // (NaN where a unit is somewhere that is not finite: the structure factors then are NaN too)
+        else excess += q + 0.0 * (A.pos[3 * (size_t)j] + A.pos[3 * (size_t)j + 1] + A.pos[3 * (size_t)j + 2]);
+    }
+    held = wave_sum(held);
+    excess = wave_sum(excess);
+    if (lane == 0) A.cw.pairwise[i] = !(excess <= held);
+}
+
+// One wavefront per row and per wave vector.  (1000 units: 9.6 us, 8.1 without the rows' forms; summed in
+// each row's own workgroup they took 3.5 us a launch.)
 __global__ __launch_bounds__(ET) void coulomb_structure(EnergyArgs A) {
     const CoulombWork &c = A.cw;
-    const int v = blockIdx.x * (ET / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int row = blockIdx.x * (ET / 64) + (threadIdx.x >> 6), v = row - A.n, lane = threadIdx.x & 63;
+    if (row < A.n) {
+        coulomb_row_form(A, row, lane);
+        return;
+    }
     int i, j, k;
     if (v >= kvectors(c.fc) || !kvector(c.fc, v, i, j, k)) return;
     double re = 0.0, im = 0.0;
@@ -333,11 +365,11 @@ __global__ __launch_bounds__(ET) void energy_rows(EnergyArgs A) {
     const double ci = A.use_charge ? A.charge[i] : 1.0;
     const int mi = A.scope != ECMC_SCOPE_ALL ? A.mol[i] : 0;
     const PairConstants pc = pair_constants(A, POT);
+    const bool direct = COULOMB && (A.cw.direct || A.cw.pairwise[i]);
     for (int j = t; j < A.n; j += nt) {
         if (j == i) continue;
-        const bool same = A.scope != ECMC_SCOPE_ALL && A.mol[j] == mi;
-        const bool in = A.scope == ECMC_SCOPE_ALL || same == (A.scope == ECMC_SCOPE_INTRA);
-        if (!in && !(COULOMB && !A.cw.direct)) continue;
+        const bool in = in_scope(A, mi, j);
+        if (!in && !(COULOMB && !direct)) continue;
         const double cj = A.use_charge ? A.charge[j] : 1.0;
         if (COULOMB) {
             if (in) {
@@ -349,7 +381,7 @@ __global__ __launch_bounds__(ET) void energy_rows(EnergyArgs A) {
                 if (BW)
                     for (int d = 0; d < 3; d++) acc[1 + d] = fma(cj, der[d], acc[1 + d]);
             }
-            if (in == (A.cw.direct != 0)) {   // scope intra: the pairs in it; else what S(k) holds too much
+            if (in == direct) {   // the row's own pairs, or those that S(k) holds too much
                 double psi, der[3];
                 coulomb_fourier_pair<BW>(A.cw, A.n, i, j, psi, der);
                 const double w = in ? cj : -cj;
@@ -372,7 +404,7 @@ __global__ __launch_bounds__(ET) void energy_rows(EnergyArgs A) {
             }
         }
     }
-    if (COULOMB && !A.cw.direct) {
+    if (COULOMB && !direct) {
         // Re and Im of exp(-i k.x_i) S(k) over the half space, less the row's own term
         const int nv = kvectors(A.cw.fc), nn = A.cw.fc + 1;
         for (int v = t; v < nv; v += nt) {
@@ -441,9 +473,9 @@ __global__ __launch_bounds__(ET) void energy_finish(const double *rows, int n, i
 
 using namespace ecmc;
 
-// Doubles behind the rows: phases, structure factors, Fourier weights, image offsets.
+// Doubles behind the rows: phases, structure factors, Fourier weights, image offsets, the rows' forms.
 struct CoulombSizes {
-    int64_t phase, S, g, img;
+    int64_t phase, S, g, img, form;
     int32_t n_img;
 };
 static CoulombSizes coulomb_sizes(const ecmc_energy_term *t, int64_t n) {
@@ -458,13 +490,14 @@ static CoulombSizes coulomb_sizes(const ecmc_energy_term *t, int64_t n) {
     z.S = 2 * nn * (2 * fc + 1) * (2 * fc + 1);
     z.g = nn * nn * nn;
     z.img = 3 * (int64_t)z.n_img;
+    z.form = (n + 1) / 2;
     return z;
 }
 
 extern "C" int ecmc_energy_workspace_bytes(const ecmc_energy_term *term, int32_t n, int64_t *bytes) {
     if (!term || !bytes || n < 0) return ecmc_fail(ECMC_ERR_ARGUMENT, "null argument or negative size");
     const CoulombSizes z = coulomb_sizes(term, n);
-    *bytes = ((int64_t)n * EROW + (z.n_img ? 1 : 0) + z.phase + z.S + z.g + z.img) * 8;
+    *bytes = ((int64_t)n * EROW + (z.n_img ? 1 : 0) + z.phase + z.S + z.g + z.img + z.form) * 8;
     return ECMC_OK;
 }
 
@@ -533,6 +566,7 @@ static int energy_launch(const ecmc_energy_term *term, int32_t n, const double *
         c.S = (double2 *)(w + z.phase);
         c.g = w + z.phase + z.S;
         c.img = c.g + z.g;
+        c.pairwise = (int32_t *)(c.img + z.img);
         c.n_img = z.n_img;
         c.fc = fc;
         c.direct = A.scope == ECMC_SCOPE_INTRA;
@@ -546,7 +580,7 @@ static int energy_launch(const ecmc_energy_term *term, int32_t n, const double *
         hipLaunchKernelGGL(coulomb_setup, dim3((tasks + ET - 1) / ET), dim3(ET), 0, st, A, pc, alpha);
         if (!c.direct) {
             const int nv = nn * (2 * fc + 1) * (2 * fc + 1);
-            hipLaunchKernelGGL(coulomb_structure, dim3((nv + 3) / 4), dim3(ET), 0, st, A);
+            hipLaunchKernelGGL(coulomb_structure, dim3((n + nv + 3) / 4), dim3(ET), 0, st, A);
         }
         break;
     }
