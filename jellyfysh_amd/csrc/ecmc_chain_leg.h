@@ -2665,9 +2665,11 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
             }
         }
         // Words ahead of the stream, made by the wavefront that inverts no contenders: as many as
-        // this leg drew and some more, as far as the ring holds them beside this leg's.
+        // this leg drew and some more, as far as the ring holds them beside this leg's and the two
+        // before it (a direct leg has no barrier up to here, and a slower wavefront may still be
+        // taking the last leg's thinning draw).
         const int drawn = (int)word, ready = (int)(g.produced - cursor0);
-        const int want = min(2 * drawn + drawn / 4 + 640, q.ring_mask + 1) - ready;
+        const int want = min(2 * drawn + drawn / 4 + 640, q.ring_mask + 1 - 2) - ready;
         constexpr int maker = NW > 1 ? 1 : 0;
         int steps = 0;
         if (want >= RING_STEP) {

@@ -1,7 +1,7 @@
 """Unlogged chains of four wavefronts whose legs have one barrier each (a single set inverted without
-a quick test, the active unit kept by cell boundaries), and chains whose sampling events send the leg
-through the general form, end in the state of the logged run, which has barriers of its own between
-two legs' exchanges of winners."""
+a quick test, the active unit kept by cell boundaries or refused cell vetoes, the random words made
+ahead filling the ring), and chains whose sampling events send the leg through the general form, end in
+the state of the logged run, which has barriers of its own between two legs' exchanges of winners."""
 import numpy as np
 import pytest
 
@@ -32,6 +32,37 @@ def test_gpu_unlogged_chain_ends_where_the_logged_one_does(device, name, factors
     assert not sampling or (kinds == len(factors) + 1).any()
     print(name, "unlogged run", flush=True)
     assert [plain.run(700, log=False) for _ in range(2)] == [700, 700]
+    assert plain.active() == logged.active() and plain.rng_words() == logged.rng_words()
+    assert np.array_equal(plain.positions(), logged.positions())
+    assert np.array_equal(plain.estimators(), logged.estimators())
+    logged.close()
+    plain.close()
+
+
+def test_gpu_unlogged_direct_legs_with_a_cell_veto_and_a_full_ring(device):
+    from jellyfysh_amd.chain import DeviceChain, make_desc
+    from jellyfysh_amd.batch import lattice_positions
+    n, legs = 2800, 250
+    length = n ** (1 / 3)
+    pos = lattice_positions(n, length, 0.02, np.random.default_rng(3))
+    charges = np.where(np.arange(n) % 2 == 0, 1.0, -1.0)
+    wiring = S.standard_wiring([dict(S.factor_tagger("lj", "lennard_jones", [1.0, 0.8]), kind="pair_all")], 0.9, 1.0e9)
+    pairs = wiring[0]["create"]
+    for t in wiring:
+        for key in ("create", "trash"):
+            if set(pairs) <= set(t[key]):
+                t[key] = t[key] + ["veto"]
+    wiring.append(dict(tag="veto", kind="cell_veto", potential="merged_image_coulomb", params=[3.45, 6.0, 2.0, 1.0],
+                       bounding_params=[1.5, 10, 1.0, float("inf")], charge=True, create=wiring[0]["create"],
+                       trash=wiring[0]["trash"], number_event_handlers=1))
+    desc = make_desc(3, n, length, 2.0, 5, wiring, 12, scheduler="heap", max_occupants=1)
+    logged, plain = DeviceChain(desc, pos, charges), DeviceChain(desc, pos, charges)
+    print("logged run", flush=True)
+    ev = logged.run(legs)
+    veto = ev["tagger"] == len(wiring) - 1
+    assert (veto & (ev["flags"] & 1 == 0)).any()         # vetoes that are refused: the active unit stays
+    print("unlogged run", flush=True)
+    assert plain.run(legs, log=False) == legs
     assert plain.active() == logged.active() and plain.rng_words() == logged.rng_words()
     assert np.array_equal(plain.positions(), logged.positions())
     assert np.array_equal(plain.estimators(), logged.estimators())
