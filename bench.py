@@ -464,7 +464,7 @@ def main():
     launch_ms = dom_ms / max(dom_launches, 1)
     achieved = flops_per_launch / (launch_ms * 1e-3) / 1e12
     exact = float((s1["stats"][:, 3] - s0["stats"][:, 3]).sum())
-    dom_name = "ecmc::batched_kernel<%d,false>" % batch.classes[1][dom]
+    dom_name = "ecmc::batched_kernel<%d,false>" % batch.widths()[dom]
     traffic = profiled_traffic(dom_name, args.legs)
     # pressure from untimed production steps after the timed region (each replica then has
     # (warmup + steps) x legs legs behind it)
@@ -482,7 +482,7 @@ def main():
                                "beta 1/1.5, chain 1.0, %d legs per replica per step" % (len(n), args.legs),
                    "replicas": int(len(n)), "units": int(np.sum(n)), "legs_per_step": args.legs,
                    "classes": {"max_n": [int(v) for v in batch.classes[0]],
-                               "wavefronts_per_replica": [int(v) for v in batch.classes[1]]}},
+                               "wavefronts_per_replica": batch.widths()}},
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_TFLOPS, "traffic": traffic,
                      "peak_fp64": PEAK_FP64_TFLOPS, "frac_fp64": achieved / PEAK_FP64_TFLOPS,

@@ -266,8 +266,15 @@ int ecmc_batch_create(const ecmc_batch_desc *desc, const int32_t *n_per_replica,
                       const double *positions, ecmc_batch **out);
 void ecmc_batch_destroy(ecmc_batch *batch);
 /* Size classes: replicas with n <= class_max_n[c] (first such c) run with class_wpr[c]
- * wavefronts per replica; one persistent kernel per class, all launched together. */
+ * wavefronts per replica; one persistent kernel per class, all launched together.  Turns the
+ * automatic width off. */
 int ecmc_batch_set_classes(ecmc_batch *batch, int32_t n_classes, const int32_t *class_max_n, const int32_t *class_wpr);
+/* Automatic width: when on, classes of one wavefront per replica are launched with two or four
+ * where the replicas are too few to fill the card (the events are the same);
+ * ecmc_batch_class_width returns the wavefronts per replica that a class is launched with.  No
+ * reference counterpart. */
+int ecmc_batch_set_automatic_width(ecmc_batch *batch, int32_t on);
+int ecmc_batch_class_width(const ecmc_batch *batch, int32_t cls, int32_t *width);
 /* 0: FP32 filter (default); 1: every candidate inverted in FP64; 2: filter plus audit of
  * every bound against the exact value (violations counted, see ecmc_batch_audit). */
 int ecmc_batch_set_mode(ecmc_batch *batch, int32_t mode);

@@ -108,6 +108,8 @@ def _signatures():
         "ecmc_batch_create": (i32, [vp, vp, pd, pd, ctypes.POINTER(vp)]),
         "ecmc_batch_destroy": (None, [vp]),
         "ecmc_batch_set_classes": (i32, [vp, i32, vp, vp]),
+        "ecmc_batch_set_automatic_width": (i32, [vp, i32]),
+        "ecmc_batch_class_width": (i32, [vp, i32, vp]),
         "ecmc_batch_set_mode": (i32, [vp, i32]),
         "ecmc_batch_set_log": (i32, [vp, i32]),
         "ecmc_batch_run": (i32, [vp, i32]),

@@ -87,9 +87,9 @@ class DeviceBatch:
         L.check(self._L.ecmc_batch_create(ctypes.byref(d), n.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)),
                                           lengths.ctypes.data_as(pd), pos.ctypes.data_as(pd), ctypes.byref(h)))
         self._h = h
+        self.set_classes(*(default_classes() if classes is None else classes))
         if classes is None:
-            classes = default_classes()
-        self.set_classes(*classes)
+            L.check(self._L.ecmc_batch_set_automatic_width(self._h, 1))
 
     def _sig(self):
         self._L = L.lib()
@@ -109,6 +109,16 @@ class DeviceBatch:
         p = ctypes.POINTER(ctypes.c_int32)
         L.check(self._L.ecmc_batch_set_classes(self._h, len(mx), mx.ctypes.data_as(p), wp.ctypes.data_as(p)))
         self.classes = (list(mx), list(wp))
+
+    def widths(self):
+        """Per size class, the wavefronts per replica that it is launched with: the class's own, or more
+        where the classes were not given and the replicas are too few to fill the card."""
+        w = ctypes.c_int32()
+        out = []
+        for c in range(len(self.classes[0])):
+            L.check(self._L.ecmc_batch_class_width(self._h, c, ctypes.byref(w)))
+            out.append(w.value)
+        return out
 
     def set_mode(self, mode):
         L.check(self._L.ecmc_batch_set_mode(self._h, int(mode)))

@@ -77,6 +77,7 @@ struct ecmc_batch {
     int32_t graph_legs = -1;
     bool class_timing = false;
     int32_t max_blocks = 0;   // limit of every class's persistent grid (0 = as many as fit)
+    bool automatic = false;   // classes of one wavefront per replica may run wider (class_widths)
 };
 
 // Add the kernel time of every class of the step that just completed.
@@ -92,7 +93,53 @@ static int add_class_times(ecmc_batch *b) {
     return ECMC_OK;
 }
 
-static int launch_class(ecmc_batch *b, int c, int legs, hipStream_t st) {
+static int compute_units() {
+    int dev = 0, cus = 0;
+    hipGetDevice(&dev);
+    hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    return std::max(cus, 1);
+}
+
+// Workgroups of w wavefronts that a CU holds for replicas of a class.
+static int blocks_per_cu(int w, int nmax, int cellmax) {
+    int fit = 0;
+    const size_t lds = batched_lds_bytes(nmax, cellmax, w);
+    switch (w) {
+    case 1: hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<1, false>, 64, lds); break;
+    case 2: hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<2, false>, 128, lds); break;
+    case 4: hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<4, false>, 256, lds); break;
+    case 8: hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<8, false>, 512, lds); break;
+    }
+    return fit;
+}
+
+// The wavefronts per replica that every class is launched with: its own, or wider where the choice is
+// automatic.  One wavefront per replica is the best use of a full card; replicas too few to fill it are
+// run by the idle wavefronts too (the events are the same).  Beyond 27 cells' worth of candidates the
+// leg's first pass is long enough: 64 to 256 replicas of 2048 units 14.3 -> 12.2 ms with four, 1024
+// replicas 15.9 -> 14.3 ms with two, 64 replicas of 512 units 12.8 -> 11.6 ms with four; 64 replicas of
+// 128 units lose (9.3 against 11.1 ms), and so does every size where the workgroups no longer are
+// resident at once (1024 replicas with four: 22.6 ms).  The classes run beside each other, so the
+// replicas and workgroups of all of them count.
+static void class_widths(const ecmc_batch *b, int32_t *width) {
+    constexpr int WIDE_UNITS = 384;
+    for (int c = 0; c < b->n_classes; c++) width[c] = b->class_wpr[c];
+    if (!b->automatic || b->max_blocks > 0) return;
+    const int cus = compute_units();
+    if (b->n_rep > 4 * cus) return;
+    const int wide = b->n_rep <= 2 * cus ? 4 : 2;
+    int64_t cus_taken = 0;
+    for (int c = 0; c < b->n_classes; c++) {
+        if (b->class_count[c] == 0) continue;
+        if (width[c] == 1 && b->class_nmax[c] >= WIDE_UNITS) width[c] = wide;
+        const int fit = blocks_per_cu(width[c], b->class_nmax[c], b->class_cellmax[c]);
+        cus_taken += fit > 0 ? (b->class_count[c] + fit - 1) / fit : (int64_t)cus + 1;
+    }
+    if (cus_taken > cus)
+        for (int c = 0; c < b->n_classes; c++) width[c] = b->class_wpr[c];
+}
+
+static int launch_class(ecmc_batch *b, int c, int wpr, int legs, hipStream_t st) {
     if (b->class_count[c] == 0) return ECMC_OK;
     BatchArgs A;
     memset(&A, 0, sizeof(A));
@@ -121,33 +168,13 @@ static int launch_class(ecmc_batch *b, int c, int legs, hipStream_t st) {
     hipLaunchKernelGGL(reset_work, dim3((A.count + 255) / 256), dim3(256), 0, st, A.state, A.count, A.queue);
     A.log = b->d_log;
     A.audit = b->d_audit;
-    int wpr = b->class_wpr[c];
-    int dev = 0, cus = 0;
-    hipGetDevice(&dev);
-    hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    // One wavefront per replica is the best use of a full card; replicas too few to fill it are run by
-    // the idle wavefronts too (the events are the same).  Beyond 27 cells' worth of candidates the
-    // leg's first pass is long enough: 64 to 256 replicas of 2048 units 14.3 -> 12.2 ms with four,
-    // 1024 replicas 15.9 -> 14.3 ms with two, 64 replicas of 512 units 12.8 -> 11.6 ms with four; 64
-    // replicas of 128 units lose (9.3 against 11.1 ms), and so does every size where the workgroups
-    // no longer are resident at once (1024 replicas with four: 22.6 ms).
-    constexpr int WIDE_UNITS = 384;
-    if (wpr == 1 && b->max_blocks == 0 && A.nmax >= WIDE_UNITS) {
-        if (A.count <= 2 * cus) wpr = 4;
-        else if (A.count <= 4 * cus) wpr = 2;
-        int fit = 0;
-        if (wpr == 4) hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<4, false>, 256, batched_lds_bytes(A.nmax, A.cellmax, 4));
-        if (wpr == 2) hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, batched_kernel<2, false>, 128, batched_lds_bytes(A.nmax, A.cellmax, 2));
-        if (fit * cus < A.count) wpr = 1;
-    }
     size_t lds = batched_lds_bytes(A.nmax, A.cellmax, wpr);
-    int per_cu = 1;
+    const int per_cu = blocks_per_cu(wpr, A.nmax, A.cellmax);
+    if (per_cu < 1) return ecmc_fail(ECMC_ERR_CONFIGURATION, "replica does not fit in LDS");
+    int grid = std::min(A.count, per_cu * compute_units());
+    if (b->max_blocks > 0) grid = std::min(grid, b->max_blocks);
 #define ECMC_LAUNCH(W)                                                                                     \
     {                                                                                                      \
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batched_kernel<W, false>, 64 * W, lds);       \
-        if (per_cu < 1) return ecmc_fail(ECMC_ERR_CONFIGURATION, "replica does not fit in LDS");           \
-        int grid = std::min(A.count, per_cu * std::max(cus, 1));                                           \
-        if (b->max_blocks > 0) grid = std::min(grid, b->max_blocks);                                       \
         if (A.mode) hipLaunchKernelGGL((batched_kernel<W, true>), dim3(grid), dim3(64 * W), lds, st, A);   \
         else hipLaunchKernelGGL((batched_kernel<W, false>), dim3(grid), dim3(64 * W), lds, st, A);         \
     }
@@ -165,13 +192,15 @@ static int launch_class(ecmc_batch *b, int c, int legs, hipStream_t st) {
 
 // One step: reset the work queues, then every size class on its own stream.
 static int enqueue_step(ecmc_batch *b, int legs, hipStream_t main, bool timed) {
+    int32_t width[8];
+    class_widths(b, width);
     hipEventRecord(b->fork[0], main);
     // largest replicas first: their blocks are resident from the start, and the smaller
     // classes fill the slots left beside them
     for (int c = b->n_classes - 1; c >= 0; c--) {
         hipStreamWaitEvent(b->streams[c], b->fork[0], 0);
         if (timed) hipEventRecord(b->cls_ev0[c], b->streams[c]);
-        int rc = launch_class(b, c, legs, b->streams[c]);
+        int rc = launch_class(b, c, width[c], legs, b->streams[c]);
         if (rc) return rc;
         if (timed) hipEventRecord(b->cls_ev1[c], b->streams[c]);
         hipEventRecord(b->fork[c + 1], b->streams[c]);
@@ -297,6 +326,7 @@ extern "C" int ecmc_batch_set_classes(ecmc_batch *b, int32_t n_classes, const in
     b->d_order.clear(); b->streams.clear(); b->fork.clear(); b->cls_ev0.clear(); b->cls_ev1.clear();
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
+    b->automatic = false;
     b->n_classes = n_classes;
     b->class_max_n.assign(class_max_n, class_max_n + n_classes);
     b->class_wpr.assign(class_wpr, class_wpr + n_classes);
@@ -432,6 +462,23 @@ extern "C" int ecmc_batch_set_max_blocks(ecmc_batch *b, int32_t max_blocks) {
     b->max_blocks = max_blocks;
     if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
     if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
+    return ECMC_OK;
+}
+
+extern "C" int ecmc_batch_set_automatic_width(ecmc_batch *b, int32_t on) {
+    if (!b) return ecmc_fail(ECMC_ERR_ARGUMENT, "null batch");
+    b->automatic = on != 0;
+    if (b->graph_exec) { hipGraphExecDestroy(b->graph_exec); b->graph_exec = nullptr; }
+    if (b->graph) { hipGraphDestroy(b->graph); b->graph = nullptr; }
+    return ECMC_OK;
+}
+
+extern "C" int ecmc_batch_class_width(const ecmc_batch *b, int32_t cls, int32_t *width) {
+    if (!b || !width) return ecmc_fail(ECMC_ERR_ARGUMENT, "null argument");
+    if (cls < 0 || cls >= b->n_classes) return ecmc_fail(ECMC_ERR_ARGUMENT, "no such class");
+    int32_t all[8];
+    class_widths(b, all);
+    *width = all[cls];
     return ECMC_OK;
 }
 
