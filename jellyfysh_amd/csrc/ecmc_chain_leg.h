@@ -1340,7 +1340,7 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
     const float ibf = q.inv_beta;
     const float inv_L = __builtin_amdgcn_rcpf(Lf);
     const int act = g.active, dir = g.adir;
-    const float caf = q.charged ? (float)charge_of<RES>(a, q, act) : 1.f;   // (any pair potential may take the charges)
+    const float caf = (FM & FEAT_EWALD) && q.charged ? (float)charge_of<RES>(a, q, act) : 1.f;
     float cell_rate_max = 0.f;
     if (FM & FEAT_CELL_BOUNDING) cell_rate_max = pick_axis<3>(q.cb_max, dir);
     int qn = 0;
@@ -1419,8 +1419,11 @@ __device__ __forceinline__ int gather_contenders(const ChainArgs &a, const Geo<D
                             pp[u] = pref;
                         }
                         if ((q.charged >> tag) & 1u) {
+                            // any pair potential may take the charges; variants without the Coulomb
+                            // machinery hold no register for the active unit's
+                            const float ca = FM & FEAT_EWALD ? caf : (float)charge_of<RES>(a, q, act);
 #pragma unroll
-                            for (int u = 0; u < U; u++) pp[u] *= caf * (float)charge_of<RES>(a, q, target[u]);
+                            for (int u = 0; u < U; u++) pp[u] *= ca * (float)charge_of<RES>(a, q, target[u]);
                         }
 #pragma unroll
                         for (int u = 0; u < U; u++) {
