@@ -351,6 +351,81 @@ static void cell_bound_cache_store(const std::vector<double> &key, const std::ve
     g_cb_cache.push_back({dev, key, table});
 }
 
+// The host views of the live systems, in slabs of pinned memory: one device's views of one size, as many
+// slots in a new slab as the slabs of that size already have (at most VIEW_SLAB bytes), so that a lone
+// system takes one view and 256 of them ten allocations, of 50 to 130 us each, instead of 256.  A slab
+// goes back to the system with its last view.
+struct ViewSlab {
+    int device;
+    size_t bytes;                 // of one view
+    int32_t slots;
+    unsigned char *base, *seen;   // host address, and the device's
+    std::vector<int32_t> free;
+};
+static std::mutex g_view_mutex;
+static std::vector<ViewSlab> g_view_slabs;
+constexpr size_t VIEW_SLAB = 1 << 20;
+
+// A view of `bytes` for the current device, its device address in `seen`; null: pinned memory exhausted.
+static HostView *take_view(int device, size_t bytes, HostView **seen) {
+    bytes = (bytes + 255) & ~(size_t)255;
+    std::lock_guard<std::mutex> lock(g_view_mutex);
+    size_t at = g_view_slabs.size();
+    int64_t have = 0;
+    for (size_t k = 0; k < g_view_slabs.size(); k++) {
+        const ViewSlab &v = g_view_slabs[k];
+        if (v.device != device || v.bytes != bytes) continue;
+        have += v.slots;
+        if (!v.free.empty()) at = k;
+    }
+    if (at == g_view_slabs.size()) {
+        ViewSlab v = {device, bytes, 0, nullptr, nullptr, {}};
+        const int64_t most = std::max<int64_t>(1, (int64_t)(VIEW_SLAB / bytes));
+        void *base = nullptr, *dev = nullptr;
+        for (int64_t slots = std::min(std::max<int64_t>(1, have), most); slots > 0 && !base; slots = slots > 1 ? 1 : 0) {
+            v.slots = (int32_t)slots;
+            if (hipHostMalloc(&base, bytes * slots, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+                base = nullptr;
+                (void)hipGetLastError();
+            }
+        }
+        if (!base) return nullptr;
+        if (hipHostGetDevicePointer(&dev, base, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            hipHostFree(base);
+            return nullptr;
+        }
+        v.base = (unsigned char *)base;
+        v.seen = (unsigned char *)dev;
+        for (int32_t i = v.slots; i-- > 0;) v.free.push_back(i);
+        g_view_slabs.push_back(v);
+    }
+    ViewSlab &v = g_view_slabs[at];
+    const size_t off = (size_t)v.free.back() * v.bytes;
+    v.free.pop_back();
+    *seen = (HostView *)(v.seen + off);
+    return (HostView *)(v.base + off);
+}
+
+// Returns a view that no launch writes any more.
+static void release_view(HostView *view) {
+    unsigned char *const p = (unsigned char *)view, *empty = nullptr;
+    {
+        std::lock_guard<std::mutex> lock(g_view_mutex);
+        for (size_t k = 0; k < g_view_slabs.size(); k++) {
+            ViewSlab &v = g_view_slabs[k];
+            if (p < v.base || p >= v.base + v.bytes * v.slots) continue;
+            v.free.push_back((int32_t)((p - v.base) / v.bytes));
+            if ((int32_t)v.free.size() == v.slots) {
+                empty = v.base;
+                g_view_slabs.erase(g_view_slabs.begin() + k);
+            }
+            break;
+        }
+    }
+    if (empty) hipHostFree(empty);
+}
+
 extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *positions, const double *charges,
                                   ecmc_system **out) {
     if (!desc || !positions || !out) return ecmc_fail(ECMC_ERR_ARGUMENT, "null argument");
@@ -744,21 +819,13 @@ extern "C" int ecmc_system_create(const ecmc_system_desc *desc, const double *po
         }
     }
     plan_lds(s);
-    // the host view; a system without one (pinned memory exhausted) copies what it reads.  The allocation
-    // takes 50 to 130 us of a system's creation (0.37 to 0.61 ms each where 256 are created), what the copies of
-    // one or two calls took.
+    // the host view; a system without one (pinned memory exhausted) copies what it reads
     const bool res_positions = s->args.resident != 0;
-    if (hipHostMalloc((void **)&s->host, sizeof(HostView) + (res_positions ? sizeof(double) * dim * n : 0),
-                      hipHostMallocPortable | hipHostMallocMapped) == hipSuccess) {
-        void *seen = nullptr;
-        if (hipHostGetDevicePointer(&seen, s->host, 0) != hipSuccess) { ecmc_system_destroy(s); return ecmc_fail(ECMC_ERR_HIP, "hipHostGetDevicePointer failed"); }
+    s->host = take_view(s->device, sizeof(HostView) + (res_positions ? sizeof(double) * dim * n : 0), &a.host);
+    if (s->host) {
         s->host->st = st;
         s->host->n_out = 0;
         s->host->has_positions = 0;
-        a.host = (HostView *)seen;
-    } else {
-        s->host = nullptr;
-        (void)hipGetLastError();
     }
     *out = s;
     return ECMC_OK;
@@ -770,11 +837,11 @@ extern "C" void ecmc_system_destroy(ecmc_system *s) {
     hipFree(s->d_occ); hipFree(s->d_occ_n); hipFree(s->d_ring); hipFree(s->d_st);
     hipFree(s->d_sur_cell); hipFree(s->d_sur_id); hipFree(s->d_cbt); hipFree(s->d_corners);
     hipFree(s->d_cvw);
-    if (s->host) hipHostFree(s->host);
     hipFree(s->d_tg); hipFree(s->d_nout); hipFree(s->d_log); hipFree(s->d_ewald); hipFree(s->d_ewald_codes); hipFree(s->d_step_ev); hipFree(s->d_args);
     if (s->ev0) hipEventDestroy(s->ev0);
     if (s->ev1) hipEventDestroy(s->ev1);
     if (s->stream) hipStreamDestroy(s->stream);
+    if (s->host) release_view(s->host);   // (freeing device memory has waited for the launches)
     delete s;
 }
 
