@@ -544,6 +544,19 @@ struct SettledPowers {   // powers 6 and 12
     __device__ __forceinline__ double root(double x, double power) { return root36_settled(x, power == 12.0, ok); }
 };
 __device__ __forceinline__ double over_speed(double x, double speed) { return speed == 1.0 ? x : x / speed; }
+// A displacement that the reference code answers with a ValueError because a root's argument rounds
+// below zero (an attractive unit passed so closely that the draw is lost in the energy there): NaN, with
+// the time t of the closest approach, where the event would be, as a float in the low word.
+__device__ __forceinline__ double error_at(double t) {
+    return __hiloint2double(0x7ff80000, __float_as_int((float)fmax(t, 0.0) * (1.f - 0x1p-22f)));
+}
+// The time of a NaN displacement as a positive number that is larger for earlier times (every other
+// NaN: time 0), and the time of that number.
+__device__ __forceinline__ int error_code(double dt) {
+    const int bits = __double2loint(dt);
+    return 0x7f800001 - (bits < 0 || bits > 0x7f800000 ? 0 : bits);
+}
+__device__ __forceinline__ float error_time(int code) { return __int_as_float(0x7f800001 - code); }
 template <int D, class Powers>
 __device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, const double *sep, double pp, double power, double rc2,
                                           double urc, double dU) {
@@ -563,7 +576,8 @@ __device__ __forceinline__ double ip_time(Powers &m, int dir, double speed, cons
     const double nsq = m.root(live ? pp / (cur + dU) : 1.0, power);
     const double a = nsq - perp2;
     const double sq = sqrt(fmax(a, 0.0));
-    const double res = a < 0.0 ? NAN : over_speed(rep ? sdd - sq : disp + (sdd + sq), speed);
+    const double t = over_speed(rep ? sdd - sq : disp + (sdd + sq), speed);
+    const double res = a < 0.0 ? error_at(t) : t;
     return live ? res : INFINITY;
 }
 
@@ -691,8 +705,8 @@ struct Contender {
     uint32_t word;
     int32_t rank, target, tag_cell;
 };
-// An earliest pair candidate: its time, push rank (NO_RANK: none), tagger and unit; bad: some
-// candidate was NaN (a ValueError of the reference code).
+// An earliest pair candidate: its time, push rank (NO_RANK: none), tagger and unit; bad: not 0 where
+// some candidate was NaN (a ValueError of the reference code), the larger the earlier (error_code).
 constexpr int NO_RANK = 0x7fffffff;
 struct Winner {
     Time t;
@@ -1518,7 +1532,7 @@ __device__ __forceinline__ Winner no_winner() {
 // push rank.
 __device__ __forceinline__ Winner wave_winner(const Winner &m) {
     Winner w = no_winner();
-    w.bad = __ballot(m.bad) ? 1 : 0;
+    if (__ballot(m.bad)) w.bad = -wave_min(-m.bad);
     const double dmin = wave_min(m.rank == NO_RANK ? INFINITY : m.dt);
     unsigned long long eq = __ballot(m.rank != NO_RANK && m.dt == dmin);
     if (!eq) return w;
@@ -1736,7 +1750,12 @@ __device__ __forceinline__ void store_winner(const ChainArgs &a, const Geo<D> &q
         lane_slot(g, t, Time{0.0, 0.0}, 0, 0);
         return;
     }
-    if (w.bad) { g.err = ECMC_ERR_NUMERIC; return; }
+    // an error counts if no event of its set comes before it (legs with a quick test see no more of
+    // them); a set without a quick test is evaluated whole in every leg, and any counts
+    if (w.bad && (((q.tests >> (2 * t)) & 3) == QT_DIRECT || ub((double)error_time(w.bad) <= w.dt))) {
+        g.err = ECMC_ERR_NUMERIC;
+        return;
+    }
     double tp[D], p[D];
     load_pos<RES>(a, q, w.target, tp);
 #pragma unroll
@@ -2382,7 +2401,7 @@ __device__ __forceinline__ Winner group_winner(Winner *win, const Winner &m, boo
             // read as uniform values: the comparison is then a scalar branch
             Winner o;
             o.rank = uni(win[v].rank);
-            w.bad |= uni(win[v].bad);
+            w.bad = max(w.bad, uni(win[v].bad));
             if (o.rank == NO_RANK) continue;
             o.t.q = uni(win[v].t.q);
             o.t.r = uni(win[v].t.r);
@@ -2443,14 +2462,14 @@ __device__ __forceinline__ void create_pair_full(const ChainArgs &a, const Geo<D
                     c.tag = t;
                     c.target = target;
                     c.bad = m.bad;
-                    if (isnan(dt)) m.bad = 1;
+                    if (isnan(dt)) m.bad = max(m.bad, error_code(dt));
                     else if (winner_lt(c, m)) m = c;
                 }
             }
             if (!cs.far() || cs.first + FAR_BLOCK >= q.ncells) break;
         }
         const Winner w = group_winner<NT>(sh.win[2], m, true);
-        const int bad = w.bad | acc.bad;
+        const int bad = max(w.bad, acc.bad);
         if (w.rank != NO_RANK && (acc.rank == NO_RANK || ub(winner_lt(w, acc)))) acc = w;
         acc.bad = bad;
     }
@@ -2734,13 +2753,13 @@ __device__ __forceinline__ int hot_events(const ChainArgs &a, const Geo<D> &q, L
                 v.tag = c.tag_cell & 15;
                 v.target = c.target;
                 v.bad = m.bad;
-                if (isnan(dt)) m.bad = 1;
+                if (isnan(dt)) m.bad = max(m.bad, error_code(dt));
                 else if (winner_lt(v, m)) m = v;
             }
         }
         P = group_winner<NT>(sh.win[turn], m, false);
         g.produced += (uint64_t)steps * RING_STEP;
-        if (P.bad) return general();   // which reports it, unless another candidate set errs first
+        if (P.bad) return general();   // which reports it, unless its set has an earlier event or another set errs first
         const bool any = P.rank != NO_RANK;
         if (direct || (any && ub(P.dt <= h)) || (S.w >= 0 && ub(dS <= h))) break;
         // nothing within the horizon: a wider one
