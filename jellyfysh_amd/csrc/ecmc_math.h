@@ -330,7 +330,9 @@ ECMC_FN double root_pow_fast(double x, bool six, double &lo) {
 }
 
 // FP32 seeds: log2 of a double in the normal float range and 2 ** y, each within 2^-20
-// (relative to max(|log2 x|, 1) and to 2 ** y), and the reciprocal to about 2^-46.
+// (relative to max(|log2 x|, 1) and to 2 ** y), and the reciprocal to about 2^-46.  (A host build may
+// bring seeds of its own, as inexact as these bounds say.)
+#ifndef ECMC_HOST_SEEDS
 ECMC_FN float seed_log2(double x) {
 #if defined(__HIPCC__) && !defined(ECMC_HOST_BUILD)
     return __builtin_amdgcn_logf((float)x);
@@ -353,9 +355,10 @@ ECMC_FN double seed_rcp(double x) {
     return 1.0 / x;
 #endif
 }
+#endif
 
 // t0 (1 + u) ** (-1/k) for u = t0^k / X - 1 (ik = 1/k), the k-th root of X from a seed t0 within
-// 2^-17: the third-order series leaves below 2^-56, the roundings 2^-50.
+// 2^-15 (u below 2^-13): the third-order series leaves below 2^-56, the roundings 2^-50.
 ECMC_FN double root_refine(double t0, double u, double ik) {
     const double c2 = 0.5 * (1.0 + ik), c3 = c2 * (1.0 / 3.0) * (1.0 + ik + ik);
     return fma(-t0 * ik * u, fma(u, fma(u, c3, -c2), 1.0), t0);
