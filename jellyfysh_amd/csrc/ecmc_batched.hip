@@ -11,7 +11,7 @@
 //      enter a contender list in LDS;
 //   3. the contenders are inverted exactly in FP64 (correctly rounded pow/log) and a
 //      workgroup min-reduce over (displacement, kind, target, factor) picks the event;
-//   4. thread 0 commits it (lifting, wall snap, or end of chain with a Philox-drawn new
+//   4. wavefront 0 commits it (lifting, wall snap, or end of chain with a Philox-drawn new
 //      active unit) and updates the cell lists.
 // Because a factor left out has no event within h, the committed event is the one a full
 // FP64 evaluation of every candidate selects; the audit mode checks that on the device.

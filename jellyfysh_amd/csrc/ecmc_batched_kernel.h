@@ -490,11 +490,11 @@ __host__ __device__ inline size_t batched_lds_bytes(int nmax, int cellmax, int w
 //   4. pass 2, one contender per thread: its FP64 position from global memory, exact FP64
 //      inversion with correctly rounded pow/log, workgroup min-reduce over (displacement,
 //      kind, target, factor);
-//   5. thread 0 commits.
+//   5. wavefront 0 commits.
 // Bound by the instructions it issues: with two wavefronts per SIMD (LDS for the largest replica
 // and 256 VGPRs) the VALU is busy 72% of the time.  1697 vector instructions a leg before the
 // cell-sorted records, the runs, the energy test, the division-free cells and the inlined
-// inversion, 1280 with them; 4096 replicas of 64 to 2048 units, 20 000 legs each: 343 -> 270 ms.
+// inversion, 1267 with them; 4096 replicas of 64 to 2048 units, 20 000 legs each: 343 -> 270 ms.
 //
 // CHECK: modes 1 and 2 (their own instance, so that the filtered mode's registers hold nothing of
 // them).

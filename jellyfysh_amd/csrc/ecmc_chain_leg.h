@@ -43,7 +43,6 @@
 
 namespace ecmc {
 
-constexpr int NT_MAX = 256;
 constexpr int AXIS_CELLS = 32;    // cells per side whose bounds are kept in LDS
 constexpr int QCAP = 64;          // contenders queued per wavefront
 constexpr int RING_STEP = 192;    // words one wavefront makes at a time (at most 227: see ring_make)
@@ -97,8 +96,8 @@ struct ChainState {
     Slot slot[ECMC_MAX_TAGGERS];
 };
 
-// What the host reads after a launch, written by the launch's last instructions into pinned host
-// memory that the system owns: the state, the committed legs and, of a launch that kept the
+// What the host reads after a launch, written by the launch's last instructions into the system's view in
+// pinned host memory: the state, the committed legs and, of a launch that kept the
 // positions in LDS, the positions (n x dim) behind this block.  Reading it costs no copy command:
 // the four of a system (committed legs, state, positions, estimators), at 10 to 17 us each, were
 // 14.1 of 40.6 ms where 256 systems of 512 units run 1000 legs and 14.6 of 26.5 ms where 256
@@ -738,7 +737,7 @@ struct Leg {
 };
 
 // The create list of the pair and cell-boundary events' own legs, which nearly every leg runs: pair
-// taggers, at most one cell boundary and, first, at most one cell veto.  Legs of this list take the
+// taggers, at most one cell boundary and at most one cell veto, at any places.  Legs of this list take the
 // short path (hot_events); the others (a sampling event's, the run's start) the general one.
 constexpr int HOT_ITEMS = 4;
 struct HotList {
@@ -1907,7 +1906,8 @@ __device__ __noinline__ static EwaldBound ewald_derivative_fp32(double sx, doubl
 }
 
 // ---- commit -------------------------------------------------------------------------------
-// The event to commit: a stored one (from the wavefront's LDS copy) or one of this leg's.
+// The event to commit: a stored one (its payload from LDS, its time from the tagger's lane) or one of
+// this leg's.
 template <int D>
 struct Event {
     int tagger, target, adir, cell;
@@ -2145,8 +2145,8 @@ __device__ __forceinline__ HotList hot_list(const ChainShared<NT> &sh, const ecm
     return l;
 }
 
-// Copies a system's launch state into LDS and registers; every wavefront gets its own copy of the
-// stored events.
+// Copies a system's launch state into LDS and registers: the stored events' payloads once into LDS, their
+// times into the lanes of every wavefront.
 template <int D, int NT, bool RES>
 __device__ __forceinline__ void launch_load(const ChainArgs &a, Geo<D> &q, Leg<D> &g, ChainShared<NT> &sh) {
     const int tid = threadIdx.x, lane = tid & 63;

@@ -90,7 +90,7 @@ __global__ __launch_bounds__(PT) void pair_kernel(PairArgs a, int derivative) {
 }
 
 // FP32 brackets of the time displacement of inverse-power rows and of inverse-power Coulomb
-// bound rows (the chain kernel's candidate filter), the potential change drawn from the leading
+// bound rows (ecmc_pair_time_bounds), the potential change drawn from the leading
 // word of the random pair.
 template <int D>
 __global__ __launch_bounds__(PT) void pair_bounds_kernel(int64_t n, int trunc, int ipcb, double power, double prefactor,
